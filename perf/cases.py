@@ -4,9 +4,10 @@ Each case is one pass through a public entry point at a size that is used:
 the standalone operators on device buffers (quantised and fp32 matvec, fp32
 matmul), two decoded tokens and whole prompts (and the token that follows
 them, which reads the cache they wrote) through quantised models with their
-logits, whole generate calls (greedy and sampled), and the fp32 model path. The shapes are the repository's synthetic workloads: the TinyLlama
-shape, the Llama-2-7B widths and the small test shapes. ``listed`` names
-twelve of them, ``draw`` makes more of the same kinds over the whole ranges.
+logits, whole generate calls (greedy and sampled), and the fp32 model path.
+The shapes are the repository's synthetic workloads: the TinyLlama shape, the
+Llama-2-7B widths and the small test shapes. ``listed`` names twelve of them,
+``draw`` makes more of the same kinds over the whole ranges.
 
 Inputs come from the seed alone (torch's generator on the GPU): N(0, 0.02)
 weights quantised in blocks, norms around one, uniform token ids, and K/V

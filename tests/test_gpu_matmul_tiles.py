@@ -1,0 +1,44 @@
+"""The fp32 GEMM at the edges of its tiles.
+
+Each shape is one where a tile, its k chunk or its last columns can go wrong:
+fewer rows, columns or k than a tile, one more or less than a whole number of
+them, and one shape for every tile size that the launch chooses among. The
+bound is that of any summation order in fp32: every output's error is at most
+k 2^-23 sum |a b| (k fused steps of half an ulp each, doubled for the partial
+sums' additions)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mkn", [
+    (1, 1, 1), (1, 33, 2), (3, 31, 3), (2, 64, 5), (17, 32, 16), (16, 33, 17),
+    (15, 95, 31), (33, 4001, 130), (48, 257, 768), (768, 100, 768),
+    (1000, 63, 1531), (313, 313, 313), (64, 1000, 63), (500, 65, 777),
+    (65, 129, 4100), (2049, 40, 129),
+])
+def test_matmul_tile_edges(gpu, mkn):
+    m, k, n = mkn
+    rng = np.random.default_rng(m * 7 + k * 3 + n)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    c = gpu.matmul_f32(a, b)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    bound = k * 2.0 ** -23 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.all(np.abs(c - exact) <= bound)
+    assert np.array_equal(gpu.matmul_f32(a, b), c)
+
+
+def test_matmul_non_finite_rows_stay_apart(gpu):
+    """A row of A or a column of B that holds a NaN or an infinity changes
+    that row or column alone, at every ragged edge."""
+    rng = np.random.default_rng(5)
+    a = rng.standard_normal((37, 45)).astype(np.float32)
+    b = rng.standard_normal((45, 51)).astype(np.float32)
+    a[36, 44] = np.nan
+    b[44, 50] = np.inf
+    c = gpu.matmul_f32(a, b)
+    assert np.all(np.isnan(c[36]))
+    assert not np.any(np.isfinite(c[:, 50]))
+    assert np.all(np.isfinite(c[:36, :50]))

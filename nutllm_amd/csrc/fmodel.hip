@@ -2,17 +2,25 @@
 // prefill_tokens (src/kvcache.cpp:237-284) over the device KV cache, with
 // ModelWeights' [in x out] fp32 projections resident in HBM.
 //
-// One decode step per layer: the Q/K/V, Wo, gate/up and down projections
-// are column GEMVs (y_j = sum_i x_i W[i][j], linear_threaded,
-// src/threading.cpp:200-215): a workgroup takes 256 consecutive columns and
-// a run of the input, reads each weight row run coalesced, and writes a
-// partial sum; a small epilogue kernel adds the partials in order and
-// applies what follows the projection (RoPE and the cache store for Q/K/V,
-// the residual add, silu(gate) * up). RMSNorm (src/ops.cpp:111-134) is the
-// GEMV's prologue: every workgroup forms x * scale * w for its run after
-// summing the squares of all of x. Attention is the quantised decode step's
-// kernel (decode.hip), since the cache and the arithmetic are the same.
+// All tokens of a call go through a layer together, in five launches:
+//   Q/K/V     rmsnorm prologue, RoPE, q and the K/V cache rows
+//   attention causal, fp32 MFMA (a decode step: the split attention of the
+//             quantised step kernels, step.hip)
+//   Wo        added into the hidden rows
+//   gate/up   rmsnorm prologue, silu(gate) * up
+//   W2        added into the hidden rows
+// The four projections are the fp32 matrix-core tile of gemm_f32.hpp with an
+// epilogue of their own (fgemm_kernel). One token is a tile of one row: what
+// the matrix cores do for the fifteen rows it leaves unused takes less time
+// than the weights take from HBM (a 16-column tile: 64 bytes of each of 32
+// weight rows per 256 cycles and SIMD, 39 GB/s per cycle and chip against
+// the 2.7 that HBM gives).
+// RMSNorm (src/ops.cpp:111-134) is folded in: the norm weights multiply A on
+// its way to the tile, every wave gathers its share of the row's squares,
+// and the row's factor 1 / sqrt(mean + 1e-5) multiplies the finished sums.
 #include "fmodel.hpp"
+#include "gemm_f32.hpp"
+#include "prefill.hpp"
 #include "runtime.hpp"
 
 #include <algorithm>
@@ -23,137 +31,358 @@ namespace nut {
 
 namespace {
 
-constexpr int kCols = 256;
-// a GEMV's partial sums, per projection: splits x out floats
-constexpr size_t kPartialFloats = size_t(1) << 20;
+// What the product of a launch becomes.
+enum FEpilogue { kFAdd, kFSwiglu, kFQkv };
 
-template <bool NORM>
-__global__ __launch_bounds__(kCols) void colgemv_kernel(const float *x, int in,
-                                                        const float *norm_w, const float *w,
-                                                        int out, int run, float *partial)
+struct FGemm {
+    const float *x, *norm_w; // rows [m][k], norm weights [k] (not kFAdd)
+    int m, k;
+    // the matrices, [k][n] each: q, k, v (kFQkv, column tiles in that order),
+    // gate and up (kFSwiglu, both in every tile) or the one (kFAdd)
+    const float *w[3];
+    int n[3], tiles[3];
+    int tiles_m, tiles_n;
+    float *out; // rows of n[0]: hidden rows, activations, query rows
+    const float2 *rope;
+    float *k_layer, *v_layer;
+    int first_pos, head_dim, max_seq;
+};
+
+template <int TI, int TJ, int WK, int D, int EPI>
+__global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
 {
-    extern __shared__ float xs[];
-    __shared__ float red[kCols / kWave];
-    const int k0 = blockIdx.y * run, k1 = min(in, k0 + run);
-    float scale = 1.0f;
+    constexpr bool NORM = EPI != kFAdd;
+    constexpr int NB = EPI == kFSwiglu ? 2 : 1, TB = TJ / NB;
+    constexpr int kStage = WK * 16 * TI * kChunkLd, kRed = WK * TJ * 256;
+    __shared__ __attribute__((aligned(16))) float lds[kStage > kRed ? kStage : kRed];
+    __shared__ float squares[NORM ? WK : 1][16 * TI];
+    int tm, tn;
+    if (!gemm_f32_tile(f.tiles_m, f.tiles_n, tm, tn))
+        return; // workgroup-uniform
+    int seg = 0;
+    if (EPI == kFQkv)
+        while (seg < 2 && tn >= f.tiles[seg])
+            tn -= f.tiles[seg++]; // workgroup-uniform
+    const int n = f.n[seg], m = f.m, k = f.k;
+    const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = tm * 16 * TI, col = tn * 16 * TB + TB * li;
+    const int first = min(col, n - TB); // n >= TB
+    const float *pa[2 * TI];
+#pragma unroll
+    for (int t = 0; t < 2 * TI; t++)
+        pa[t] = f.x + size_t(min(row0 + 8 * t + (lane >> 3), m - 1)) * k + 4 * (lane & 7);
+    const float *pb[NB];
+#pragma unroll
+    for (int q = 0; q < NB; q++)
+        pb[q] = f.w[EPI == kFSwiglu ? q : seg] + size_t(8 * g) * n + first;
+    floatx4 acc[1][TI][TJ];
+    float sq[2 * TI] = {};
+    gemm_f32_clear(acc);
+    int c0, c1;
+    bool tail;
+    gemm_f32_share<WK>(k, wave, c0, c1, tail);
+    gemm_f32_run<TI, TJ, NB, 0, D, NORM>(pa, pb, size_t(n),
+                                          NORM ? f.norm_w + 4 * (lane & 7) : nullptr, k, c0, c1,
+                                          tail, lds + wave * 16 * TI * kChunkLd, acc, sq);
     if (NORM) {
-        float sq = 0.0f;
-        for (int i = threadIdx.x; i < in; i += kCols)
-            sq = fmaf(x[i], x[i], sq);
-        scale = 1.0f / sqrtf(block_sum(sq, red, kCols / kWave) / float(in) + 1e-5f);
+        // eight lanes hold a row's squares of this wave's share
+#pragma unroll
+        for (int t = 0; t < 2 * TI; t++) {
+            float s = sq[t];
+            s += __shfl_xor(s, 1);
+            s += __shfl_xor(s, 2);
+            s += __shfl_xor(s, 4);
+            if ((lane & 7) == 0)
+                squares[wave][8 * t + (lane >> 3)] = s;
+        }
     }
-    for (int k = k0 + threadIdx.x; k < k1; k += kCols)
-        xs[k - k0] = NORM ? x[k] * scale * norm_w[k] : x[k];
     __syncthreads();
-    const int j = blockIdx.x * kCols + threadIdx.x;
-    if (j >= out)
+    gemm_f32_reduce<TI, TJ, WK>(acc, lds, wave, [&](int i, int v, float (&out)[TJ]) {
+        const int r = 16 * i + 4 * g + v, row = row0 + r;
+        if (row >= m || col >= n)
+            return;
+        if (NORM) {
+            float s = squares[0][r];
+#pragma unroll
+            for (int w = 1; w < WK; w++)
+                s += squares[w][r];
+            const float scale = 1.0f / sqrtf(s / float(k) + 1e-5f);
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+                out[j] *= scale;
+        }
+        float vals[TB];
+        float *dst;
+        if constexpr (EPI == kFSwiglu) {
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                vals[j] = out[j] / (1.0f + expf(-out[j])) * out[TB + j];
+            dst = f.out + size_t(row) * n + first;
+        } else if constexpr (EPI == kFAdd) {
+            dst = f.out + size_t(row) * n + first;
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                vals[j] = dst[j] + out[j];
+        } else {
+            // RoPE (rotate_vector, src/kvcache.cpp:48-59) on the pairs of q
+            // and k; TB, n and head_dim are even, so a pair is a lane's
+            static_assert(EPI != kFQkv || TB % 2 == 0, "whole RoPE pairs");
+            const int pos = f.first_pos + row;
+            const int head = first / f.head_dim, d = first % f.head_dim;
+#pragma unroll
+            for (int j = 0; j < TB; j += 2) {
+                float e = out[j], o = out[j + 1];
+                if (seg < 2) {
+                    const float2 cs = f.rope[size_t(pos) * (f.head_dim / 2) + (d + j) / 2];
+                    const float even = e, odd = o;
+                    e = fmaf(even, cs.x, -(odd * cs.y));
+                    o = fmaf(even, cs.y, odd * cs.x);
+                }
+                vals[j] = e;
+                vals[j + 1] = o;
+            }
+            if (seg == 0) {
+                dst = f.out + size_t(row) * n + first;
+            } else {
+                // head_dim is a multiple of 4 and TB 2 or 4, first a multiple
+                // of TB: a lane's columns are of one head
+                dst = (seg == 1 ? f.k_layer : f.v_layer) +
+                      (size_t(head) * f.max_seq + pos) * f.head_dim + d;
+            }
+        }
+        if (first == col) {
+            store_u<TB>(dst, vals);
+        } else {
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                if (first + j >= col)
+                    dst[j] = vals[j];
+        }
+    });
+}
+
+template <int TI, int TJ, int WK, int D, int EPI>
+void launch_ftile(FGemm &f, hipStream_t stream)
+{
+    const int cols = 16 * TJ / (EPI == kFSwiglu ? 2 : 1);
+    f.tiles_m = (f.m + 16 * TI - 1) / (16 * TI);
+    f.tiles_n = 0;
+    for (int s = 0; s < (EPI == kFQkv ? 3 : 1); s++) {
+        f.tiles[s] = (f.n[s] + cols - 1) / cols;
+        f.tiles_n += f.tiles[s];
+    }
+    hipLaunchKernelGGL((fgemm_kernel<TI, TJ, WK, D, EPI>),
+                       dim3(gemm_f32_grid(f.tiles_m, f.tiles_n)), dim3(64 * WK), 0, stream, f);
+    check_launch("fp32 model: projection");
+}
+
+// The tile by the model of gemm_f32_choose over all the launch's columns
+// (gate and up count twice). Up to 16 rows the weights' way from HBM is what
+// counts: sixteen waves share the k of a narrow tile, so that the whole chip
+// has its loads in flight at once.
+template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
+{
+    int n = f.n[0];
+    if (EPI == kFQkv)
+        n += f.n[1] + f.n[2];
+    if (EPI == kFSwiglu)
+        n *= 2;
+    if (f.m <= 16) {
+        if constexpr (EPI == kFAdd) {
+            n >= 4096 ? launch_ftile<1, 2, 16, 2, EPI>(f, stream)
+                      : launch_ftile<1, 1, 16, 3, EPI>(f, stream);
+        } else {
+            n >= 8192 ? launch_ftile<1, 4, 16, 1, EPI>(f, stream)
+                      : launch_ftile<1, 2, 16, 2, EPI>(f, stream);
+        }
         return;
-    const float *col = w + size_t(k0) * out + j;
-    float acc = 0.0f;
-    for (int k = 0; k < k1 - k0; k++)
-        acc = fmaf(xs[k], col[size_t(k) * out], acc);
-    partial[size_t(blockIdx.y) * out + j] = acc;
-}
-
-__device__ __forceinline__ float sum_parts(const float *partial, int splits, int out, int j)
-{
-    float s = 0.0f;
-    for (int p = 0; p < splits; p++)
-        s += partial[size_t(p) * out + j];
-    return s;
-}
-
-__global__ void residual_kernel(const float *partial, int splits, int out, float *h)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < out)
-        h[j] += sum_parts(partial, splits, out, j);
-}
-
-__global__ void swiglu_kernel(const float *pg, int gs, const float *pu, int us, int ffn,
-                              float *act)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < ffn) {
-        const float g = sum_parts(pg, gs, ffn, j), u = sum_parts(pu, us, ffn, j);
-        act[j] = g / (1.0f + expf(-g)) * u;
+    }
+    const GemmTile t = gemm_f32_choose(f.m, f.k, n);
+    switch (t.ti * 10 + t.tj) {
+    case 44:
+        launch_ftile<4, 4, 4, 1, EPI>(f, stream);
+        break;
+    case 34:
+    case 33: // whole RoPE pairs, and gate and up alike
+        launch_ftile<3, 4, 4, 2, EPI>(f, stream);
+        break;
+    case 24:
+        launch_ftile<2, 4, 4, 2, EPI>(f, stream);
+        break;
+    case 22:
+        launch_ftile<2, 2, 8, 1, EPI>(f, stream);
+        break;
+    default:
+        launch_ftile<1, 2, 8, 2, EPI>(f, stream);
     }
 }
 
-// attention_step's projections after the matvecs (src/kvcache.cpp:84-100):
-// column pairs of q, k, v; RoPE (rotate_vector, lines 48-59) on q and k with
-// the host-built table; k and v stored at position *length.
-__global__ void qkv_kernel(const float *pq, int qs, const float *pk, int ks, const float *pv,
-                           int vs, DecodeShape s, const float2 *rope, const int *length,
-                           float *query, float *k_layer, float *v_layer)
+// Causal attention of a prompt's T rows (src/kvcache.cpp:102-130 for every
+// row) on v_mfma_f32_16x16x4f32: one wave per (16 query rows, head), over
+// blocks of KB keys. Scores S = Q K^T with both operands read as rows, lane
+// group g holding dims [g HD / 4, (g + 1) HD / 4) of row li, so a lane's
+// values are consecutive; the online softmax on S in registers (a score row
+// is one 16-lane DPP row); P through LDS into the A layout; O += P V with V
+// read as rows (lane li: dims TJ li ..). The next block's K and V loads are
+// in flight while one block is used.
+// A key past a row's own position has weight 0; where such a key's V is not
+// finite (0 times it would not be 0) the block is summed key by key instead.
+template <int HD>
+__global__ __launch_bounds__(64) void fattention_kernel(const float *q, const float *k_layer,
+                                                        const float *v_layer, float *ctx, int t,
+                                                        int heads, int kv_heads, int max_seq,
+                                                        float scale)
 {
-    const int kvd = s.kv_heads * s.head_dim;
-    const int pairs = s.dim / 2 + kvd;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= pairs)
-        return;
-    const int pos = *length;
-    int which, c;
-    if (t < s.dim / 2) {
-        which = 0;
-        c = 2 * t;
-    } else if (t < s.dim / 2 + kvd / 2) {
-        which = 1;
-        c = 2 * (t - s.dim / 2);
-    } else {
-        which = 2;
-        c = 2 * (t - s.dim / 2 - kvd / 2);
+    constexpr int QS = HD / 4;             // dims per lane group
+    constexpr int KT = HD == 128 ? 2 : 4;  // 16-key tiles per block
+    constexpr int KB = 16 * KT;
+    constexpr int TJ = HD / 16;            // output columns per lane
+    constexpr int PLD = KB + 4;
+    __shared__ __attribute__((aligned(16))) float ps[16 * PLD];
+    const int lane = threadIdx.x, li = lane & 15, g = lane >> 4;
+    const int head = blockIdx.x, kvh = head / (heads / kv_heads);
+    // the last rows (the most keys) are dispatched first
+    const int row0 = int(gridDim.y - 1 - blockIdx.y) * 16;
+    const size_t ldq = size_t(heads) * HD;
+    const float *kh = k_layer + size_t(kvh) * max_seq * HD;
+    const float *vh = v_layer + size_t(kvh) * max_seq * HD;
+    float qf[QS];
+    {
+        const float *src = q + size_t(min(row0 + li, t - 1)) * ldq + size_t(head) * HD + g * QS;
+#pragma unroll
+        for (int s = 0; s < QS; s += 4)
+            load_u<4>(src + s, &qf[s]);
     }
-    const float *part = which == 0 ? pq : which == 1 ? pk : pv;
-    const int splits = which == 0 ? qs : which == 1 ? ks : vs;
-    const int out = which == 0 ? s.dim : kvd;
-    float e = sum_parts(part, splits, out, c), o = sum_parts(part, splits, out, c + 1);
-    const int head = c / s.head_dim, d = c % s.head_dim;
-    if (which < 2) {
-        const float2 cs = rope[size_t(pos) * (s.head_dim / 2) + d / 2];
-        const float even = e, odd = o;
-        e = fmaf(even, cs.x, -(odd * cs.y));
-        o = fmaf(even, cs.y, odd * cs.x);
+    floatx4 o[TJ];
+#pragma unroll
+    for (int j = 0; j < TJ; j++)
+        o[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    float mx[4], sum[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        mx[v] = -INFINITY;
+        sum[v] = 0.0f;
     }
-    if (which == 0) {
-        query[c] = e;
-        query[c + 1] = o;
-    } else {
-        float *cache = (which == 1 ? k_layer : v_layer) +
-                       (size_t(head) * s.max_seq + pos) * s.head_dim + d;
-        cache[0] = e;
-        cache[1] = o;
+    const int keys = min(row0 + 16, t); // keys any of the rows sees
+    float kf[KT][QS], vf[KB / 4][TJ];
+    auto load_k = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < KT; u++) {
+            const float *src = kh + size_t(min(b + 16 * u + li, t - 1)) * HD + g * QS;
+#pragma unroll
+            for (int s = 0; s < QS; s += 4)
+                load_u<4>(src + s, &kf[u][s]);
+        }
+    };
+    // key 16 u + 4 g + s of the block in vf[4 u + s]
+    auto load_v = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < KT; u++)
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                load_u<TJ>(vh + size_t(min(b + 16 * u + 4 * g + s, t - 1)) * HD + TJ * li,
+                           vf[4 * u + s]);
+    };
+    load_k(0);
+    load_v(0);
+    for (int b = 0; b < keys; b += KB) {
+        floatx4 sc[KT];
+#pragma unroll
+        for (int u = 0; u < KT; u++)
+            sc[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < QS; s++)
+#pragma unroll
+            for (int u = 0; u < KT; u++)
+                sc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[s], kf[u][s], sc[u], 0, 0, 0);
+        if (b + KB < keys)
+            load_k(b + KB);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = row0 + 4 * g + v;
+            float m = mx[v];
+#pragma unroll
+            for (int u = 0; u < KT; u++) {
+                const float x = sc[u][v] * scale;
+                sc[u][v] = b + 16 * u + li <= row ? x : -INFINITY;
+                m = fmaxf(m, sc[u][v]);
+            }
+            m = row16_max(m);
+            // no key with a score above -inf yet: weights 0, not NaN
+            const float base = m == -INFINITY ? 0.0f : m;
+            const float alpha = expf(mx[v] - base);
+            mx[v] = m;
+            float part = 0.0f;
+#pragma unroll
+            for (int u = 0; u < KT; u++) {
+                const float e = expf(sc[u][v] - base);
+                part += e;
+                ps[(4 * g + v) * PLD + 16 * u + li] = e;
+            }
+            sum[v] = sum[v] * alpha + row16_sum(part);
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+                o[j][v] *= alpha;
+        }
+        __syncthreads(); // one wave: orders the LDS accesses
+        bool apart = false;
+        if (b + KB > row0 + 1) { // wave-uniform: keys past some row
+            bool finite = true;
+#pragma unroll
+            for (int e = 0; e < KB / 4; e++)
+#pragma unroll
+                for (int j = 0; j < TJ; j++)
+                    finite = finite && isfinite(vf[e][j]);
+            apart = !__all(finite);
+        }
+        if (!apart) {
+#pragma unroll
+            for (int u = 0; u < KT; u++) {
+                const float4 p4 =
+                    *reinterpret_cast<const float4 *>(&ps[li * PLD + 16 * u + 4 * g]);
+                const float p[4] = {p4.x, p4.y, p4.z, p4.w};
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+#pragma unroll
+                    for (int j = 0; j < TJ; j++)
+                        o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], vf[4 * u + s][j], o[j],
+                                                                    0, 0, 0);
+            }
+        } else {
+            for (int e = 0; e < KB && b + e < keys; e++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (b + e <= row0 + 4 * g + v)
+#pragma unroll
+                        for (int j = 0; j < TJ; j++)
+                            o[j][v] = fmaf(ps[(4 * g + v) * PLD + e],
+                                           vh[size_t(b + e) * HD + TJ * li + j], o[j][v]);
+        }
+        if (b + KB < keys)
+            load_v(b + KB);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = row0 + 4 * g + v;
+        if (row < t) {
+            float out[TJ];
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+                out[j] = o[j][v] / sum[v];
+            store_u<TJ>(ctx + size_t(row) * ldq + size_t(head) * HD + TJ * li, out);
+        }
     }
 }
 
-__global__ void copy_kernel(const float *src, float *dst, int n)
+template <int HD>
+void launch_fattention(const DecodeShape &s, const float *q, const float *kc, const float *vc,
+                       float *ctx, int t, hipStream_t stream)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        dst[i] = src[i];
-}
-
-int blocks(int n) { return (n + 255) / 256; }
-
-// partial <- the GEMV of x (rmsnorm'd with norm_w when given) by w
-// [in x out]; returns the number of partial rows (splits).
-int colgemv(const float *x, int in, const float *norm_w, const float *w, int out,
-            float *partial, hipStream_t stream)
-{
-    const int col_blocks = (out + kCols - 1) / kCols;
-    int splits = std::max(1, std::min((1024 + col_blocks - 1) / col_blocks, (in + 31) / 32));
-    splits = std::max(1, std::min<int>(splits, int(kPartialFloats / size_t(out))));
-    const int run = (in + splits - 1) / splits;
-    splits = (in + run - 1) / run;
-    const size_t lds = size_t(run) * sizeof(float);
-    if (norm_w != nullptr)
-        hipLaunchKernelGGL(colgemv_kernel<true>, dim3(col_blocks, splits), dim3(kCols), lds,
-                           stream, x, in, norm_w, w, out, run, partial);
-    else
-        hipLaunchKernelGGL(colgemv_kernel<false>, dim3(col_blocks, splits), dim3(kCols), lds,
-                           stream, x, in, nullptr, w, out, run, partial);
-    check_launch("fp32 decode: projection");
-    return splits;
+    hipLaunchKernelGGL(fattention_kernel<HD>, dim3(s.heads, (t + 15) / 16), dim3(64), 0, stream,
+                       q, kc, vc, ctx, t, s.heads, s.kv_heads, s.max_seq, s.attn_scale);
+    check_launch("fp32 prefill: attention");
 }
 
 void check_fready(const nut_fmodel &m)
@@ -163,46 +392,68 @@ void check_fready(const nut_fmodel &m)
         require(l.set, NUT_EINVAL, "kv cache: layer count mismatch");
 }
 
-// One token through every layer at position *length (device), its hidden
-// state left in m.hidden; the device length advances.
-void enqueue_token(nut_fmodel &m, nut_kvcache &kv, int token)
+// The t tokens whose embeddings stand in h through every layer at positions
+// first .. first + t - 1 (first == 0 unless t == 1); their hidden states
+// stay in h.
+void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, float *q,
+                    float *ctx, float *act)
 {
     const DecodeShape &s = m.shape;
-    const nut_config &c = m.config;
     const int kvd = s.kv_heads * s.head_dim;
-    StepState *state = m.state.as<StepState>();
-    float *h = m.hidden.as<float>(), *q = m.query.as<float>(), *ctx = m.context.as<float>(),
-          *act = m.act.as<float>();
-    float *p0 = m.partial.as<float>(), *p1 = p0 + kPartialFloats, *p2 = p1 + kPartialFloats;
-    launch_reset_state(state, token, m.stream);
-    launch_embed(s, m.embeddings.as<float>(), &state->token, state, h, m.stream);
     const size_t layer_elems = kv.layer_elements();
-    for (size_t l = 0; l < c.layers; l++) {
+    const StepState *state = m.state.as<StepState>();
+    const int *length = kv.device_length.as<int>();
+    for (size_t l = 0; l < m.config.layers; l++) {
         const nut_fmodel::Layer &L = m.layers[l];
         float *kc = kv.keys.as<float>() + l * layer_elems;
         float *vc = kv.values.as<float>() + l * layer_elems;
-        const float *an = L.attention_norm.as<float>(), *fn = L.ffn_norm.as<float>();
-        const int qs = colgemv(h, s.dim, an, L.w[0].as<float>(), s.dim, p0, m.stream);
-        const int ks = colgemv(h, s.dim, an, L.w[1].as<float>(), kvd, p1, m.stream);
-        const int vs = colgemv(h, s.dim, an, L.w[2].as<float>(), kvd, p2, m.stream);
-        hipLaunchKernelGGL(qkv_kernel, dim3(blocks(s.dim / 2 + kvd)), dim3(256), 0, m.stream, p0,
-                           qs, p1, ks, p2, vs, s, m.rope.as<float2>(),
-                           kv.device_length.as<int>(), q, kc, vc);
-        check_launch("fp32 decode: rope and cache store");
-        launch_attention(s, q, kc, vc, kv.device_length.as<int>(), ctx, state, m.stream);
-        const int os = colgemv(ctx, s.dim, nullptr, L.w[3].as<float>(), s.dim, p0, m.stream);
-        hipLaunchKernelGGL(residual_kernel, dim3(blocks(s.dim)), dim3(256), 0, m.stream, p0, os,
-                           s.dim, h);
-        const int gs = colgemv(h, s.dim, fn, L.w[4].as<float>(), s.ffn_dim, p1, m.stream);
-        const int us = colgemv(h, s.dim, fn, L.w[5].as<float>(), s.ffn_dim, p2, m.stream);
-        hipLaunchKernelGGL(swiglu_kernel, dim3(blocks(s.ffn_dim)), dim3(256), 0, m.stream, p1, gs,
-                           p2, us, s.ffn_dim, act);
-        const int ds = colgemv(act, s.ffn_dim, nullptr, L.w[6].as<float>(), s.dim, p0, m.stream);
-        hipLaunchKernelGGL(residual_kernel, dim3(blocks(s.dim)), dim3(256), 0, m.stream, p0, ds,
-                           s.dim, h);
-        check_launch("fp32 decode: epilogue");
+        FGemm f{};
+        f.m = t;
+        f.rope = m.rope.as<float2>();
+        f.k_layer = kc;
+        f.v_layer = vc;
+        f.first_pos = first;
+        f.head_dim = s.head_dim;
+        f.max_seq = s.max_seq;
+        auto gemm = [&](const float *x, const DeviceBuffer *norm, int k, int w0, int count, int n0,
+                        float *out) {
+            f.x = x;
+            f.norm_w = norm != nullptr ? norm->as<float>() : nullptr;
+            f.k = k;
+            for (int i = 0; i < count; i++) {
+                f.w[i] = L.w[w0 + i].as<float>();
+                f.n[i] = i == 0 ? n0 : w0 == 0 ? kvd : n0;
+            }
+            f.out = out;
+        };
+        gemm(h, &L.attention_norm, s.dim, 0, 3, s.dim, q);
+        launch_fgemm<kFQkv>(f, m.stream);
+        if (t == 1 && m.split_attention) {
+            launch_attention_split(s, q, kc, vc, length, m.attn_part.as<uint64_t>(),
+                                   m.attn_count.as<int>(), ctx, state, m.stream);
+        } else if (first == 0 && s.head_dim == 64) {
+            launch_fattention<64>(s, q, kc, vc, ctx, t, m.stream);
+        } else if (first == 0 && s.head_dim == 128) {
+            launch_fattention<128>(s, q, kc, vc, ctx, t, m.stream);
+        } else if (first == 0 && s.head_dim == 32) {
+            launch_fattention<32>(s, q, kc, vc, ctx, t, m.stream);
+        } else if (first == 0 && s.head_dim == 16) {
+            launch_fattention<16>(s, q, kc, vc, ctx, t, m.stream);
+        } else {
+            for (int i = 0; i < t; i++) {
+                if (t > 1)
+                    launch_set_int(kv.device_length.as<int>(), first + i, m.stream);
+                launch_attention(s, q + size_t(i) * s.dim, kc, vc, length, ctx + size_t(i) * s.dim,
+                                 state, m.stream);
+            }
+        }
+        gemm(ctx, nullptr, s.dim, 3, 1, s.dim, h);
+        launch_fgemm<kFAdd>(f, m.stream);
+        gemm(h, &L.ffn_norm, s.dim, 4, 2, s.ffn_dim, act);
+        launch_fgemm<kFSwiglu>(f, m.stream);
+        gemm(act, nullptr, s.ffn_dim, 6, 1, s.dim, h);
+        launch_fgemm<kFAdd>(f, m.stream);
     }
-    launch_finish_step(state, kv.device_length.as<int>(), m.stream);
 }
 
 void check_cache(const nut_fmodel &m, const nut_kvcache &kv)
@@ -248,10 +499,22 @@ nut_fmodel *create_fmodel(const nut_config &config, bool tied)
     m->query.allocate(config.dim * sizeof(float));
     m->context.allocate(config.dim * sizeof(float));
     m->act.allocate(config.ffn_dim * sizeof(float));
-    m->partial.allocate(3 * kPartialFloats * sizeof(float));
     m->state.allocate(sizeof(StepState));
     m->token.allocate(sizeof(int));
     hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "hipStreamCreate");
+    // the attention kernels' stop flag: never set on this path
+    launch_reset_state(m->state.as<StepState>(), 0, m->stream);
+    m->split_attention = attention_split_supported(s);
+    if (m->split_attention) {
+        // one token's partial results (no word carries a live tag) and
+        // arrival counters
+        const size_t part = step_attn_part_words(s) / kStepTokensMax * sizeof(uint64_t);
+        const size_t count = 2 * size_t(s.heads) * sizeof(int);
+        m->attn_part.allocate(part);
+        m->attn_count.allocate(count);
+        hip_check(hipMemsetAsync(m->attn_part.get(), 0xff, part, m->stream), "hipMemsetAsync");
+        hip_check(hipMemsetAsync(m->attn_count.get(), 0, count, m->stream), "hipMemsetAsync");
+    }
     return m.release();
 }
 
@@ -295,7 +558,11 @@ void decode_token(nut_fmodel &m, nut_kvcache &kv, int token, float *hidden)
     require(token >= 0 && size_t(token) < m.config.vocab_size, NUT_EOUTOFRANGE,
             "kv cache: token id out of range");
     kv.sync_length(m.stream);
-    enqueue_token(m, kv, token);
+    launch_set_int(m.token.as<int>(), token, m.stream);
+    launch_embed_rows(m.embeddings.as<float>(), m.token.as<int>(), m.hidden.as<float>(), 1,
+                      m.shape.dim, m.stream);
+    enqueue_layers(m, kv, m.hidden.as<float>(), 1, int(kv.length), m.query.as<float>(),
+                   m.context.as<float>(), m.act.as<float>());
     if (hidden != nullptr)
         hip_check(hipMemcpyAsync(hidden, m.hidden.get(), m.config.dim * sizeof(float),
                                  hipMemcpyDeviceToHost, m.stream),
@@ -316,15 +583,26 @@ void prefill_tokens(nut_fmodel &m, nut_kvcache &kv, const int *tokens, size_t co
     for (size_t t = 0; t < count; t++)
         require(tokens[t] >= 0 && size_t(tokens[t]) < m.config.vocab_size, NUT_EOUTOFRANGE,
                 "kv cache: token id out of range");
-    DeviceBuffer out(count * m.config.dim * sizeof(float));
-    launch_set_int(kv.device_length.as<int>(), 0, m.stream);
-    for (size_t t = 0; t < count; t++) {
-        enqueue_token(m, kv, tokens[t]);
-        hipLaunchKernelGGL(copy_kernel, dim3(blocks(m.shape.dim)), dim3(256), 0, m.stream,
-                           m.hidden.as<float>(), out.as<float>() + t * m.config.dim, m.shape.dim);
+    if (count > m.rows_held) {
+        // rows of every activation for the longest prompt so far
+        m.rows_held = 0;
+        m.pf_tokens.allocate(count * sizeof(int));
+        m.pf_h.allocate(count * m.config.dim * sizeof(float));
+        m.pf_q.allocate(count * m.config.dim * sizeof(float));
+        m.pf_ctx.allocate(count * m.config.dim * sizeof(float));
+        m.pf_act.allocate(count * m.config.ffn_dim * sizeof(float));
+        m.rows_held = count;
     }
+    hip_check(hipMemcpyAsync(m.pf_tokens.get(), tokens, count * sizeof(int),
+                             hipMemcpyHostToDevice, m.stream),
+              "hipMemcpyAsync");
+    launch_set_int(kv.device_length.as<int>(), 0, m.stream);
+    launch_embed_rows(m.embeddings.as<float>(), m.pf_tokens.as<int>(), m.pf_h.as<float>(),
+                      int(count), m.shape.dim, m.stream);
+    enqueue_layers(m, kv, m.pf_h.as<float>(), int(count), 0, m.pf_q.as<float>(),
+                   m.pf_ctx.as<float>(), m.pf_act.as<float>());
     if (rows != nullptr)
-        hip_check(hipMemcpyAsync(rows, out.get(), count * m.config.dim * sizeof(float),
+        hip_check(hipMemcpyAsync(rows, m.pf_h.get(), count * m.config.dim * sizeof(float),
                                  hipMemcpyDeviceToHost, m.stream),
                   "hipMemcpyAsync");
     hip_check(hipStreamSynchronize(m.stream), "hipStreamSynchronize");

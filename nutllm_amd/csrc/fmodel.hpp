@@ -24,7 +24,13 @@ struct nut_fmodel {
     std::vector<Layer> layers;
     nut::DeviceBuffer embeddings, final_norm, lm_head, rope;
     // workspace of one decode step
-    nut::DeviceBuffer hidden, query, context, act, partial, state, token;
+    nut::DeviceBuffer hidden, query, context, act, state, token;
+    // a decode step's split attention (step.hip), where the shape has it
+    bool split_attention = false;
+    nut::DeviceBuffer attn_part, attn_count;
+    // a prompt's rows, for rows_held tokens
+    nut::DeviceBuffer pf_tokens, pf_h, pf_q, pf_ctx, pf_act;
+    size_t rows_held = 0;
     hipStream_t stream = nullptr;
     ~nut_fmodel();
 };

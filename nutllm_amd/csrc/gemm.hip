@@ -26,10 +26,11 @@ void launch_matmul_f32(const float *a, const float *b, float *c, int m, int k,
 {
     const GemmTile t = gemm_f32_choose(m, k, n);
     // Eight waves per tile where the grid gives a CU one workgroup of a small
-    // tile (33 x 4001 x 3333: 25.7 us against 30.4 with four), four elsewhere.
+    // tile and k gives every wave a chunk (33 x 4001 x 3333: 25.7 us against
+    // 30.4 with four), four elsewhere.
     // Two accumulators per output keep a chain of additions as short as eight
     // waves' (768^3: rel error 1.8e-7 against 2.5e-7 with one).
-    const bool deep = t.count <= 256;
+    const bool deep = t.count <= 256 && k >= 8 * kChunk;
     switch (t.ti * 10 + t.tj) {
     case 44:
         launch_tile<4, 4, 4, 1, 1>(a, b, c, m, k, n, stream);

@@ -74,12 +74,16 @@ constexpr int kChunkLd = 36; // floats per A row in LDS: 16-byte reads of 16
 // it (each supplies TJ / NB columns per lane). NORM: A's values are
 // multiplied by nw[k] (nw at 4 (lane % 8)) and sq[t] gathers the squares of
 // the values before that. NA: accumulators per output, each taking a run of
-// a chunk's k (shorter chains of additions, a smaller rounding error).
+// a chunk's k (shorter chains of additions, a smaller rounding error); NA 0:
+// one accumulator, to which every chunk's own sum is added, the shortest
+// chains of all.
+constexpr int gemm_f32_accs(int na) { return na == 0 ? 1 : na; }
+
 template <int TI, int TJ, int NB, int NA, int D, bool NORM>
 __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
                                              const float *const (&pb)[NB], size_t ldb,
                                              const float *nw, int k, int c0, int c1, bool tail,
-                                             float *as, floatx4 (&acc)[NA][TI][TJ],
+                                             float *as, floatx4 (&acc)[gemm_f32_accs(NA)][TI][TJ],
                                              float (&sq)[2 * TI])
 {
     constexpr int TB = TJ / NB;
@@ -140,14 +144,32 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
                 fa[i][4 * h + 3] = v.w;
             }
         __builtin_amdgcn_wave_barrier();
+        if constexpr (NA == 0) {
+            floatx4 part[TI][TJ];
 #pragma unroll
-        for (int s = 0; s < 8; s++)
+            for (int s = 0; s < 8; s++)
+#pragma unroll
+                for (int i = 0; i < TI; i++)
+#pragma unroll
+                    for (int j = 0; j < TJ; j++)
+                        part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            fa[i][s], fb[s][j],
+                            s == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : part[i][j], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < TI; i++)
 #pragma unroll
                 for (int j = 0; j < TJ; j++)
-                    acc[s * NA / 8][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        fa[i][s], fb[s][j], acc[s * NA / 8][i][j], 0, 0, 0);
+                    acc[0][i][j] += part[i][j];
+        } else {
+#pragma unroll
+            for (int s = 0; s < 8; s++)
+#pragma unroll
+                for (int i = 0; i < TI; i++)
+#pragma unroll
+                    for (int j = 0; j < TJ; j++)
+                        acc[s * NA / 8][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            fa[i][s], fb[s][j], acc[s * NA / 8][i][j], 0, 0, 0);
+        }
     };
     const int count = c1 - c0;
 #pragma unroll
@@ -225,14 +247,14 @@ __device__ __forceinline__ void gemm_f32_clear(floatx4 (&acc)[NA][TI][TJ])
 // row's columns to epi(i, v, vals): row 16 i + 4 g + v of the tile, this
 // lane's TJ columns. Wave wk takes the v of 4 wk / WK ..; called by the whole
 // workgroup.
-template <int TI, int TJ, int WK, int NA, class Epi>
-__device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NA][TI][TJ], float *red,
+template <int TI, int TJ, int WK, int NS, class Epi>
+__device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NS][TI][TJ], float *red,
                                                 int wk, Epi &&epi)
 {
     const int lane = threadIdx.x & 63;
     floatx4(&acc)[TI][TJ] = parts[0];
 #pragma unroll
-    for (int u = 1; u < NA; u++)
+    for (int u = 1; u < NS; u++)
 #pragma unroll
         for (int i = 0; i < TI; i++)
 #pragma unroll
@@ -366,7 +388,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f32_wave(
     for (int t = 0; t < 2 * TI; t++)
         pa[t] = a + size_t(min(row0 + 8 * t + (lane >> 3), m - 1)) * k + 4 * (lane & 7);
     const float *pb[1] = {b + size_t(8 * g) * n + first};
-    floatx4 acc[NA][TI][TJ];
+    floatx4 acc[gemm_f32_accs(NA)][TI][TJ];
     float sq[2 * TI] = {};
     gemm_f32_clear(acc);
     int c0, c1;
@@ -376,7 +398,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f32_wave(
                                     lds + wave * 16 * TI * kChunkLd, acc, sq);
     if (WK > 1)
         __syncthreads();
-    gemm_f32_reduce<TI, TJ, WK, NA>(
+    gemm_f32_reduce<TI, TJ, WK>(
         acc, lds + (wm * WN + wn) * WK * TJ * 256, wk,
         [&](int i, int v, const float (&out)[TJ]) {
             const int row = row0 + 16 * i + 4 * g + v;

@@ -122,6 +122,13 @@ struct StepBuffers {
 };
 bool step_fast_supported(const DecodeShape &s, const LayerView &w);
 size_t step_attn_part_words(const DecodeShape &s);
+// The step kernels' attention alone, for one token at position *length:
+// query and context [heads][head_dim], part step_attn_part_words(s) /
+// kStepTokensMax words and count 2 * heads ints, kept as in StepBuffers.
+bool attention_split_supported(const DecodeShape &s);
+void launch_attention_split(const DecodeShape &s, const float *query, const float *k_layer,
+                            const float *v_layer, const int *length, uint64_t *part, int *count,
+                            float *context, const StepState *state, hipStream_t stream);
 void launch_layer_fast(const DecodeShape &s, const LayerView &w,
                        const float2 *rope, const int *length, float *k_layer,
                        float *v_layer, const StepBuffers &b, int tokens,

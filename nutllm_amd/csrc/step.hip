@@ -674,14 +674,28 @@ bool step_fast_supported(const DecodeShape &s, const LayerView &w)
     for (const QMat *m : mats)
         if (!fast_layout(*m) || m->type != w.query.type)
             return false;
-    const int group = s.kv_heads > 0 ? s.heads / s.kv_heads : 0;
     // the staged x of every matvec fits a workgroup's 64 KB of LDS
     const int cols = std::max(s.dim, s.ffn_dim);
     const size_t staged = w.query.type == 1 ? staged_x_bytes<1>(cols) : staged_x_bytes<0>(cols);
-    return (s.head_dim == 64 || s.head_dim == 128) && staged <= 65536 &&
-           s.heads == group * s.kv_heads &&
-           (group == 1 || group == 2 || group == 4 || group == 8) &&
-           s.dim % 2 == 0 && (s.kv_heads * s.head_dim) % 2 == 0;
+    return attention_split_supported(s) && staged <= 65536 && s.dim % 2 == 0 &&
+           (s.kv_heads * s.head_dim) % 2 == 0;
+}
+
+bool attention_split_supported(const DecodeShape &s)
+{
+    const int group = s.kv_heads > 0 ? s.heads / s.kv_heads : 0;
+    return (s.head_dim == 64 || s.head_dim == 128) && s.heads == group * s.kv_heads &&
+           (group == 1 || group == 2 || group == 4 || group == 8);
+}
+
+void launch_attention_split(const DecodeShape &s, const float *query, const float *k_layer,
+                            const float *v_layer, const int *length, uint64_t *part, int *count,
+                            float *context, const StepState *state, hipStream_t stream)
+{
+    const StepBuffers b{nullptr, const_cast<float *>(query), context, nullptr, part, count};
+    s.head_dim == 128 ? launch_attention_g<128>(s, k_layer, v_layer, length, b, 1, state, stream)
+                      : launch_attention_g<64>(s, k_layer, v_layer, length, b, 1, state, stream);
+    check_launch("decode: attention");
 }
 
 size_t step_attn_part_words(const DecodeShape &s)

@@ -193,7 +193,7 @@ template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
             n >= 4096 ? launch_ftile<1, 2, 16, 2, EPI>(f, stream)
                       : launch_ftile<1, 1, 16, 3, EPI>(f, stream);
         } else {
-            n >= 8192 ? launch_ftile<1, 4, 16, 1, EPI>(f, stream)
+            n >= 8192 ? launch_ftile<1, 4, 8, 1, EPI>(f, stream)
                       : launch_ftile<1, 2, 16, 2, EPI>(f, stream);
         }
         return;

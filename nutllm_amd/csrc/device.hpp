@@ -167,41 +167,48 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v)
 // Byte b of word j holds weights 8j+2b (low nibble) and 8j+2b+1 (high).
 // High nibbles are converted in place (16 u) and their accumulator scaled
 // by 1/16 once; power-of-two scaling commutes with rounding, so the result
-// equals accumulating u x.
+// equals accumulating u x. SIGNED: sum_k q_k x[k] instead, the offset taken
+// off every code (one more operation a weight, and partial sums without the
+// offset's share, whose rounding is most of the other form's error).
+template <bool SIGNED = false>
 __device__ __forceinline__ float dot_int4_chunk(uint4 w, const float *x)
 {
     const uint32_t words[4] = {w.x, w.y, w.z, w.w};
+    constexpr float kLo = SIGNED ? 8.0f : 0.0f, kHi = SIGNED ? 128.0f : 0.0f;
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const uint32_t lo = opaque((words[j] ^ 0x88888888u) & 0x0f0f0f0fu);
         const uint32_t hi = opaque((words[j] ^ 0x88888888u) & 0xf0f0f0f0u);
         const float *xs = x + 8 * j;
-        a0 = fmaf(ubyte0(lo), xs[0], a0);
-        a1 = fmaf(ubyte0(hi), xs[1], a1);
-        a0 = fmaf(ubyte1(lo), xs[2], a0);
-        a1 = fmaf(ubyte1(hi), xs[3], a1);
-        a0 = fmaf(ubyte2(lo), xs[4], a0);
-        a1 = fmaf(ubyte2(hi), xs[5], a1);
-        a0 = fmaf(ubyte3(lo), xs[6], a0);
-        a1 = fmaf(ubyte3(hi), xs[7], a1);
+        a0 = fmaf(ubyte0(lo) - kLo, xs[0], a0);
+        a1 = fmaf(ubyte0(hi) - kHi, xs[1], a1);
+        a0 = fmaf(ubyte1(lo) - kLo, xs[2], a0);
+        a1 = fmaf(ubyte1(hi) - kHi, xs[3], a1);
+        a0 = fmaf(ubyte2(lo) - kLo, xs[4], a0);
+        a1 = fmaf(ubyte2(hi) - kHi, xs[5], a1);
+        a0 = fmaf(ubyte3(lo) - kLo, xs[6], a0);
+        a1 = fmaf(ubyte3(hi) - kHi, xs[7], a1);
     }
     return fmaf(a1, 0.0625f, a0);
 }
 
-// sum_k u_k x[k] over one INT8 chunk (16 weights, offset-binary codes).
+// sum_k u_k x[k] over one INT8 chunk (16 weights, offset-binary codes), or
+// sum_k q_k x[k] (SIGNED).
+template <bool SIGNED = false>
 __device__ __forceinline__ float dot_int8_chunk(uint4 w, const float *x)
 {
     const uint32_t words[4] = {w.x ^ 0x80808080u, w.y ^ 0x80808080u,
                                w.z ^ 0x80808080u, w.w ^ 0x80808080u};
+    constexpr float kOff = SIGNED ? 128.0f : 0.0f;
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const float *xs = x + 4 * j;
-        a0 = fmaf(ubyte0(words[j]), xs[0], a0);
-        a1 = fmaf(ubyte1(words[j]), xs[1], a1);
-        a0 = fmaf(ubyte2(words[j]), xs[2], a0);
-        a1 = fmaf(ubyte3(words[j]), xs[3], a1);
+        a0 = fmaf(ubyte0(words[j]) - kOff, xs[0], a0);
+        a1 = fmaf(ubyte1(words[j]) - kOff, xs[1], a1);
+        a0 = fmaf(ubyte2(words[j]) - kOff, xs[2], a0);
+        a1 = fmaf(ubyte3(words[j]) - kOff, xs[3], a1);
     }
     return a0 + a1;
 }
@@ -213,9 +220,18 @@ struct QMat {
     int rows, cols, block_size, type; // type: 0 INT8, 1 INT4
 };
 
+// Whole blocks along the rows, of 32, 64, 128, ... weights: every 16-byte
+// chunk lies in one block, whose index within its row is the chunk's 32-wide
+// group shifted right by scale_shift(m).
 __host__ __device__ __forceinline__ bool fast_layout(const QMat &m)
 {
-    return m.block_size == 32 && (m.cols & 31) == 0;
+    return m.block_size >= 32 && (m.block_size & (m.block_size - 1)) == 0 &&
+           m.cols % m.block_size == 0;
+}
+
+__host__ __device__ __forceinline__ int scale_shift(const QMat &m)
+{
+    return __builtin_ctz(unsigned(m.block_size)) - 5;
 }
 
 // Weights per 16-byte chunk.
@@ -255,7 +271,8 @@ __device__ __forceinline__ void qrows_fast(const QMat &m, int row0,
     const bool int4 = m.type == 1;
     const int row_bytes = int4 ? m.cols / 2 : m.cols;
     const int chunks = row_bytes / 16;
-    const int blocks_per_row = m.cols / 32;
+    const int shift = scale_shift(m);
+    const int blocks_per_row = m.cols >> (shift + 5);
     const float bias = int4 ? 8.0f : 128.0f;
     float acc[R];
 #pragma unroll
@@ -264,7 +281,7 @@ __device__ __forceinline__ void qrows_fast(const QMat &m, int row0,
     for (int c = lane; c < chunks; c += kWave) {
         uint4 w[R];
         float s[R];
-        const int block = int4 ? c : (c >> 1);
+        const int block = (int4 ? c : (c >> 1)) >> shift;
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int rr = min(row0 + r, m.rows - 1);

@@ -103,8 +103,8 @@ void launch_classifier_screen(const float *weights, int vocab, int dim, int8_t *
 void launch_pick_token(const DecodeShape &s, const float *part_val,
                        const int *part_idx, int parts, StepState *state,
                        int *tokens, hipStream_t stream);
-// Fast step kernels (step.hip): layers whose matrices all use 32-wide
-// blocks along whole rows, head_dim 64 or 128, 1, 2, 4 or 8 query heads per
+// Fast step kernels (step.hip): layers whose matrices all use blocks of one
+// size, 32, 64, ..., along whole rows, head_dim 64 or 128, 1, 2, 4 or 8 query heads per
 // KV head. One launch runs 1 .. kStepTokensMax consecutive tokens at
 // positions *length, *length + 1, ...: hidden, query and context hold a
 // [tokens][dim] row per token, act a [tokens][ffn] row. attn_part holds

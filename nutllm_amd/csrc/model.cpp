@@ -674,7 +674,10 @@ void decode_noalloc(nut_model &m, nut_kvcache &kv, int token, float *d_hidden)
             "quantized decode: token out of range");
     require(kv.length < kv.config.max_seq, NUT_ELENGTH,
             "quantized decode: context is full");
-    require(fast_steps(m), NUT_EINVAL,
+    bool blocks32 = true;
+    for (const DeviceLayer &l : m.layers)
+        blocks32 = blocks32 && l.in_arena;
+    require(fast_steps(m) && blocks32, NUT_EINVAL,
             "no-alloc decode: needs 32-wide quant blocks along whole rows and head_dim "
             "64 or 128");
     const DecodeShape &s = m.shape;

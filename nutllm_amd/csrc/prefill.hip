@@ -1072,7 +1072,7 @@ bool prefill_gemm_supported(const DecodeShape &s, const LayerView &w)
     // whole blocks per row, and an even block count (a row's scales are
     // DMA'd as dwords)
     for (const QMat *m : mats)
-        if (!fast_layout(*m) || m->cols % 64 != 0)
+        if (m->block_size != 32 || m->cols % 64 != 0)
             return false;
     return s.head_dim == 64 || s.head_dim == 128;
 }

@@ -1,10 +1,10 @@
 // rows.hpp — the decode matvec's row dot with x staged in LDS, shared by
 // the step kernels and the standalone quantised matvec (matvec_quantized,
-// src/quant.cpp:257-321, for 32-wide blocks along whole rows).
+// src/quant.cpp:257-321, for blocks of 32, 64, ... along whole rows).
 //
 // A workgroup of kRowThreads threads stages x (times the RMSNorm weights
 // when asked) once in LDS; each wave streams R rows with nontemporal
-// 16-byte loads (one INT4 block or half an INT8 block per chunk), dots them
+// 16-byte loads (32 INT4 or 16 INT8 weights, all of one block), dots them
 // with the staged x chunk, subtracts the offset-binary bias through the x
 // chunk sum, and reduces the R row sums with DPP.
 #pragma once
@@ -36,13 +36,13 @@ __device__ __forceinline__ uint4 load_chunk(const uint8_t *p)
 
 // Pointers of rows row0 .. row0 + n - 1 of m (rows past the end re-read the
 // last row) into slots base .. base + n - 1.
-template <int QT, int R>
+template <int QT, int R, bool WB>
 __device__ __forceinline__ void row_ptrs(const QMat &m, int row0, int base, int n,
                                          const uint8_t *(&rp)[R],
                                          const uint16_t *(&sp)[R])
 {
     const int row_bytes = QT == 1 ? m.cols / 2 : m.cols;
-    const int bpr = m.cols / 32;
+    const int bpr = WB ? m.cols >> (scale_shift(m) + 5) : m.cols / 32;
 #pragma unroll
     for (int r = 0; r < R; r++)
         if (r >= base && r < base + n) {
@@ -65,16 +65,16 @@ template <int QT> inline size_t staged_x_bytes(int cols)
 }
 
 // out[r] = sum_k q_k s x'_k over row r of R rows (pointers rp / sp, `cols`
-// columns), x'_k = x_k * nw_k when NORM, then times the RMS factor of x;
+// columns; WB: blocks wider than 32, scale_shift `shift`), x'_k = x_k * nw_k when NORM, then times the RMS factor of x;
 // every lane gets all sums. Every wave of the workgroup calls it (`active`
 // false for waves without rows): the workgroup stages x' once into LDS (xs,
 // staged_x_bytes) and reduces sum x^2 in red[kRowWaves]; each wave issues its
 // first weight chunks before the staging, so they load meanwhile. STREAM:
 // the weight loads' cache policy (load_chunk).
-template <int QT, int R, bool NORM, bool STREAM = true>
+template <int QT, int R, bool WB, bool NORM, bool STREAM = true>
 __device__ __forceinline__ void rows_matvec(const uint8_t *const (&rp)[R],
                                             const uint16_t *const (&sp)[R], int cols,
-                                            const float *x, const float *nw, bool active,
+                                            int shift, const float *x, const float *nw, bool active,
                                             float *xs, float *red, float (&out)[R])
 {
     constexpr int CW = chunk_cw<QT>(), XS = chunk_xs<QT>();
@@ -88,7 +88,7 @@ __device__ __forceinline__ void rows_matvec(const uint8_t *const (&rp)[R],
 #pragma unroll
         for (int r = 0; r < R; r++) {
             w0[r] = load_chunk<STREAM>(rp[r] + 16 * lane);
-            s0[r] = half_bits_to_float(sp[r][QT == 1 ? lane : lane >> 1]);
+            s0[r] = half_bits_to_float(sp[r][(QT == 1 ? lane : lane >> 1) >> (WB ? shift : 0)]);
         }
     }
     float sq = 0.0f;
@@ -136,6 +136,17 @@ __device__ __forceinline__ void rows_matvec(const uint8_t *const (&rp)[R],
             xc[4 * q + 2] = v.z;
             xc[4 * q + 3] = v.w;
         }
+        if (WB) {
+            // wider blocks keep the error of a sum of q s x itself (5000 x
+            // 4096 INT4 at block 64: 7.7e-7 in offset binary, 1.1e-7 so)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float d =
+                    QT == 1 ? dot_int4_chunk<true>(w[r], xc) : dot_int8_chunk<true>(w[r], xc);
+                acc[r] = fmaf(s[r], d, acc[r]);
+            }
+            return;
+        }
         float xsum = 0.0f;
 #pragma unroll
         for (int i = 0; i < CW; i++)
@@ -155,7 +166,7 @@ __device__ __forceinline__ void rows_matvec(const uint8_t *const (&rp)[R],
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 w[r] = load_chunk<STREAM>(rp[r] + 16 * c);
-                s[r] = half_bits_to_float(sp[r][QT == 1 ? c : c >> 1]);
+                s[r] = half_bits_to_float(sp[r][(QT == 1 ? c : c >> 1) >> (WB ? shift : 0)]);
             }
             chunk(c, w, s);
         }

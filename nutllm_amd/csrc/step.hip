@@ -1,6 +1,6 @@
 // step.hip — fast kernels of one decode step (decode_quantized_token,
-// src/quant_model.cpp:158-206) for layers whose matrices use 32-wide quant
-// blocks along whole rows. Five launches per layer:
+// src/quant_model.cpp:158-206) for layers whose matrices use quant blocks of
+// 32, 64, ... weights along whole rows. Five launches per layer:
 //   qkv        xn = rmsnorm(h) * attention_norm folded into the Q/K/V
 //              rows, RoPE, K/V into the cache at *length
 //   attention  one workgroup per (KV head, split of the positions) for all
@@ -71,7 +71,7 @@ __device__ __forceinline__ bool chunk_cell(int blocks, int tokens, int &block, i
 // rows, value rows; R divides dim and kv_heads * head_dim), RoPE on the
 // query and key pairs at position *length (src/quant_model.cpp:26-37), key
 // and value rows into the layer's cache.
-template <int QT, int R, bool CHUNK = false>
+template <int QT, int R, bool WB, bool CHUNK>
 __global__ __launch_bounds__(kThreads) void qkv_fast_kernel(
     DecodeShape s, const float *hidden, const float *norm, QMat wq, QMat wk,
     QMat wv, const float2 *rope, const int *length, float *k_layer,
@@ -91,9 +91,10 @@ __global__ __launch_bounds__(kThreads) void qkv_fast_kernel(
     const int local = which == 0 ? row : which == 1 ? row - s.dim : row - s.dim - kvd;
     const uint8_t *rp[R];
     const uint16_t *sp[R];
-    row_ptrs<QT, R>(which == 0 ? wq : which == 1 ? wk : wv, local, 0, R, rp, sp);
+    row_ptrs<QT, R, WB>(which == 0 ? wq : which == 1 ? wk : wv, local, 0, R, rp, sp);
     float out[R];
-    rows_matvec<QT, R, true, !CHUNK>(rp, sp, s.dim, hidden, norm, active, xs, red, out);
+    rows_matvec<QT, R, WB, true, !CHUNK>(rp, sp, s.dim, scale_shift(wq), hidden, norm, active,
+                                         xs, red, out);
     if (!active)
         return;
     const int pos = *length + t;
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(kThreads) void qkv_fast_kernel(
 }
 
 // y[r] += (W x)[r]  (Wo + residual, W2 + residual)
-template <int QT, int R, bool CHUNK = false>
+template <int QT, int R, bool WB, bool CHUNK>
 __global__ __launch_bounds__(kThreads) void residual_fast_kernel(
     QMat m, const float *x, float *y, int blocks, int tokens, const StepState *state)
 {
@@ -131,10 +132,10 @@ __global__ __launch_bounds__(kThreads) void residual_fast_kernel(
     const int row = wave_id(block) * R;
     const uint8_t *rp[R];
     const uint16_t *sp[R];
-    row_ptrs<QT, R>(m, row, 0, R, rp, sp);
+    row_ptrs<QT, R, WB>(m, row, 0, R, rp, sp);
     float out[R];
-    rows_matvec<QT, R, false, !CHUNK>(rp, sp, m.cols, x, nullptr, row < m.rows, xs, nullptr,
-                                      out);
+    rows_matvec<QT, R, WB, false, !CHUNK>(rp, sp, m.cols, scale_shift(m), x, nullptr,
+                                      row < m.rows, xs, nullptr, out);
     if (row < m.rows && (threadIdx.x & (kWave - 1)) == 0)
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void residual_fast_kernel(
 
 // act[r] = silu((Wg xn)[r]) * (Wu xn)[r], xn = rmsnorm(h) * ffn_norm
 // (src/quant_model.cpp:194-198); R rows of each matrix per wave.
-template <int QT, int R, bool CHUNK = false>
+template <int QT, int R, bool WB, bool CHUNK>
 __global__ __launch_bounds__(kThreads) void gate_up_fast_kernel(
     const float *hidden, const float *norm, QMat wg, QMat wu, float *act, int blocks,
     int tokens, const StepState *state)
@@ -159,11 +160,11 @@ __global__ __launch_bounds__(kThreads) void gate_up_fast_kernel(
     const int row = wave_id(block) * R;
     const uint8_t *rp[2 * R];
     const uint16_t *sp[2 * R];
-    row_ptrs<QT, 2 * R>(wg, row, 0, R, rp, sp);
-    row_ptrs<QT, 2 * R>(wu, row, R, R, rp, sp);
+    row_ptrs<QT, 2 * R, WB>(wg, row, 0, R, rp, sp);
+    row_ptrs<QT, 2 * R, WB>(wu, row, R, R, rp, sp);
     float gu[2 * R];
-    rows_matvec<QT, 2 * R, true, !CHUNK>(rp, sp, wg.cols, hidden, norm, row < wg.rows, xs, red,
-                                         gu);
+    rows_matvec<QT, 2 * R, WB, true, !CHUNK>(rp, sp, wg.cols, scale_shift(wg), hidden, norm,
+                                         row < wg.rows, xs, red, gu);
     if (row < wg.rows && (threadIdx.x & (kWave - 1)) == 0)
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -589,10 +590,10 @@ dim3 row_grid(int blocks, int tokens, bool chunk)
     return dim3(((blocks + kXcds - 1) / kXcds) * kXcds * tokens);
 }
 
-// One layer on the step kernels. CHUNK: a prompt chunk of several tokens,
+// One layer on the step kernels. WB: blocks wider than 32. CHUNK: a prompt chunk of several tokens,
 // whose workgroups of one row block share an XCD and read the weights
 // through the caches; otherwise one token, weights streamed.
-template <int QT, int HD, bool CHUNK>
+template <int QT, int HD, bool WB, bool CHUNK>
 void launch_layer_fast_c(const DecodeShape &s, const LayerView &w,
                          const float2 *rope, const int *length, float *k_layer,
                          float *v_layer, const StepBuffers &b, int tokens,
@@ -611,13 +612,13 @@ void launch_layer_fast_c(const DecodeShape &s, const LayerView &w,
     const bool wide_chunk = CHUNK && tokens >= 6;
     if ((qkv_rows >= 8192 || wide_chunk) && s.dim % 4 == 0 && kvd % 4 == 0) {
         const int blocks = blocks_for_rows(qkv_rows, 4);
-        hipLaunchKernelGGL((qkv_fast_kernel<QT, 4, CHUNK>), row_grid(blocks, tokens, CHUNK),
+        hipLaunchKernelGGL((qkv_fast_kernel<QT, 4, WB, CHUNK>), row_grid(blocks, tokens, CHUNK),
                            dim3(kThreads), x_dim, stream, s, b.hidden, w.attention_norm,
                            w.query, w.key, w.value, rope, length, k_layer, v_layer,
                            b.query, blocks, tokens, state);
     } else {
         const int blocks = blocks_for_rows(qkv_rows, 2);
-        hipLaunchKernelGGL((qkv_fast_kernel<QT, 2, CHUNK>), row_grid(blocks, tokens, CHUNK),
+        hipLaunchKernelGGL((qkv_fast_kernel<QT, 2, WB, CHUNK>), row_grid(blocks, tokens, CHUNK),
                            dim3(kThreads), x_dim, stream, s, b.hidden, w.attention_norm,
                            w.query, w.key, w.value, rope, length, k_layer, v_layer,
                            b.query, blocks, tokens, state);
@@ -627,23 +628,23 @@ void launch_layer_fast_c(const DecodeShape &s, const LayerView &w,
     const int dim_blocks = blocks_for_rows(s.dim, wide_chunk ? 4 : 2);
     auto residual = [&](const QMat &m, const float *x, size_t x_bytes) {
         if (wide_chunk)
-            hipLaunchKernelGGL((residual_fast_kernel<QT, 4, CHUNK>),
+            hipLaunchKernelGGL((residual_fast_kernel<QT, 4, WB, CHUNK>),
                                row_grid(dim_blocks, tokens, CHUNK), dim3(kThreads), x_bytes,
                                stream, m, x, b.hidden, dim_blocks, tokens, state);
         else
-            hipLaunchKernelGGL((residual_fast_kernel<QT, 2, CHUNK>),
+            hipLaunchKernelGGL((residual_fast_kernel<QT, 2, WB, CHUNK>),
                                row_grid(dim_blocks, tokens, CHUNK), dim3(kThreads), x_bytes,
                                stream, m, x, b.hidden, dim_blocks, tokens, state);
     };
     residual(w.output, b.context, x_dim);
     if (s.ffn_dim >= 8192 || wide_chunk) {
         const int blocks = blocks_for_rows(s.ffn_dim, 4);
-        hipLaunchKernelGGL((gate_up_fast_kernel<QT, 4, CHUNK>), row_grid(blocks, tokens, CHUNK),
+        hipLaunchKernelGGL((gate_up_fast_kernel<QT, 4, WB, CHUNK>), row_grid(blocks, tokens, CHUNK),
                            dim3(kThreads), x_dim, stream, b.hidden, w.ffn_norm, w.gate, w.up,
                            b.act, blocks, tokens, state);
     } else {
         const int blocks = blocks_for_rows(s.ffn_dim, 2);
-        hipLaunchKernelGGL((gate_up_fast_kernel<QT, 2, CHUNK>), row_grid(blocks, tokens, CHUNK),
+        hipLaunchKernelGGL((gate_up_fast_kernel<QT, 2, WB, CHUNK>), row_grid(blocks, tokens, CHUNK),
                            dim3(kThreads), x_dim, stream, b.hidden, w.ffn_norm, w.gate, w.up,
                            b.act, blocks, tokens, state);
     }
@@ -657,12 +658,17 @@ void launch_layer_fast_t(const DecodeShape &s, const LayerView &w,
                          float *v_layer, const StepBuffers &b, int tokens,
                          const StepState *state, hipStream_t stream)
 {
+    const bool wide = w.query.block_size > 32;
     if (tokens > 1)
-        launch_layer_fast_c<QT, HD, true>(s, w, rope, length, k_layer, v_layer, b, tokens,
-                                          state, stream);
+        wide ? launch_layer_fast_c<QT, HD, true, true>(s, w, rope, length, k_layer, v_layer, b,
+                                                       tokens, state, stream)
+             : launch_layer_fast_c<QT, HD, false, true>(s, w, rope, length, k_layer, v_layer, b,
+                                                        tokens, state, stream);
     else
-        launch_layer_fast_c<QT, HD, false>(s, w, rope, length, k_layer, v_layer, b, tokens,
-                                           state, stream);
+        wide ? launch_layer_fast_c<QT, HD, true, false>(s, w, rope, length, k_layer, v_layer, b,
+                                                        tokens, state, stream)
+             : launch_layer_fast_c<QT, HD, false, false>(s, w, rope, length, k_layer, v_layer, b,
+                                                         tokens, state, stream);
 }
 
 } // namespace
@@ -672,7 +678,8 @@ bool step_fast_supported(const DecodeShape &s, const LayerView &w)
     const QMat *mats[7] = {&w.query, &w.key, &w.value, &w.output,
                            &w.gate, &w.up, &w.down};
     for (const QMat *m : mats)
-        if (!fast_layout(*m) || m->type != w.query.type)
+        if (!fast_layout(*m) || m->type != w.query.type ||
+            m->block_size != w.query.block_size)
             return false;
     // the staged x of every matvec fits a workgroup's 64 KB of LDS
     const int cols = std::max(s.dim, s.ffn_dim);

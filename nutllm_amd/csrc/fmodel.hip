@@ -21,6 +21,7 @@
 #include "fmodel.hpp"
 #include "gemm_f32.hpp"
 #include "prefill.hpp"
+#include "project.hpp"
 #include "runtime.hpp"
 
 #include <algorithm>
@@ -31,28 +32,22 @@ namespace nut {
 
 namespace {
 
-// What the product of a launch becomes.
-enum FEpilogue { kFAdd, kFSwiglu, kFQkv };
-
 struct FGemm {
-    const float *x, *norm_w; // rows [m][k], norm weights [k] (not kFAdd)
+    const float *x, *norm_w; // rows [m][k], norm weights [k] (not kAdd)
     int m, k;
-    // the matrices, [k][n] each: q, k, v (kFQkv, column tiles in that order),
-    // gate and up (kFSwiglu, both in every tile) or the one (kFAdd)
+    // the matrices, [k][n] each: q, k, v (kQkv, column tiles in that order),
+    // gate and up (kSwiglu, both in every tile) or the one (kAdd)
     const float *w[3];
     int n[3], tiles[3];
     int tiles_m, tiles_n;
-    float *out; // rows of n[0]: hidden rows, activations, query rows
-    const float2 *rope;
-    float *k_layer, *v_layer;
-    int first_pos, head_dim, max_seq;
+    ProjectOut to;
 };
 
 template <int TI, int TJ, int WK, int D, int EPI>
 __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
 {
-    constexpr bool NORM = EPI != kFAdd;
-    constexpr int NB = EPI == kFSwiglu ? 2 : 1, TB = TJ / NB;
+    constexpr bool NORM = EPI != kAdd;
+    constexpr int NB = EPI == kSwiglu ? 2 : 1, TB = TJ / NB;
     constexpr int kStage = WK * 16 * TI * kChunkLd, kRed = WK * TJ * 256;
     __shared__ __attribute__((aligned(16))) float lds[kStage > kRed ? kStage : kRed];
     __shared__ float squares[NORM ? WK : 1][16 * TI];
@@ -60,7 +55,7 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
     if (!gemm_f32_tile(f.tiles_m, f.tiles_n, tm, tn))
         return; // workgroup-uniform
     int seg = 0;
-    if (EPI == kFQkv)
+    if (EPI == kQkv)
         while (seg < 2 && tn >= f.tiles[seg])
             tn -= f.tiles[seg++]; // workgroup-uniform
     const int n = f.n[seg], m = f.m, k = f.k;
@@ -75,7 +70,7 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
     const float *pb[NB];
 #pragma unroll
     for (int q = 0; q < NB; q++)
-        pb[q] = f.w[EPI == kFSwiglu ? q : seg] + size_t(8 * g) * n + first;
+        pb[q] = f.w[EPI == kSwiglu ? q : seg] + size_t(8 * g) * n + first;
     floatx4 acc[1][TI][TJ];
     float sq[2 * TI] = {};
     gemm_f32_clear(acc);
@@ -102,73 +97,23 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
         const int r = 16 * i + 4 * g + v, row = row0 + r;
         if (row >= m || col >= n)
             return;
-        if (NORM) {
-            float s = squares[0][r];
-#pragma unroll
-            for (int w = 1; w < WK; w++)
-                s += squares[w][r];
-            const float scale = 1.0f / sqrtf(s / float(k) + 1e-5f);
+        if constexpr (NORM) {
+            const float scale = row_scale<WK>(squares, r, k);
 #pragma unroll
             for (int j = 0; j < TJ; j++)
                 out[j] *= scale;
         }
-        float vals[TB];
-        float *dst;
-        if constexpr (EPI == kFSwiglu) {
-#pragma unroll
-            for (int j = 0; j < TB; j++)
-                vals[j] = out[j] / (1.0f + expf(-out[j])) * out[TB + j];
-            dst = f.out + size_t(row) * n + first;
-        } else if constexpr (EPI == kFAdd) {
-            dst = f.out + size_t(row) * n + first;
-#pragma unroll
-            for (int j = 0; j < TB; j++)
-                vals[j] = dst[j] + out[j];
-        } else {
-            // RoPE (rotate_vector, src/kvcache.cpp:48-59) on the pairs of q
-            // and k; TB, n and head_dim are even, so a pair is a lane's
-            static_assert(EPI != kFQkv || TB % 2 == 0, "whole RoPE pairs");
-            const int pos = f.first_pos + row;
-            const int head = first / f.head_dim, d = first % f.head_dim;
-#pragma unroll
-            for (int j = 0; j < TB; j += 2) {
-                float e = out[j], o = out[j + 1];
-                if (seg < 2) {
-                    const float2 cs = f.rope[size_t(pos) * (f.head_dim / 2) + (d + j) / 2];
-                    const float even = e, odd = o;
-                    e = fmaf(even, cs.x, -(odd * cs.y));
-                    o = fmaf(even, cs.y, odd * cs.x);
-                }
-                vals[j] = e;
-                vals[j + 1] = o;
-            }
-            if (seg == 0) {
-                dst = f.out + size_t(row) * n + first;
-            } else {
-                // head_dim is a multiple of 4 and TB 2 or 4, first a multiple
-                // of TB: a lane's columns are of one head
-                dst = (seg == 1 ? f.k_layer : f.v_layer) +
-                      (size_t(head) * f.max_seq + pos) * f.head_dim + d;
-            }
-        }
-        if (first == col) {
-            store_u<TB>(dst, vals);
-        } else {
-#pragma unroll
-            for (int j = 0; j < TB; j++)
-                if (first + j >= col)
-                    dst[j] = vals[j];
-        }
+        project_store<EPI, TJ>(f.to, seg, n, row, col, first, out);
     });
 }
 
 template <int TI, int TJ, int WK, int D, int EPI>
 void launch_ftile(FGemm &f, hipStream_t stream)
 {
-    const int cols = 16 * TJ / (EPI == kFSwiglu ? 2 : 1);
+    const int cols = 16 * TJ / (EPI == kSwiglu ? 2 : 1);
     f.tiles_m = (f.m + 16 * TI - 1) / (16 * TI);
     f.tiles_n = 0;
-    for (int s = 0; s < (EPI == kFQkv ? 3 : 1); s++) {
+    for (int s = 0; s < (EPI == kQkv ? 3 : 1); s++) {
         f.tiles[s] = (f.n[s] + cols - 1) / cols;
         f.tiles_n += f.tiles[s];
     }
@@ -184,12 +129,12 @@ void launch_ftile(FGemm &f, hipStream_t stream)
 template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
 {
     int n = f.n[0];
-    if (EPI == kFQkv)
+    if (EPI == kQkv)
         n += f.n[1] + f.n[2];
-    if (EPI == kFSwiglu)
+    if (EPI == kSwiglu)
         n *= 2;
     if (f.m <= 16) {
-        if constexpr (EPI == kFAdd) {
+        if constexpr (EPI == kAdd) {
             n >= 4096 ? launch_ftile<1, 2, 16, 2, EPI>(f, stream)
                       : launch_ftile<1, 1, 16, 3, EPI>(f, stream);
         } else {
@@ -409,12 +354,7 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
         float *vc = kv.values.as<float>() + l * layer_elems;
         FGemm f{};
         f.m = t;
-        f.rope = m.rope.as<float2>();
-        f.k_layer = kc;
-        f.v_layer = vc;
-        f.first_pos = first;
-        f.head_dim = s.head_dim;
-        f.max_seq = s.max_seq;
+        f.to = ProjectOut{nullptr, m.rope.as<float2>(), kc, vc, first, s.head_dim, s.max_seq};
         auto gemm = [&](const float *x, const DeviceBuffer *norm, int k, int w0, int count, int n0,
                         float *out) {
             f.x = x;
@@ -424,21 +364,15 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
                 f.w[i] = L.w[w0 + i].as<float>();
                 f.n[i] = i == 0 ? n0 : w0 == 0 ? kvd : n0;
             }
-            f.out = out;
+            f.to.out = out;
         };
         gemm(h, &L.attention_norm, s.dim, 0, 3, s.dim, q);
-        launch_fgemm<kFQkv>(f, m.stream);
+        launch_fgemm<kQkv>(f, m.stream);
         if (t == 1 && m.split_attention) {
             launch_attention_split(s, q, kc, vc, length, m.attn_part.as<uint64_t>(),
                                    m.attn_count.as<int>(), ctx, state, m.stream);
-        } else if (first == 0 && s.head_dim == 64) {
-            launch_fattention<64>(s, q, kc, vc, ctx, t, m.stream);
-        } else if (first == 0 && s.head_dim == 128) {
-            launch_fattention<128>(s, q, kc, vc, ctx, t, m.stream);
-        } else if (first == 0 && s.head_dim == 32) {
-            launch_fattention<32>(s, q, kc, vc, ctx, t, m.stream);
-        } else if (first == 0 && s.head_dim == 16) {
-            launch_fattention<16>(s, q, kc, vc, ctx, t, m.stream);
+        } else if (first == 0 && attention_f32_supported(s)) {
+            launch_attention_f32(s, q, kc, vc, ctx, t, m.stream);
         } else {
             for (int i = 0; i < t; i++) {
                 if (t > 1)
@@ -448,11 +382,11 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
             }
         }
         gemm(ctx, nullptr, s.dim, 3, 1, s.dim, h);
-        launch_fgemm<kFAdd>(f, m.stream);
+        launch_fgemm<kAdd>(f, m.stream);
         gemm(h, &L.ffn_norm, s.dim, 4, 2, s.ffn_dim, act);
-        launch_fgemm<kFSwiglu>(f, m.stream);
+        launch_fgemm<kSwiglu>(f, m.stream);
         gemm(act, nullptr, s.ffn_dim, 6, 1, s.dim, h);
-        launch_fgemm<kFAdd>(f, m.stream);
+        launch_fgemm<kAdd>(f, m.stream);
     }
 }
 
@@ -471,6 +405,20 @@ void upload_to(DeviceBuffer &b, const float *src, size_t count)
 }
 
 } // namespace
+
+bool attention_f32_supported(const DecodeShape &s)
+{
+    return s.head_dim == 16 || s.head_dim == 32 || s.head_dim == 64 || s.head_dim == 128;
+}
+
+void launch_attention_f32(const DecodeShape &s, const float *q, const float *k_layer,
+                          const float *v_layer, float *ctx, int t, hipStream_t stream)
+{
+    s.head_dim == 128  ? launch_fattention<128>(s, q, k_layer, v_layer, ctx, t, stream)
+    : s.head_dim == 64 ? launch_fattention<64>(s, q, k_layer, v_layer, ctx, t, stream)
+    : s.head_dim == 32 ? launch_fattention<32>(s, q, k_layer, v_layer, ctx, t, stream)
+                       : launch_fattention<16>(s, q, k_layer, v_layer, ctx, t, stream);
+}
 
 nut_fmodel *create_fmodel(const nut_config &config, bool tied)
 {

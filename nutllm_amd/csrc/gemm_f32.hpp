@@ -123,6 +123,7 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
                 sq[t] = fmaf(v.y, v.y, sq[t]);
                 sq[t] = fmaf(v.z, v.z, sq[t]);
                 sq[t] = fmaf(v.w, v.w, sq[t]);
+                asm volatile("" : "+v"(sq[t])); // now: not with every chunk's values kept
                 v.x *= fn[0];
                 v.y *= fn[1];
                 v.z *= fn[2];

@@ -134,6 +134,26 @@ void launch_layer_fast(const DecodeShape &s, const LayerView &w,
                        float *v_layer, const StepBuffers &b, int tokens,
                        const StepState *state, hipStream_t stream);
 
+// Causal attention in fp32 of t rows at positions 0 .. t - 1 (fmodel.hip):
+// q and ctx [t][heads * head_dim], K and V in the layer's cache.
+bool attention_f32_supported(const DecodeShape &s);
+void launch_attention_f32(const DecodeShape &s, const float *q, const float *k_layer,
+                          const float *v_layer, float *ctx, int t, hipStream_t stream);
+
+// The projections of a short prompt's rows on f16 MFMA (rowgemm.hip), t <=
+// kRowGemmMax rows of fp32 activations: blocks of 32, inputs a multiple of
+// 128 wide.
+constexpr int kRowGemmMax = 128;
+bool row_gemm_supported(const DecodeShape &s, const LayerView &w);
+struct RowBuffers {
+    float *hidden, *query, *context, *act; // [t][dim], [t][ffn]
+};
+// One layer for t rows at positions 0 .. t - 1: hidden in place, K and V rows
+// into the layer's cache.
+void launch_layer_rows(const DecodeShape &s, const LayerView &w, const float2 *rope,
+                       float *k_layer, float *v_layer, const RowBuffers &b, int t,
+                       hipStream_t stream);
+
 // Tiny state writers, enqueued on the stream (graph-safe, no memset).
 void launch_set_int(int *target, int value, hipStream_t stream);
 void launch_reset_state(StepState *state, int token, hipStream_t stream);

@@ -189,8 +189,9 @@ void prefill_steps(nut_model &m, nut_kvcache &kv, size_t count)
               "hipMemcpyAsync");
 }
 
-// Prompts of at least this many tokens run as a batch (GEMM prefill);
-// shorter ones run as one step-kernel chunk (kStepTokensMax = 31). A chunk
+// Of the prompts that the row tiles leave, those of at least this many
+// tokens run as a batch (GEMM prefill); shorter ones run as one step-kernel
+// chunk (kStepTokensMax = 31). A chunk
 // costs its row dots once per token, the batch one 64-token MFMA tile, so
 // the crossover depends on the width. TinyLlama INT4 (dim 2048), batch
 // against one chunk: 24 tokens 3.11 against 2.64 ms, 28 tokens 3.12
@@ -200,6 +201,60 @@ void prefill_steps(nut_model &m, nut_kvcache &kv, size_t count)
 size_t prefill_gemm_min(const DecodeShape &s)
 {
     return s.dim >= 4096 ? 16 : 30;
+}
+
+// Prompts of these lengths run on the row tiles (rowgemm.hip), where every
+// layer has their layout and per-token steps are not forced. A tile costs
+// the same for 2 rows as for 16, a step-kernel chunk a little per token; the
+// batched GEMM wins once its 64 x 128 tiles fill the chip. TinyLlama INT4,
+// row tiles against the better of the two: 5 tokens 1.01 ms (1.02), 9 1.02
+// (1.36), 16 1.05 (1.95), 20 1.53 (2.28), 64 1.83 (3.30), 96 2.58 (3.33), 128
+// 3.08 (3.39); two layers of the 7B widths INT4: 2 tokens 0.27 (0.20), 5 0.27
+// (0.31), 16 0.26 (0.55), 64 0.49 (0.57), 65 0.74 (0.62). Small widths are
+// bound by the launches, five a layer in each.
+size_t row_gemm_min(const DecodeShape &s)
+{
+    return s.dim < 1024 ? 2 : s.dim < 4096 ? 6 : 5;
+}
+
+size_t row_gemm_max(const DecodeShape &s)
+{
+    return s.dim < 4096 ? size_t(kRowGemmMax) : 64;
+}
+
+bool use_row_gemm(const nut_model &m, size_t count)
+{
+    if (m.path != 0 || count < row_gemm_min(m.shape) || count > row_gemm_max(m.shape))
+        return false;
+    for (const DeviceLayer &l : m.layers)
+        if (!row_gemm_supported(m.shape, l.view))
+            return false;
+    return true;
+}
+
+// Tokens [0, count) (device ids in m.prompt) through every layer on the row
+// tiles; the last token's hidden state lands in m.hidden.
+void prefill_rows(nut_model &m, nut_kvcache &kv, size_t count)
+{
+    const DecodeShape &s = m.shape;
+    if (m.rg_hidden.get() == nullptr) {
+        m.rg_hidden.allocate(size_t(kRowGemmMax) * s.dim * sizeof(float));
+        m.rg_query.allocate(size_t(kRowGemmMax) * s.dim * sizeof(float));
+        m.rg_context.allocate(size_t(kRowGemmMax) * s.dim * sizeof(float));
+        m.rg_act.allocate(size_t(kRowGemmMax) * s.ffn_dim * sizeof(float));
+    }
+    const RowBuffers b{m.rg_hidden.as<float>(), m.rg_query.as<float>(), m.rg_context.as<float>(),
+                       m.rg_act.as<float>()};
+    launch_embed_rows(m.embeddings.as<float>(), m.prompt.as<int>(), b.hidden, int(count), s.dim,
+                      m.stream);
+    const size_t layer_elems = kv.layer_elements();
+    for (size_t l = 0; l < m.layers.size(); l++)
+        launch_layer_rows(s, m.layers[l].view, m.rope.as<float2>(),
+                          kv.keys.as<float>() + l * layer_elems,
+                          kv.values.as<float>() + l * layer_elems, b, int(count), m.stream);
+    hip_check(hipMemcpyAsync(m.hidden.get(), b.hidden + (count - 1) * s.dim,
+                             s.dim * sizeof(float), hipMemcpyDeviceToDevice, m.stream),
+              "hipMemcpyAsync");
 }
 
 // The batched prefill applies when every layer uses 32-wide blocks, the
@@ -734,7 +789,9 @@ void prefill(nut_model &m, nut_kvcache &kv, const int *tokens, size_t count,
         hip_check(hipMemcpyAsync(m.prompt.get(), tokens, valid * sizeof(int),
                                  hipMemcpyHostToDevice, m.stream),
                   "hipMemcpyAsync");
-        if (use_prefill_gemm(m, valid)) {
+        if (use_row_gemm(m, valid)) {
+            prefill_rows(m, kv, valid);
+        } else if (use_prefill_gemm(m, valid)) {
             prefill_batch(m, kv, valid);
         } else if (m.path != 2 && valid > 1 && fast_steps(m)) {
             prefill_steps(m, kv, valid);

@@ -70,6 +70,8 @@ struct nut_model {
     nut::DeviceBuffer attn_part, attn_count; // fast step kernels
     // Prompt chunks on the step kernels: kStepTokensMax rows each.
     nut::DeviceBuffer mt_hidden, mt_query, mt_context, mt_act;
+    // Short prompts on the row tiles: kRowGemmMax rows each.
+    nut::DeviceBuffer rg_hidden, rg_query, rg_context, rg_act;
     // One greedy iteration (classifier, argmax, decode step) captured as a
     // graph for the generation cache; replayed once per generated token.
     hipGraphExec_t step_graph = nullptr;

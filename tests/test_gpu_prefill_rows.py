@@ -1,0 +1,47 @@
+"""Short prompts on the row tiles against the per-token step kernels.
+
+Lengths at the edges of the tiles (16 and 32 rows) and of the range that takes
+them, INT8 and INT4, head sizes 64 and 128: the last hidden state, the K/V rows
+of every position and the step that follows. The bar is 5e-6 on the relative
+error: fp32 sums, and activations as two f16 limbs (2^-22 each), over two
+layers; the step kernels themselves are within 2e-6 of 64 bits here."""
+import numpy as np
+import pytest
+
+from nutllm_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.fixture(scope="module", params=[("step_gqa2", 0), ("step_gqa4", 1), ("step_mha128", 0),
+                                        ("step_mha128", 1)], ids=lambda p: f"{p[0]}-{p[1]}")
+def model(request, gpu):
+    shape, qtype = request.param
+    m = W.build(shape, qtype, 31, max_seq=160, norm_seed=5)
+    dev = m.to_device()
+    yield m.config, dev
+    dev.close()
+
+
+@pytest.mark.parametrize("tokens", [2, 3, 15, 16, 17, 31, 32, 33, 64, 65, 127, 128])
+def test_row_tiles_match_steps(gpu, model, tokens):
+    cfg, dev = model
+    ids = gpu.synth_tokens(9, cfg.vocab_size, tokens).astype(np.int32)
+    rows, steps = gpu.KVCache(cfg), gpu.KVCache(cfg)
+    try:
+        got = dev.prefill(rows, ids)
+        dev.set_path(1)
+        want = dev.prefill(steps, ids)
+        dev.set_path(0)
+        assert rel(got, want) <= 5e-6
+        for a, b in zip(rows.read_positions(0, tokens), steps.read_positions(0, tokens)):
+            assert rel(a, b) <= 5e-6
+        assert rel(dev.decode(rows, 3), dev.decode(steps, 3)) <= 5e-6
+    finally:
+        dev.set_path(0)
+        rows.close(), steps.close()

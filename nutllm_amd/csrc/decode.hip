@@ -435,6 +435,20 @@ __global__ __launch_bounds__(kThreads) void classifier_screen_kernel(
     scales[i] = bits;
 }
 
+__global__ __launch_bounds__(kThreads) void copy_words_kernel(const uint32_t *src, uint32_t *dst,
+                                                              size_t n, const int *flag,
+                                                              int *flag_out)
+{
+    const size_t t = size_t(blockIdx.x) * kThreads + threadIdx.x, step = size_t(gridDim.x) * kThreads;
+    const size_t n4 = n / 4; // src and dst are 16-byte aligned
+    for (size_t i = t; i < n4; i += step)
+        reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    for (size_t i = 4 * n4 + t; i < n; i += step)
+        dst[i] = src[i];
+    if (flag != nullptr && t == 0)
+        *flag_out = *flag;
+}
+
 __global__ void set_int_kernel(int *target, int value) { *target = value; }
 
 __global__ void reset_state_kernel(StepState *state, int token)
@@ -546,6 +560,16 @@ void launch_classifier_screen(const float *weights, int vocab, int dim, int8_t *
     hipLaunchKernelGGL(classifier_screen_kernel, dim3(unsigned((cells + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, stream, weights, vocab, dim, codes, scales);
     check_launch("classifier screening copy");
+}
+
+void launch_copy_words(const void *src, void *dst, size_t n, const int *flag, int *flag_out,
+                       hipStream_t stream)
+{
+    const size_t blocks = (n / 4 + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(copy_words_kernel, dim3(unsigned(blocks < 1 ? 1 : blocks > 64 ? 64 : blocks)),
+                       dim3(kThreads), 0, stream, static_cast<const uint32_t *>(src),
+                       static_cast<uint32_t *>(dst), n, flag, flag_out);
+    check_launch("copy");
 }
 
 void launch_set_int(int *target, int value, hipStream_t stream)

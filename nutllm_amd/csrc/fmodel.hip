@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <memory>
 
 namespace nut {
@@ -447,6 +448,7 @@ nut_fmodel *create_fmodel(const nut_config &config, bool tied)
     m->query.allocate(config.dim * sizeof(float));
     m->context.allocate(config.dim * sizeof(float));
     m->act.allocate(config.ffn_dim * sizeof(float));
+    m->host.allocate(config.dim * sizeof(float));
     m->state.allocate(sizeof(StepState));
     m->token.allocate(sizeof(int));
     hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "hipStreamCreate");
@@ -511,11 +513,11 @@ void decode_token(nut_fmodel &m, nut_kvcache &kv, int token, float *hidden)
                       m.shape.dim, m.stream);
     enqueue_layers(m, kv, m.hidden.as<float>(), 1, int(kv.length), m.query.as<float>(),
                    m.context.as<float>(), m.act.as<float>());
-    if (hidden != nullptr)
-        hip_check(hipMemcpyAsync(hidden, m.hidden.get(), m.config.dim * sizeof(float),
-                                 hipMemcpyDeviceToHost, m.stream),
-                  "hipMemcpyAsync");
+    launch_copy_words(m.hidden.get(), m.host.as<float>(), m.config.dim, nullptr, nullptr,
+                      m.stream);
     hip_check(hipStreamSynchronize(m.stream), "hipStreamSynchronize");
+    if (hidden != nullptr)
+        std::memcpy(hidden, m.host.as<float>(), m.config.dim * sizeof(float));
     kv.length += 1;
 }
 

@@ -31,6 +31,7 @@ struct nut_fmodel {
     // a prompt's rows, for rows_held tokens
     nut::DeviceBuffer pf_tokens, pf_h, pf_q, pf_ctx, pf_act;
     size_t rows_held = 0;
+    nut::PinnedBuffer host; // a decode step's hidden state
     hipStream_t stream = nullptr;
     ~nut_fmodel();
 };

@@ -154,6 +154,14 @@ void launch_layer_rows(const DecodeShape &s, const LayerView &w, const float2 *r
                        float *k_layer, float *v_layer, const RowBuffers &b, int t,
                        hipStream_t stream);
 
+// dst[i] = src[i] for n 32-bit words; with `flag`, *flag_out = *flag too.
+// Either side may be page-locked host memory: a kernel between two others on
+// the stream, where a copy call for pageable memory stages, waits and returns
+// only when the stream is done (a decode step's 8 KB hidden state and its
+// error flag took two such calls, about 30 us).
+void launch_copy_words(const void *src, void *dst, size_t n, const int *flag, int *flag_out,
+                       hipStream_t stream);
+
 // Tiny state writers, enqueued on the stream (graph-safe, no memset).
 void launch_set_int(int *target, int value, hipStream_t stream);
 void launch_reset_state(StepState *state, int token, hipStream_t stream);

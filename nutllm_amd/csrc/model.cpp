@@ -148,6 +148,19 @@ void enqueue_step(nut_model &m, nut_kvcache &kv, const int *token_ptr)
     launch_finish_step(state, kv.device_length.as<int>(), m.stream);
 }
 
+HostArea &host_area(nut_model &m) { return *m.host.as<HostArea>(); }
+
+void *host_words(nut_model &m) { return m.host.as<char>() + sizeof(HostArea); }
+
+// Enqueues the copy of n words from device memory, and of the token kernels'
+// error flag, to the host area; valid after sync.
+void enqueue_out(nut_model &m, const void *src, size_t n)
+{
+    host_area(m).error = 0;
+    launch_copy_words(src, host_words(m), n, m.token_error.as<int>(), &host_area(m).error,
+                      m.stream);
+}
+
 void sync(nut_model &m) { hip_check(hipStreamSynchronize(m.stream), "hipStreamSynchronize"); }
 
 // Tokens [0, count) (device ids in m.prompt) through the step kernels in
@@ -184,9 +197,8 @@ void prefill_steps(nut_model &m, nut_kvcache &kv, size_t count)
                               kv.values.as<float>() + l * layer_elems, b, int(t), state,
                               m.stream);
     }
-    hip_check(hipMemcpyAsync(m.hidden.get(), m.mt_hidden.as<float>() + (t - 1) * s.dim,
-                             s.dim * sizeof(float), hipMemcpyDeviceToDevice, m.stream),
-              "hipMemcpyAsync");
+    launch_copy_words(m.mt_hidden.as<float>() + (t - 1) * s.dim, m.hidden.get(), s.dim, nullptr,
+                      nullptr, m.stream);
 }
 
 // Of the prompts that the row tiles leave, those of at least this many
@@ -252,9 +264,8 @@ void prefill_rows(nut_model &m, nut_kvcache &kv, size_t count)
         launch_layer_rows(s, m.layers[l].view, m.rope.as<float2>(),
                           kv.keys.as<float>() + l * layer_elems,
                           kv.values.as<float>() + l * layer_elems, b, int(count), m.stream);
-    hip_check(hipMemcpyAsync(m.hidden.get(), b.hidden + (count - 1) * s.dim,
-                             s.dim * sizeof(float), hipMemcpyDeviceToDevice, m.stream),
-              "hipMemcpyAsync");
+    launch_copy_words(b.hidden + (count - 1) * s.dim, m.hidden.get(), s.dim, nullptr, nullptr,
+                      m.stream);
 }
 
 // The batched prefill applies when every layer uses 32-wide blocks, the
@@ -320,10 +331,8 @@ void prefill_batch(nut_model &m, nut_kvcache &kv, size_t count)
         launch_qgemm_rows(act_h, act_h + size_t(t) * s.ffn_dim, t, &wd, ss + 6, &h, &s.dim, 1,
                           true, m.stream);
     }
-    hip_check(hipMemcpyAsync(m.hidden.get(), h + size_t(t - 1) * s.dim,
-                             s.dim * sizeof(float), hipMemcpyDeviceToDevice,
-                             m.stream),
-              "hipMemcpyAsync");
+    launch_copy_words(h + size_t(t - 1) * s.dim, m.hidden.get(), s.dim, nullptr, nullptr,
+                      m.stream);
 }
 
 double now() { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
@@ -378,6 +387,7 @@ nut_model *create_model(const nut_config &config, int type, bool tied)
     m->state.allocate(sizeof(StepState));
     m->tokens.allocate((config.max_seq + 1) * sizeof(int));
     m->prompt.allocate((config.max_seq + 1) * sizeof(int));
+    m->host.allocate(sizeof(HostArea) + host_words(config) * sizeof(int));
     hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking),
               "hipStreamCreate");
     hip_check(hipEventCreate(&m->decode_begin), "hipEventCreate");
@@ -671,27 +681,24 @@ void run_token_kernel(nut_model &m, nut_kvcache &kv, size_t start, size_t n_iter
     launch_token_kernel(m.type, s, a, m.stream);
 }
 
-// After the stream synchronised: raise the kernel's bounded-wait failure,
-// once (the flag is cleared, so later calls that run no token kernel do
-// not report it again).
+// After enqueue_out and sync: raise the kernel's bounded-wait failure, once
+// (the flag is cleared, so later calls that run no token kernel do not report
+// it again).
 void check_token_error(nut_model &m)
 {
-    if (m.token_error.get() == nullptr)
+    if (host_area(m).error == 0)
         return;
-    int error = 0;
-    hip_check(hipMemcpy(&error, m.token_error.get(), sizeof error, hipMemcpyDeviceToHost),
-              "hipMemcpy");
-    if (error != 0) {
-        const int zero = 0;
-        hip_check(hipMemcpy(m.token_error.get(), &zero, sizeof zero, hipMemcpyHostToDevice),
-                  "hipMemcpy");
-        fail(NUT_EDEVICE, "token kernel: phase exchange timed out");
-    }
+    launch_set_int(m.token_error.as<int>(), 0, m.stream);
+    sync(m);
+    fail(NUT_EDEVICE, "token kernel: phase exchange timed out");
 }
 
 } // namespace
 
-void decode(nut_model &m, nut_kvcache &kv, int token, float *hidden)
+namespace {
+
+// One decode step enqueued, its hidden state for m.hidden; kv.length stays.
+void enqueue_decode(nut_model &m, nut_kvcache &kv, int token)
 {
     require(config_valid(m.config), NUT_EINVAL, "model config: invalid dimensions");
     require(kv_compatible(kv, m.config), NUT_EINVAL,
@@ -710,12 +717,18 @@ void decode(nut_model &m, nut_kvcache &kv, int token, float *hidden)
         launch_reset_state(m.state.as<StepState>(), token, m.stream);
         enqueue_step(m, kv, &m.state.as<StepState>()->token);
     }
-    if (hidden != nullptr)
-        hip_check(hipMemcpyAsync(hidden, m.hidden.get(), m.config.dim * sizeof(float),
-                                 hipMemcpyDeviceToHost, m.stream),
-                  "hipMemcpyAsync");
+}
+
+} // namespace
+
+void decode(nut_model &m, nut_kvcache &kv, int token, float *hidden)
+{
+    enqueue_decode(m, kv, token);
+    enqueue_out(m, m.hidden.get(), m.config.dim);
     sync(m);
     check_token_error(m);
+    if (hidden != nullptr)
+        std::memcpy(hidden, host_words(m), m.config.dim * sizeof(float));
     kv.length += 1;
 }
 
@@ -786,9 +799,8 @@ void prefill(nut_model &m, nut_kvcache &kv, const int *tokens, size_t count,
            size_t(tokens[valid]) < m.config.vocab_size)
         valid++;
     if (valid > 0) {
-        hip_check(hipMemcpyAsync(m.prompt.get(), tokens, valid * sizeof(int),
-                                 hipMemcpyHostToDevice, m.stream),
-                  "hipMemcpyAsync");
+        std::memcpy(host_words(m), tokens, valid * sizeof(int));
+        launch_copy_words(host_words(m), m.prompt.get(), valid, nullptr, nullptr, m.stream);
         if (use_row_gemm(m, valid)) {
             prefill_rows(m, kv, valid);
         } else if (use_prefill_gemm(m, valid)) {
@@ -804,16 +816,15 @@ void prefill(nut_model &m, nut_kvcache &kv, const int *tokens, size_t count,
             for (size_t t = 0; t < valid; t++)
                 enqueue_step(m, kv, m.prompt.as<int>() + t);
         }
-        if (hidden != nullptr)
-            hip_check(hipMemcpyAsync(hidden, m.hidden.get(), m.config.dim * sizeof(float),
-                                     hipMemcpyDeviceToHost, m.stream),
-                      "hipMemcpyAsync");
+        enqueue_out(m, m.hidden.get(), m.config.dim);
         kv.length = valid;
         // the step kernels read the length from the device; the batched and
         // token-kernel paths do not advance it themselves
         kv.sync_length(m.stream);
         sync(m);
         check_token_error(m);
+        if (hidden != nullptr)
+            std::memcpy(hidden, host_words(m), m.config.dim * sizeof(float));
     }
     require(valid == count, NUT_EOUTOFRANGE, "quantized decode: token out of range");
 }
@@ -823,17 +834,16 @@ void logits(nut_model &m, const float *hidden, float *out)
     require(hidden != nullptr && out != nullptr, NUT_EINVAL, "logits: null pointer");
     check_ready(m, "logits");
     const size_t dim = m.config.dim;
-    hip_check(hipMemcpyAsync(m.scratch_hidden.get(), hidden, dim * sizeof(float),
-                             hipMemcpyHostToDevice, m.stream),
-              "hipMemcpyAsync");
+    std::memcpy(host_words(m), hidden, dim * sizeof(float));
+    launch_copy_words(host_words(m), m.scratch_hidden.get(), dim, nullptr, nullptr, m.stream);
     launch_reset_state(m.state.as<StepState>(), 0, m.stream);
     launch_classifier(m.shape, m.scratch_hidden.as<float>(), m.final_norm.as<float>(),
                       m.output_weights(), m.logits.as<float>(), m.part_val.as<float>(),
                       m.part_idx.as<int>(), m.state.as<StepState>(), m.stream);
-    hip_check(hipMemcpyAsync(out, m.logits.get(), m.config.vocab_size * sizeof(float),
-                             hipMemcpyDeviceToHost, m.stream),
-              "hipMemcpyAsync");
+    launch_copy_words(m.logits.get(), host_words(m), m.config.vocab_size, nullptr, nullptr,
+                      m.stream);
     sync(m);
+    std::memcpy(out, host_words(m), m.config.vocab_size * sizeof(float));
 }
 
 void generate_greedy(nut_model &m, const int *prompt, size_t prompt_len,
@@ -897,11 +907,11 @@ void generate_greedy(nut_model &m, const int *prompt, size_t prompt_len,
         }
     }
     hip_check(hipEventRecord(m.decode_end, m.stream), "hipEventRecord");
-    StepState host_state{};
-    hip_check(hipMemcpyAsync(&host_state, state, sizeof host_state,
-                             hipMemcpyDeviceToHost, m.stream),
-              "hipMemcpyAsync");
+    launch_copy_words(state, &host_area(m).state, sizeof(StepState) / sizeof(int), nullptr,
+                      nullptr, m.stream);
+    enqueue_out(m, m.tokens.get(), steps);
     sync(m);
+    const StepState host_state = host_area(m).state;
     const double t2 = now();
     check_token_error(m);
     float device_ms = 0.0f;
@@ -910,9 +920,7 @@ void generate_greedy(nut_model &m, const int *prompt, size_t prompt_len,
     m.last_decode_device_ms = device_ms;
     const size_t count = size_t(host_state.count);
     if (count > 0)
-        hip_check(hipMemcpy(out, m.tokens.get(), count * sizeof(int),
-                            hipMemcpyDeviceToHost),
-                  "hipMemcpy");
+        std::memcpy(out, host_words(m), count * sizeof(int));
     kv.length = prompt_len + count; // every emitted token was decoded
     *out_count = count;
     if (stats != nullptr) {
@@ -954,7 +962,6 @@ void generate_sampled(nut_model &m, const int *prompt, size_t prompt_len,
     std::vector<float> p;
     std::vector<int> ids;
     std::vector<double> totals;
-    constexpr size_t kChunk = 4096;
     size_t count = 0;
     StepState *state = m.state.as<StepState>();
     const int parts = classifier_blocks(s);
@@ -972,15 +979,20 @@ void generate_sampled(nut_model &m, const int *prompt, size_t prompt_len,
         const int nt = sample_sort(m.logits.as<float>(), vocab, m.part_val.as<float>(), parts,
                                    temperature, m.sample_ws.get(), &sorted_p, &sorted_ids,
                                    &token_p, &block_totals, &bad, m.stream);
+        // the block totals, the flag and the first candidates in one wait
         totals.resize(nt);
-        int bad_host = 0;
-        hip_check(hipMemcpyAsync(totals.data(), block_totals, nt * sizeof(double),
-                                 hipMemcpyDeviceToHost, m.stream),
-                  "hipMemcpyAsync");
-        hip_check(hipMemcpyAsync(&bad_host, bad, sizeof bad_host, hipMemcpyDeviceToHost,
-                                 m.stream),
-                  "hipMemcpyAsync");
+        const size_t first = std::min(kSampleChunk, size_t(vocab));
+        int *words = static_cast<int *>(host_words(m));
+        int *host_p = words + 2 * nt, *host_ids = host_p + kSampleChunk;
+        host_area(m).error = 0;
+        launch_copy_words(block_totals, words, 2 * size_t(nt), bad, &host_area(m).bad, m.stream);
+        launch_copy_words(sorted_p, host_p, first, nullptr, nullptr, m.stream);
+        launch_copy_words(sorted_ids, host_ids, first, m.token_error.as<int>(),
+                          &host_area(m).error, m.stream);
         sync(m);
+        check_token_error(m); // of the decode step before
+        std::memcpy(totals.data(), words, nt * sizeof(double));
+        const int bad_host = host_area(m).bad;
         if (bad_host != 0)
             fail(NUT_ERUNTIME, "sampling: non-finite probability");
         double total = 0.0;
@@ -990,11 +1002,11 @@ void generate_sampled(nut_model &m, const int *prompt, size_t prompt_len,
             fail(NUT_ERUNTIME, "sampling: zero probability mass");
         // the nucleus: the sorted prefix until its mass reaches top_p of the
         // total (src/generate.cpp:63-68), read in chunks
-        p.clear();
-        ids.clear();
+        p.assign(reinterpret_cast<float *>(host_p), reinterpret_cast<float *>(host_p) + first);
+        ids.assign(host_ids, host_ids + first);
         auto sorted = [&](size_t i) {
             if (i == p.size()) {
-                const size_t n = std::min(kChunk, size_t(vocab) - p.size());
+                const size_t n = std::min(kSampleChunk, size_t(vocab) - p.size());
                 p.resize(p.size() + n);
                 ids.resize(ids.size() + n);
                 hip_check(hipMemcpy(p.data() + i, sorted_p + i, n * sizeof(float),
@@ -1041,8 +1053,14 @@ void generate_sampled(nut_model &m, const int *prompt, size_t prompt_len,
         if (size_t(token) == m.config.eos_token)
             break;
         out[count++] = token;
-        decode(m, kv, token, nullptr);
+        // the step's end and its error flag are taken with the next token's
+        // candidates
+        enqueue_decode(m, kv, token);
+        kv.length += 1;
     }
+    enqueue_out(m, m.hidden.get(), 0);
+    sync(m);
+    check_token_error(m);
     const double t2 = now();
     *out_count = count;
     if (stats != nullptr) {

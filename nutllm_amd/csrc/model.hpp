@@ -86,6 +86,9 @@ struct nut_model {
     nut::DeviceBuffer pf_h, pf_x, pf_q, pf_ctx, pf_act;
     nut::DeviceBuffer pf_kv; // the batch's K and V as f16 limbs (prefill attention)
     nut::DeviceBuffer sample_ws; // sampling: numerators, sort buffers
+    // Page-locked host memory that calls exchange their arguments and results
+    // through (HostArea).
+    nut::PinnedBuffer host;
     size_t timeline_entries = 0; // > 0 when the phase timeline is recorded
     int timeline_wgs = 0;        // workgroups it covers
     unsigned launch_count = 0;
@@ -101,6 +104,25 @@ struct nut_model {
 };
 
 namespace nut {
+
+// Layout of nut_model::host: a header, then `words` (a hidden state, logits,
+// prompt or emitted tokens, or the sampler's totals and candidates), 16-byte
+// aligned.
+struct HostArea {
+    StepState state;
+    int error; // the token kernels' bounded-wait flag
+    int bad;   // sampling: a non-finite probability
+    int pad[2];
+};
+static_assert(sizeof(HostArea) % 16 == 0, "words are 16-byte aligned");
+constexpr size_t kSampleChunk = 4096; // sorted candidates read at once
+inline size_t host_words(const nut_config &c)
+{
+    const size_t sampler = 2 * 128 + 2 * kSampleChunk; // totals, then p and ids
+    size_t n = c.dim > c.vocab_size ? c.dim : c.vocab_size;
+    n = c.max_seq + 1 > n ? c.max_seq + 1 : n;
+    return (sampler > n ? sampler : n) + 4;
+}
 
 nut_model *create_model(const nut_config &config, int type, bool tied);
 void set_globals(nut_model &m, const float *embeddings,

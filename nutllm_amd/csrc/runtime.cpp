@@ -83,4 +83,17 @@ void DeviceBuffer::release()
     bytes_ = 0;
 }
 
+void PinnedBuffer::allocate(size_t bytes)
+{
+    release();
+    hip_check(hipHostMalloc(&ptr_, bytes, hipHostMallocMapped), "hipHostMalloc");
+}
+
+void PinnedBuffer::release()
+{
+    if (ptr_ != nullptr)
+        (void)hipHostFree(ptr_);
+    ptr_ = nullptr;
+}
+
 } // namespace nut

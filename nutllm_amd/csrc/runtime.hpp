@@ -55,4 +55,21 @@ private:
     size_t bytes_ = 0;
 };
 
+// RAII page-locked host memory, mapped into the device's address space:
+// kernels read and write it in place, and the host sees what a kernel wrote
+// once the stream has synchronised.
+class PinnedBuffer {
+public:
+    PinnedBuffer() = default;
+    ~PinnedBuffer() { release(); }
+    PinnedBuffer(const PinnedBuffer &) = delete;
+    PinnedBuffer &operator=(const PinnedBuffer &) = delete;
+    void allocate(size_t bytes);
+    void release();
+    template <typename T> T *as() const { return static_cast<T *>(ptr_); }
+
+private:
+    void *ptr_ = nullptr;
+};
+
 } // namespace nut

@@ -338,6 +338,40 @@ void check_fready(const nut_fmodel &m)
         require(l.set, NUT_EINVAL, "kv cache: layer count mismatch");
 }
 
+// One layer for t rows at positions first .. first + t - 1; `attend` puts
+// the rows' context into ctx from q and the layer's cache.
+template <class Attend>
+void launch_layer(const DecodeShape &s, const float *const (&w)[7], const float *attention_norm,
+                  const float *ffn_norm, const float2 *rope, float *kc, float *vc, float *h,
+                  float *q, float *ctx, float *act, int t, int first, hipStream_t stream,
+                  Attend &&attend)
+{
+    const int kvd = s.kv_heads * s.head_dim;
+    FGemm f{};
+    f.m = t;
+    f.to = ProjectOut{nullptr, rope, kc, vc, first, s.head_dim, s.max_seq};
+    auto gemm = [&](const float *x, const float *norm, int k, int w0, int count, int n0,
+                    float *out) {
+        f.x = x;
+        f.norm_w = norm;
+        f.k = k;
+        for (int i = 0; i < count; i++) {
+            f.w[i] = w[w0 + i];
+            f.n[i] = i == 0 ? n0 : w0 == 0 ? kvd : n0;
+        }
+        f.to.out = out;
+    };
+    gemm(h, attention_norm, s.dim, 0, 3, s.dim, q);
+    launch_fgemm<kQkv>(f, stream);
+    attend();
+    gemm(ctx, nullptr, s.dim, 3, 1, s.dim, h);
+    launch_fgemm<kAdd>(f, stream);
+    gemm(h, ffn_norm, s.dim, 4, 2, s.ffn_dim, act);
+    launch_fgemm<kSwiglu>(f, stream);
+    gemm(act, nullptr, s.ffn_dim, 6, 1, s.dim, h);
+    launch_fgemm<kAdd>(f, stream);
+}
+
 // The t tokens whose embeddings stand in h through every layer at positions
 // first .. first + t - 1 (first == 0 unless t == 1); their hidden states
 // stay in h.
@@ -345,7 +379,6 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
                     float *ctx, float *act)
 {
     const DecodeShape &s = m.shape;
-    const int kvd = s.kv_heads * s.head_dim;
     const size_t layer_elems = kv.layer_elements();
     const StepState *state = m.state.as<StepState>();
     const int *length = kv.device_length.as<int>();
@@ -353,41 +386,53 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
         const nut_fmodel::Layer &L = m.layers[l];
         float *kc = kv.keys.as<float>() + l * layer_elems;
         float *vc = kv.values.as<float>() + l * layer_elems;
-        FGemm f{};
-        f.m = t;
-        f.to = ProjectOut{nullptr, m.rope.as<float2>(), kc, vc, first, s.head_dim, s.max_seq};
-        auto gemm = [&](const float *x, const DeviceBuffer *norm, int k, int w0, int count, int n0,
-                        float *out) {
-            f.x = x;
-            f.norm_w = norm != nullptr ? norm->as<float>() : nullptr;
-            f.k = k;
-            for (int i = 0; i < count; i++) {
-                f.w[i] = L.w[w0 + i].as<float>();
-                f.n[i] = i == 0 ? n0 : w0 == 0 ? kvd : n0;
+        const float *w[7];
+        for (int i = 0; i < 7; i++)
+            w[i] = L.w[i].as<float>();
+        launch_layer(s, w, L.attention_norm.as<float>(), L.ffn_norm.as<float>(),
+                     m.rope.as<float2>(), kc, vc, h, q, ctx, act, t, first, m.stream, [&]() {
+            if (t == 1 && m.split_attention) {
+                launch_attention_split(s, q, kc, vc, length, m.attn_part.as<uint64_t>(),
+                                       m.attn_count.as<int>(), ctx, state, m.stream);
+            } else if (first == 0 && attention_f32_supported(s)) {
+                launch_attention_f32(s, q, kc, vc, ctx, t, m.stream);
+            } else {
+                for (int i = 0; i < t; i++) {
+                    if (t > 1)
+                        launch_set_int(kv.device_length.as<int>(), first + i, m.stream);
+                    launch_attention(s, q + size_t(i) * s.dim, kc, vc, length,
+                                     ctx + size_t(i) * s.dim, state, m.stream);
+                }
             }
-            f.to.out = out;
-        };
-        gemm(h, &L.attention_norm, s.dim, 0, 3, s.dim, q);
-        launch_fgemm<kQkv>(f, m.stream);
-        if (t == 1 && m.split_attention) {
-            launch_attention_split(s, q, kc, vc, length, m.attn_part.as<uint64_t>(),
-                                   m.attn_count.as<int>(), ctx, state, m.stream);
-        } else if (first == 0 && attention_f32_supported(s)) {
-            launch_attention_f32(s, q, kc, vc, ctx, t, m.stream);
-        } else {
-            for (int i = 0; i < t; i++) {
-                if (t > 1)
-                    launch_set_int(kv.device_length.as<int>(), first + i, m.stream);
-                launch_attention(s, q + size_t(i) * s.dim, kc, vc, length, ctx + size_t(i) * s.dim,
-                                 state, m.stream);
-            }
+        });
+    }
+}
+
+// dense[c][r] = row r, column c of m as fp32 (code times scale, exact): the
+// [in x out] layout of the projections here. A 32 x 32 tile per workgroup,
+// transposed in LDS so that both sides are read and written in rows.
+__global__ __launch_bounds__(256) void dense_kernel(QMat m, float *dense)
+{
+    __shared__ float tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
+    for (int y = ty; y < 32; y += 8) {
+        const int r = r0 + y, c = c0 + tx;
+        if (r < m.rows && c < m.cols) {
+            const size_t i = size_t(r) * m.cols + c;
+            int q;
+            if (m.type == 1)
+                q = int(uint32_t(m.data[i >> 1]) << ((i & 1) ? 24 : 28)) >> 28;
+            else
+                q = int(int8_t(m.data[i]));
+            tile[y][tx] = float(q) * half_bits_to_float(m.scales[i / m.block_size]);
         }
-        gemm(ctx, nullptr, s.dim, 3, 1, s.dim, h);
-        launch_fgemm<kAdd>(f, m.stream);
-        gemm(h, &L.ffn_norm, s.dim, 4, 2, s.ffn_dim, act);
-        launch_fgemm<kSwiglu>(f, m.stream);
-        gemm(act, nullptr, s.ffn_dim, 6, 1, s.dim, h);
-        launch_fgemm<kAdd>(f, m.stream);
+    }
+    __syncthreads();
+    for (int y = ty; y < 32; y += 8) {
+        const int r = r0 + tx, c = c0 + y;
+        if (r < m.rows && c < m.cols)
+            dense[size_t(c) * m.rows + r] = tile[tx][y];
     }
 }
 
@@ -419,6 +464,32 @@ void launch_attention_f32(const DecodeShape &s, const float *q, const float *k_l
     : s.head_dim == 64 ? launch_fattention<64>(s, q, k_layer, v_layer, ctx, t, stream)
     : s.head_dim == 32 ? launch_fattention<32>(s, q, k_layer, v_layer, ctx, t, stream)
                        : launch_fattention<16>(s, q, k_layer, v_layer, ctx, t, stream);
+}
+
+size_t dense_layer_floats(const DecodeShape &s)
+{
+    const size_t d = s.dim, kvd = size_t(s.kv_heads) * s.head_dim, f = s.ffn_dim;
+    return 2 * d * d + 2 * d * kvd + 3 * d * f;
+}
+
+void launch_layer_dense(const DecodeShape &s, const LayerView &w, const float2 *rope,
+                        float *k_layer, float *v_layer, const RowBuffers &b, int t, float *dense,
+                        hipStream_t stream)
+{
+    const QMat *mats[7] = {&w.query, &w.key, &w.value, &w.output, &w.gate, &w.up, &w.down};
+    const float *at[7];
+    for (int i = 0; i < 7; i++) {
+        const QMat &m = *mats[i];
+        hipLaunchKernelGGL(dense_kernel, dim3((m.cols + 31) / 32, (m.rows + 31) / 32), dim3(256),
+                           0, stream, m, dense);
+        at[i] = dense;
+        dense += size_t(m.rows) * m.cols;
+    }
+    check_launch("prefill: dense weights");
+    launch_layer(s, at, w.attention_norm, w.ffn_norm, rope, k_layer, v_layer, b.hidden, b.query,
+                 b.context, b.act, t, 0, stream, [&]() {
+        launch_attention_f32(s, b.query, k_layer, v_layer, b.context, t, stream);
+    });
 }
 
 nut_fmodel *create_fmodel(const nut_config &config, bool tied)

@@ -154,6 +154,14 @@ void launch_layer_rows(const DecodeShape &s, const LayerView &w, const float2 *r
                        float *k_layer, float *v_layer, const RowBuffers &b, int t,
                        hipStream_t stream);
 
+// The same for any block layout (fmodel.hip), attention_f32_supported shapes
+// and any t: the layer's weights as fp32 in `dense` (dense_layer_floats(s)
+// floats, free again when the layer is done), then the fp32 path's launches.
+size_t dense_layer_floats(const DecodeShape &s);
+void launch_layer_dense(const DecodeShape &s, const LayerView &w, const float2 *rope,
+                        float *k_layer, float *v_layer, const RowBuffers &b, int t, float *dense,
+                        hipStream_t stream);
+
 // dst[i] = src[i] for n 32-bit words; with `flag`, *flag_out = *flag too.
 // Either side may be page-locked host memory: a kernel between two others on
 // the stream, where a copy call for pageable memory stages, waits and returns

@@ -268,6 +268,44 @@ void prefill_rows(nut_model &m, nut_kvcache &kv, size_t count)
                       m.stream);
 }
 
+// Prompts of two tokens and more whose layers have no step kernel (head sizes
+// of 16 and 32, widths that no 32-wide block divides, other block sizes): a
+// layer's weights are written out as fp32 once for the whole prompt, where
+// the token-by-token way read and decoded them for every token (the tiny test
+// shape, 500 tokens: 42 ms of kernels, 84 ms with their launches).
+bool use_dense(const nut_model &m, size_t count)
+{
+    return m.path == 0 && count >= 2 && attention_f32_supported(m.shape) && !fast_steps(m);
+}
+
+void prefill_dense(nut_model &m, nut_kvcache &kv, size_t count)
+{
+    const DecodeShape &s = m.shape;
+    if (m.dn_weights.get() == nullptr)
+        m.dn_weights.allocate(dense_layer_floats(s) * sizeof(float));
+    if (count > m.dn_rows) {
+        // for the longest prompt so far
+        m.dn_rows = 0;
+        m.dn_hidden.allocate(count * s.dim * sizeof(float));
+        m.dn_query.allocate(count * s.dim * sizeof(float));
+        m.dn_context.allocate(count * s.dim * sizeof(float));
+        m.dn_act.allocate(count * s.ffn_dim * sizeof(float));
+        m.dn_rows = count;
+    }
+    const RowBuffers b{m.dn_hidden.as<float>(), m.dn_query.as<float>(),
+                       m.dn_context.as<float>(), m.dn_act.as<float>()};
+    launch_embed_rows(m.embeddings.as<float>(), m.prompt.as<int>(), b.hidden, int(count), s.dim,
+                      m.stream);
+    const size_t layer_elems = kv.layer_elements();
+    for (size_t l = 0; l < m.layers.size(); l++)
+        launch_layer_dense(s, m.layers[l].view, m.rope.as<float2>(),
+                           kv.keys.as<float>() + l * layer_elems,
+                           kv.values.as<float>() + l * layer_elems, b, int(count),
+                           m.dn_weights.as<float>(), m.stream);
+    launch_copy_words(b.hidden + (count - 1) * s.dim, m.hidden.get(), s.dim, nullptr, nullptr,
+                      m.stream);
+}
+
 // The batched prefill applies when every layer uses 32-wide blocks, the
 // head size matches its attention tiles, and per-token steps are not
 // forced.
@@ -805,6 +843,8 @@ void prefill(nut_model &m, nut_kvcache &kv, const int *tokens, size_t count,
             prefill_rows(m, kv, valid);
         } else if (use_prefill_gemm(m, valid)) {
             prefill_batch(m, kv, valid);
+        } else if (use_dense(m, valid)) {
+            prefill_dense(m, kv, valid);
         } else if (m.path != 2 && valid > 1 && fast_steps(m)) {
             prefill_steps(m, kv, valid);
         } else if (use_token_kernel(m, valid)) {

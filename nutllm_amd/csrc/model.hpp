@@ -72,6 +72,10 @@ struct nut_model {
     nut::DeviceBuffer mt_hidden, mt_query, mt_context, mt_act;
     // Short prompts on the row tiles: kRowGemmMax rows each.
     nut::DeviceBuffer rg_hidden, rg_query, rg_context, rg_act;
+    // Prompts of layouts without a step kernel: a layer's weights as fp32, and
+    // dn_rows rows of activations.
+    nut::DeviceBuffer dn_weights, dn_hidden, dn_query, dn_context, dn_act;
+    size_t dn_rows = 0;
     // One greedy iteration (classifier, argmax, decode step) captured as a
     // graph for the generation cache; replayed once per generated token.
     hipGraphExec_t step_graph = nullptr;

@@ -1,4 +1,5 @@
-"""Short prompts on the row tiles against the per-token step kernels.
+"""Short prompts on the row tiles, and prompts of a shape without step kernels
+(tiny) on fp32 weights, against the per-token kernels.
 
 Lengths at the edges of the tiles (16 and 32 rows) and of the range that takes
 them, INT8 and INT4, head sizes 64 and 128: the last hidden state, the K/V rows
@@ -19,7 +20,7 @@ def rel(a, b):
 
 
 @pytest.fixture(scope="module", params=[("step_gqa2", 0), ("step_gqa4", 1), ("step_mha128", 0),
-                                        ("step_mha128", 1)], ids=lambda p: f"{p[0]}-{p[1]}")
+                                        ("step_mha128", 1), ("tiny", 0), ("tiny", 1)], ids=lambda p: f"{p[0]}-{p[1]}")
 def model(request, gpu):
     shape, qtype = request.param
     m = W.build(shape, qtype, 31, max_seq=160, norm_seed=5)

@@ -333,6 +333,7 @@ void prefill_batch(nut_model &m, nut_kvcache &kv, size_t count)
         m.pf_act.allocate(rows * c.ffn_dim * sizeof(float));
         m.pf_q.allocate(rows * c.dim * sizeof(float));
         m.pf_ctx.allocate(rows * c.dim * sizeof(float));
+        m.pf_parts.allocate(3 * qgemm_parts_rows(s) * c.dim * sizeof(float));
         m.pf_kv.allocate(4 * prefill_kv_limb_elems(s) * sizeof(_Float16));
     }
     const int t = int(count);
@@ -341,7 +342,8 @@ void prefill_batch(nut_model &m, nut_kvcache &kv, size_t count)
     float *h = m.pf_h.as<float>();
     _Float16 *xh = m.pf_x.as<_Float16>(), *ch = m.pf_ctx.as<_Float16>();
     _Float16 *act_h = m.pf_act.as<_Float16>();
-    float *q = m.pf_q.as<float>();
+    float *q = m.pf_q.as<float>(), *parts = m.pf_parts.as<float>();
+    GemmParts rest{parts, 0, 0}; // products not yet added to h
     launch_embed_rows(m.embeddings.as<float>(), m.prompt.as<int>(), h, t, s.dim,
                       m.stream);
     const size_t layer_elems = kv.layer_elements();
@@ -351,8 +353,7 @@ void prefill_batch(nut_model &m, nut_kvcache &kv, size_t count)
         float *kc = kv.keys.as<float>() + l * layer_elems;
         float *vc = kv.values.as<float>() + l * layer_elems;
         const QMat *qkv_w[3] = {&w.query, &w.key, &w.value};
-        const QMat *wo = &w.output, *wd = &w.down;
-        launch_rmsnorm_rows(h, w.attention_norm, xh, xh + size_t(t) * s.dim, t, s.dim,
+        launch_rmsnorm_rows(h, rest, w.attention_norm, xh, xh + size_t(t) * s.dim, t, s.dim,
                             m.stream);
         // Q/K/V products, RoPE, the cache rows and the attention's K/V limbs
         // in one launch
@@ -360,17 +361,16 @@ void prefill_batch(nut_model &m, nut_kvcache &kv, size_t count)
                          vc, m.pf_kv.as<_Float16>(), s, m.stream);
         launch_attention_prefill(q, m.pf_kv.as<_Float16>(), ch, ch + size_t(t) * s.dim, s, t,
                                  m.stream);
-        launch_qgemm_rows(ch, ch + size_t(t) * s.dim, t, &wo, ss + 3, &h, &s.dim, 1, true,
-                          m.stream);
-        launch_rmsnorm_rows(h, w.ffn_norm, xh, xh + size_t(t) * s.dim, t, s.dim, m.stream);
+        rest = launch_qgemm_add(ch, ch + size_t(t) * s.dim, t, w.output, ss[3], h, parts,
+                                m.stream);
+        launch_rmsnorm_rows(h, rest, w.ffn_norm, xh, xh + size_t(t) * s.dim, t, s.dim, m.stream);
         // gate/up products and SwiGLU in one launch
         launch_qgemm_swiglu(xh, xh + size_t(t) * s.dim, t, w.gate, w.up, ss[4], ss[5],
                             act_h, act_h + size_t(t) * s.ffn_dim, m.stream);
-        launch_qgemm_rows(act_h, act_h + size_t(t) * s.ffn_dim, t, &wd, ss + 6, &h, &s.dim, 1,
-                          true, m.stream);
+        rest = launch_qgemm_add(act_h, act_h + size_t(t) * s.ffn_dim, t, w.down, ss[6], h, parts,
+                                m.stream);
     }
-    launch_copy_words(h + size_t(t - 1) * s.dim, m.hidden.get(), s.dim, nullptr, nullptr,
-                      m.stream);
+    launch_sum_row(h, rest, t - 1, m.hidden.as<float>(), s.dim, m.stream);
 }
 
 double now() { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); }

@@ -41,20 +41,35 @@ __global__ __launch_bounds__(kThreads) void embed_rows_kernel(
 // (wider rows read their remainder twice).
 constexpr int kRowVecs = 4;
 
-// One workgroup per token row; dim % 4 == 0.
+// One workgroup per token row; dim % 4 == 0. `count` partial products of the
+// GEMM before (launch_qgemm_add) are added to h first, in order, and h keeps
+// the sum.
 __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(
-    const float *h, const float *w, _Float16 *out_hi, _Float16 *out_lo, int dim)
+    float *h, const float *parts, int count, size_t part_stride, const float *w,
+    _Float16 *out_hi, _Float16 *out_lo, int dim)
 {
     __shared__ float red[kThreads / kWave];
-    const float4 *x = reinterpret_cast<const float4 *>(h + size_t(blockIdx.x) * dim);
+    float4 *x = reinterpret_cast<float4 *>(h + size_t(blockIdx.x) * dim);
     const float4 *w4 = reinterpret_cast<const float4 *>(w);
     const int n4 = dim / 4;
     float4 v[kRowVecs];
     float sq = 0.0f;
+    auto summed = [&](int i) {
+        float4 u = x[i];
+        if (count > 0) {
+            for (int p = 0; p < count; p++) {
+                const float4 a = reinterpret_cast<const float4 *>(
+                    parts + p * part_stride + size_t(blockIdx.x) * dim)[i];
+                u = make_float4(u.x + a.x, u.y + a.y, u.z + a.z, u.w + a.w);
+            }
+            x[i] = u;
+        }
+        return u;
+    };
 #pragma unroll
     for (int j = 0; j < kRowVecs; j++) {
         const int i = threadIdx.x + kThreads * j;
-        v[j] = i < n4 ? x[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        v[j] = i < n4 ? summed(i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
 #pragma unroll
     for (int j = 0; j < kRowVecs; j++) {
@@ -64,7 +79,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(
         sq = fmaf(v[j].w, v[j].w, sq);
     }
     for (int i = threadIdx.x + kThreads * kRowVecs; i < n4; i += kThreads) {
-        const float4 u = x[i];
+        const float4 u = summed(i);
         sq = fmaf(u.x, u.x, sq);
         sq = fmaf(u.y, u.y, sq);
         sq = fmaf(u.z, u.z, sq);
@@ -87,6 +102,20 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(
     }
     for (int i = threadIdx.x + kThreads * kRowVecs; i < n4; i += kThreads)
         put(i, x[i]);
+}
+
+// out = row + count partial rows, part_stride apart.
+__global__ __launch_bounds__(kThreads) void sum_row_kernel(const float *row, const float *parts,
+                                                           int count, size_t part_stride,
+                                                           float *out, int dim)
+{
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= dim)
+        return;
+    float v = row[i];
+    for (int p = 0; p < count; p++)
+        v += parts[p * part_stride + i];
+    out[i] = v;
 }
 
 // ------------------------------------- quantised GEMM on f16 MFMA --
@@ -132,6 +161,10 @@ struct GemmSegs {
     int ldc[3];
     int tiles[3];
     int count;
+    // kEpiAdd: k in gridDim.z runs; run 0 adds to c[0], run z stores to
+    // parts + (z - 1) * part_stride
+    float *parts;
+    size_t part_stride;
     // SwiGLU launches: w[0] gate, w[1] up; silu(gate) * up as limbs
     _Float16 *act_hi, *act_lo;
     int act_ld;
@@ -144,9 +177,9 @@ struct GemmSegs {
     int hd, max_seq, t_pad;
 };
 
-// What a GEMM launch does with its products: store, add to C (residual),
+// What a GEMM launch does with its products: add to C (residual),
 // silu(gate) * up as limbs, or RoPE + K/V cache and limb stores.
-enum Epilogue { kEpiStore = 0, kEpiAdd = 1, kEpiSwiglu = 2, kEpiQkv = 3 };
+enum Epilogue { kEpiAdd = 1, kEpiSwiglu = 2, kEpiQkv = 3 };
 
 // Source row of tile row r (0 .. 127) and its matrix (0 or 1): row n0 + r
 // of the segment's matrix; for a SwiGLU tile, gate and up rows alternate in
@@ -245,14 +278,15 @@ template <int QT, bool SWIGLU>
 __device__ __forceinline__ void qgemm_loader(const _Float16 *x_hi, const _Float16 *x_lo,
                                              int t_count, const QMat &w, const QMat &w_up,
                                              const uint32_t *st, const uint32_t *st_up,
-                                             int t0, int n0, GemmSlot<QT> *const (&slot)[kStages])
+                                             int t0, int n0, int stage0, int stages,
+                                             GemmSlot<QT> *const (&slot)[kStages])
 {
     constexpr int NW = QT == 1 ? 4 : 8; // weight instructions per stage
     constexpr int D = 16 + NW + 2;      // DMA instructions per stage
     constexpr int W_ROWS = QT == 1 ? 32 : 16;
     constexpr int W_STEP = QT == 1 ? FS / 2 : FS;
     const int lane = threadIdx.x & (kWave - 1);
-    const int k = w.cols, n_count = w.rows, stages = k / FS;
+    const int k = w.cols, n_count = w.rows;
     const size_t row_bytes = QT == 1 ? size_t(k) / 2 : size_t(k);
     size_t xoff[8];
 #pragma unroll
@@ -283,7 +317,7 @@ __device__ __forceinline__ void qgemm_loader(const _Float16 *x_hi, const _Float1
     for (int r = 0; r < kStages; r++)
         mb[r] = __builtin_amdgcn_readfirstlane(lds_addr(slot[r]));
     auto issue = [&](int r, int s) {
-        s = min(s, stages - 1); // past the end: reload the last stage
+        s = stage0 + min(s, stages - 1); // past the end: reload the last stage
         const size_t xs = size_t(s) * FS, ws = size_t(s) * W_STEP;
 #pragma unroll
         for (int i = 0; i < 8; i++)
@@ -344,15 +378,21 @@ __global__ __launch_bounds__(LOADER ? kThreads + kWave : kThreads) void qgemm_f1
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     // first output of the tile (SWIGLU: 64 outputs, 128 rows)
     const int t0 = blockIdx.y * FM_ROWS, n0 = tile * (SWIGLU ? FN / 2 : FN);
-    const int k = w.cols, n_count = w.rows, stages = k / FS;
+    const int k = w.cols, n_count = w.rows;
+    // this workgroup's run of the k stages
+    const int all = k / FS, z = ADD ? blockIdx.z : 0, runs = ADD ? gridDim.z : 1;
+    const int stage0 = ADD ? all * z / runs : 0;
+    const int stages = ADD ? all * (z + 1) / runs - stage0 : all;
+    if (ADD && z > 0)
+        c = segs.parts + size_t(z - 1) * segs.part_stride;
     const size_t row_bytes = QT == 1 ? size_t(k) / 2 : size_t(k);
     const QMat &w_up = segs.w[SWIGLU ? 1 : 0];
     const uint32_t *const st_up = segs.st[SWIGLU ? 1 : 0];
     if constexpr (LOADER) {
         if (wave == kThreads / kWave) {
             GemmSlot<QT> *const slots[kStages] = {&slot[0], &slot[1], &slot[2]};
-            qgemm_loader<QT, SWIGLU>(x_hi, x_lo, t_count, w, w_up, segs.st[seg], st_up, t0, n0,
-                                     slots);
+            qgemm_loader<QT, SWIGLU>(x_hi, x_lo, t_count, w, w_up, segs.st[seg], st_up, t0, n0, stage0,
+                                     stages, slots);
             return;
         }
     }
@@ -419,7 +459,7 @@ __global__ __launch_bounds__(LOADER ? kThreads + kWave : kThreads) void qgemm_f1
     const uint32_t m_junk = __builtin_amdgcn_readfirstlane(lds_addr(&junk[0]));
     auto issue = [&](int slot, int st) {
         const SlotM0 &m = m_slot[slot];
-        st = min(st, stages - 1); // past the end: reload the last stage
+        st = stage0 + min(st, stages - 1); // past the end: reload the last stage
         const size_t xs = size_t(st) * (FS * 2), ws = size_t(st) * W_STEP;
         dma16(xh0 + xs, m.xh0);
         dma16(xh1 + xs, m.xh1);
@@ -669,36 +709,26 @@ __global__ __launch_bounds__(LOADER ? kThreads + kWave : kThreads) void qgemm_f1
                 const int n = n0 + 32 * wave + 16 * j + li;
                 if (t < t_count && n < n_count) {
                     float *p = c + size_t(t) * ldc + n;
-                    *p = ADD ? *p + acc[i][j][v] : acc[i][j][v];
+                    *p = z == 0 ? *p + acc[i][j][v] : acc[i][j][v];
                 }
             }
 }
 
 template <int QT, int EPI>
 void launch_qgemm_form(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
-                       const GemmSegs &segs, hipStream_t stream)
+                       const GemmSegs &segs, int runs, hipStream_t stream)
 {
     int tiles = 0;
     for (int i = 0; i < segs.count; i++)
         tiles += segs.tiles[i];
-    const dim3 grid(tiles, (t_count + FM_ROWS - 1) / FM_ROWS);
+    const dim3 grid(tiles, (t_count + FM_ROWS - 1) / FM_ROWS, runs);
     // at most one workgroup per CU (MI355X: 256 CUs): the loader-wave form
-    if (size_t(grid.x) * grid.y <= 256)
+    if (size_t(grid.x) * grid.y * grid.z <= 256)
         hipLaunchKernelGGL((qgemm_f16_kernel<QT, EPI, true>), grid,
                            dim3(kThreads + kWave), 0, stream, x_hi, x_lo, t_count, segs);
     else
         hipLaunchKernelGGL((qgemm_f16_kernel<QT, EPI, false>), grid, dim3(kThreads), 0,
                            stream, x_hi, x_lo, t_count, segs);
-}
-
-template <int QT>
-void launch_qgemm(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
-                  const GemmSegs &segs, bool add, hipStream_t stream)
-{
-    if (add)
-        launch_qgemm_form<QT, kEpiAdd>(x_hi, x_lo, t_count, segs, stream);
-    else
-        launch_qgemm_form<QT, kEpiStore>(x_hi, x_lo, t_count, segs, stream);
 }
 
 // Causal attention of a prompt batch: queries t0 .. t0 + 63 at positions
@@ -990,13 +1020,22 @@ void launch_embed_rows(const float *embeddings, const int *tokens, float *h,
     check_launch("prefill embed");
 }
 
-void launch_rmsnorm_rows(const float *h, const float *w, _Float16 *out_hi,
+void launch_rmsnorm_rows(float *h, const GemmParts &add, const float *w, _Float16 *out_hi,
                          _Float16 *out_lo, int t_count, int dim, hipStream_t stream)
 {
     require(dim % 4 == 0, NUT_EINVAL, "prefill rmsnorm: dim must be a multiple of 4");
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(t_count), dim3(kThreads), 0,
-                       stream, h, w, out_hi, out_lo, dim);
+                       stream, h, add.data, add.count, add.stride, w, out_hi, out_lo, dim);
     check_launch("prefill rmsnorm");
+}
+
+void launch_sum_row(const float *h, const GemmParts &add, int row, float *out, int dim,
+                    hipStream_t stream)
+{
+    hipLaunchKernelGGL(sum_row_kernel, dim3((dim + kThreads - 1) / kThreads), dim3(kThreads), 0,
+                       stream, h + size_t(row) * dim, add.data + size_t(row) * dim, add.count,
+                       add.stride, out, dim);
+    check_launch("prefill: last row");
 }
 
 size_t stage_scale_words(const QMat &m)
@@ -1016,30 +1055,41 @@ void launch_scales_by_stage(const QMat &m, uint32_t *dst, hipStream_t stream)
     check_launch("prefill stage scales");
 }
 
-void launch_qgemm_rows(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
-                       const QMat *const *w, const uint32_t *const *stage_scales,
-                       float *const *c, const int *ldc, int count, bool add,
-                       hipStream_t stream)
+size_t qgemm_parts_rows(const DecodeShape &s)
 {
-    require(count >= 1 && count <= 3, NUT_EINVAL, "prefill gemm: 1 to 3 matrices");
+    // splits are for fewer than 256 tiles of 64 x 128
+    const size_t rows = size_t(FM_ROWS) * 256 * FN / s.dim + FM_ROWS;
+    return rows < size_t(s.max_seq) ? rows : size_t(s.max_seq);
+}
+
+GemmParts launch_qgemm_add(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
+                           const QMat &w, const uint32_t *stage_scales, float *c, float *parts,
+                           hipStream_t stream)
+{
+    require(w.cols % FS == 0 && stage_scales != nullptr, NUT_EINVAL,
+            "prefill gemm: rows of whole 64-wide stages with stage-major scales");
     GemmSegs segs{};
-    segs.count = count;
-    for (int i = 0; i < count; i++) {
-        require(w[i]->type == w[0]->type && w[i]->cols == w[0]->cols, NUT_EINVAL,
-                "prefill gemm: matrices differ in type or input size");
-        require(w[i]->cols % FS == 0 && stage_scales[i] != nullptr, NUT_EINVAL,
-                "prefill gemm: rows of whole 64-wide stages with stage-major scales");
-        segs.w[i] = *w[i];
-        segs.st[i] = stage_scales[i];
-        segs.c[i] = c[i];
-        segs.ldc[i] = ldc[i];
-        segs.tiles[i] = (w[i]->rows + FN - 1) / FN;
-    }
-    if (w[0]->type == 1)
-        launch_qgemm<1>(x_hi, x_lo, t_count, segs, add, stream);
+    segs.count = 1;
+    segs.w[0] = w;
+    segs.st[0] = stage_scales;
+    segs.c[0] = c;
+    segs.ldc[0] = w.rows;
+    segs.tiles[0] = (w.rows + FN - 1) / FN;
+    segs.parts = parts;
+    segs.part_stride = size_t(t_count) * w.rows;
+    // k in up to four runs where the tiles alone leave CUs idle; a run keeps
+    // eight stages at least
+    const int tiles = segs.tiles[0] * ((t_count + FM_ROWS - 1) / FM_ROWS);
+    int runs = tiles >= 256 ? 1 : 384 / tiles;
+    runs = runs > 4 ? 4 : runs < 1 ? 1 : runs;
+    while (runs > 1 && w.cols / FS < 8 * runs)
+        runs--;
+    if (w.type == 1)
+        launch_qgemm_form<1, kEpiAdd>(x_hi, x_lo, t_count, segs, runs, stream);
     else
-        launch_qgemm<0>(x_hi, x_lo, t_count, segs, add, stream);
+        launch_qgemm_form<0, kEpiAdd>(x_hi, x_lo, t_count, segs, runs, stream);
     check_launch("prefill gemm");
+    return GemmParts{parts, runs - 1, segs.part_stride};
 }
 
 void launch_qgemm_swiglu(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
@@ -1062,9 +1112,9 @@ void launch_qgemm_swiglu(const _Float16 *x_hi, const _Float16 *x_lo, int t_count
     segs.act_lo = act_lo;
     segs.act_ld = gate.rows;
     if (gate.type == 1)
-        launch_qgemm_form<1, kEpiSwiglu>(x_hi, x_lo, t_count, segs, stream);
+        launch_qgemm_form<1, kEpiSwiglu>(x_hi, x_lo, t_count, segs, 1, stream);
     else
-        launch_qgemm_form<0, kEpiSwiglu>(x_hi, x_lo, t_count, segs, stream);
+        launch_qgemm_form<0, kEpiSwiglu>(x_hi, x_lo, t_count, segs, 1, stream);
     check_launch("prefill gemm swiglu");
 }
 
@@ -1111,9 +1161,9 @@ void launch_qgemm_qkv(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
     segs.max_seq = s.max_seq;
     segs.t_pad = t_pad;
     if (w[0]->type == 1)
-        launch_qgemm_form<1, kEpiQkv>(x_hi, x_lo, t_count, segs, stream);
+        launch_qgemm_form<1, kEpiQkv>(x_hi, x_lo, t_count, segs, 1, stream);
     else
-        launch_qgemm_form<0, kEpiQkv>(x_hi, x_lo, t_count, segs, stream);
+        launch_qgemm_form<0, kEpiQkv>(x_hi, x_lo, t_count, segs, 1, stream);
     check_launch("prefill gemm qkv");
 }
 

@@ -14,22 +14,34 @@ bool prefill_gemm_supported(const DecodeShape &s, const LayerView &w);
 
 void launch_embed_rows(const float *embeddings, const int *tokens, float *h,
                        int t_count, int dim, hipStream_t stream);
+// Partial products that launch_qgemm_add left: `count` sets of rows, stride
+// floats apart.
+struct GemmParts {
+    const float *data;
+    int count;
+    size_t stride;
+};
 // GEMM inputs are written as two f16 limbs per value: hi = f16(v) and
-// lo = f16(v - hi), [t][k] each.
-void launch_rmsnorm_rows(const float *h, const float *w, _Float16 *out_hi,
+// lo = f16(v - hi), [t][k] each. h += the parts first.
+void launch_rmsnorm_rows(float *h, const GemmParts &add, const float *w, _Float16 *out_hi,
                          _Float16 *out_lo, int t_count, int dim, hipStream_t stream);
+// out = row `row` of h + the parts.
+void launch_sum_row(const float *h, const GemmParts &add, int row, float *out, int dim,
+                    hipStream_t stream);
 // The prefill GEMM reads each matrix's fp16 scales stage-major: dword
 // [st][row] holds the scales of blocks 2 st and 2 st + 1 of the row
 // (stage_scale_words(m) dwords, built once per matrix).
 size_t stage_scale_words(const QMat &m);
 void launch_scales_by_stage(const QMat &m, uint32_t *dst, hipStream_t stream);
-// c_i[t][n] (= or +=) sum_k x[t][k] w_i[n][k] for `count` (1 to 3)
-// matrices of one type and input size, t < t_count, in one launch; x as
-// limbs of w.cols values per row, c_i rows ldc_i floats.
-void launch_qgemm_rows(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
-                       const QMat *const *w, const uint32_t *const *stage_scales,
-                       float *const *c, const int *ldc, int count, bool add,
-                       hipStream_t stream);
+// c[t][n] += sum_k x[t][k] w[n][k], t < t_count, rows of w.rows floats; x as
+// limbs of w.cols values per row. Where the tiles leave CUs idle, k is split:
+// the first run's products are added to c and those of the others go to
+// `parts` (up to three sets of t_count rows, qgemm_parts_rows(s) rows at
+// most), which the next launch_rmsnorm_rows or launch_sum_row adds.
+size_t qgemm_parts_rows(const DecodeShape &s);
+GemmParts launch_qgemm_add(const _Float16 *x_hi, const _Float16 *x_lo, int t_count,
+                           const QMat &w, const uint32_t *stage_scales, float *c, float *parts,
+                           hipStream_t stream);
 // act[t][n] = silu(gate[n] . x[t]) * (up[n] . x[t]) as limbs (act_hi,
 // act_lo, gate.rows values per row): both products in one launch, each
 // workgroup 64 outputs of both matrices, so neither product leaves the

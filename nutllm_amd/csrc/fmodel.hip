@@ -124,7 +124,12 @@ void launch_ftile(FGemm &f, hipStream_t stream)
 }
 
 // The tile by the model of gemm_f32_choose over all the launch's columns
-// (gate and up count twice). Up to 16 rows the weights' way from HBM is what
+// (gate and up count twice), with factors measured here, where the weights
+// come from HBM and a chunk's sums are added apart: gate/up of 301 rows 24 176
+// us (44 194, 34 187, 22 192, 14 202), of 64 22 49 (44 51, 24 59), of 20 24 31
+// (44 50, 22 41); W2 of 301 rows 34 87 (44 110, 22 98), of 150 24 62 (34 87,
+// 22 64), of 64 12 28 (22 37, 14 37); Q/K/V of 301 rows 14 38 (44 48, 24 47).
+// Up to 16 rows the weights' way from HBM is what
 // counts: sixteen waves share the k of a narrow tile, so that the whole chip
 // has its loads in flight at once.
 template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
@@ -144,20 +149,24 @@ template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
         }
         return;
     }
-    const GemmTile t = gemm_f32_choose(f.m, f.k, n);
+    const GemmTile tiles[] = {{4, 4, 1.6, 0},  {3, 4, 1.65, 0}, {2, 4, 1.65, 0},
+                              {2, 2, 1.85, 0}, {1, 4, 1.95, 0}, {1, 2, 2.4, 0}};
+    const GemmTile t = gemm_f32_pick(tiles, f.m, f.k, n);
     switch (t.ti * 10 + t.tj) {
     case 44:
         launch_ftile<4, 4, 4, 1, EPI>(f, stream);
         break;
     case 34:
-    case 33: // whole RoPE pairs, and gate and up alike
-        launch_ftile<3, 4, 4, 2, EPI>(f, stream);
+        launch_ftile<3, 4, 4, 1, EPI>(f, stream);
         break;
     case 24:
         launch_ftile<2, 4, 4, 2, EPI>(f, stream);
         break;
     case 22:
-        launch_ftile<2, 2, 8, 1, EPI>(f, stream);
+        launch_ftile<2, 2, 4, 2, EPI>(f, stream);
+        break;
+    case 14:
+        launch_ftile<1, 4, 4, 1, EPI>(f, stream);
         break;
     default:
         launch_ftile<1, 2, 8, 2, EPI>(f, stream);

@@ -337,19 +337,16 @@ inline unsigned gemm_f32_grid(int tiles_m, int tiles_n)
 // 1,080 us (24 1,266, 22 1,340).
 struct GemmTile {
     int ti, tj;
+    double factor;
     long long count;
 };
 
-inline GemmTile gemm_f32_choose(int m, int k, int n)
+template <size_t N>
+inline GemmTile gemm_f32_pick(const GemmTile (&tiles)[N], int m, int k, int n)
 {
-    const struct {
-        int ti, tj;
-        double factor;
-    } tiles[] = {{4, 4, 1.24}, {3, 4, 1.39}, {3, 3, 1.31}, {2, 4, 1.45},
-                 {2, 2, 1.48}, {1, 2, 1.8},  {1, 1, 2.4}};
-    GemmTile best{1, 1, 0};
+    GemmTile best{};
     double least = 0.0;
-    for (const auto &t : tiles) {
+    for (const GemmTile &t : tiles) {
         if (n < t.tj)
             continue;
         const int rows = 16 * t.ti, cols = 16 * t.tj;
@@ -359,10 +356,18 @@ inline GemmTile gemm_f32_choose(int m, int k, int n)
             double((count + 255) / 256) * (double(rows) * cols * k / 128.0 * t.factor + 2000.0);
         if (best.count == 0 || cycles < least) {
             least = cycles;
-            best = GemmTile{t.ti, t.tj, count};
+            best = t;
+            best.count = count;
         }
     }
     return best;
+}
+
+inline GemmTile gemm_f32_choose(int m, int k, int n)
+{
+    const GemmTile tiles[] = {{4, 4, 1.24, 0}, {3, 4, 1.39, 0}, {3, 3, 1.31, 0}, {2, 4, 1.45, 0},
+                              {2, 2, 1.48, 0}, {1, 2, 1.8, 0},  {1, 1, 2.4, 0}};
+    return gemm_f32_pick(tiles, m, k, n);
 }
 
 // C = A B; a workgroup of WM x WN x WK waves owns WM x WN tiles, WK waves

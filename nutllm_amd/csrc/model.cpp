@@ -218,12 +218,13 @@ size_t prefill_gemm_min(const DecodeShape &s)
 // Prompts of these lengths run on the row tiles (rowgemm.hip), where every
 // layer has their layout and per-token steps are not forced. A tile costs
 // the same for 2 rows as for 16, a step-kernel chunk a little per token; the
-// batched GEMM wins once its 64 x 128 tiles fill the chip. TinyLlama INT4,
-// row tiles against the better of the two: 5 tokens 1.01 ms (1.02), 9 1.02
-// (1.36), 16 1.05 (1.95), 20 1.53 (2.28), 64 1.83 (3.30), 96 2.58 (3.33), 128
-// 3.08 (3.39); two layers of the 7B widths INT4: 2 tokens 0.27 (0.20), 5 0.27
-// (0.31), 16 0.26 (0.55), 64 0.49 (0.57), 65 0.74 (0.62). Small widths are
-// bound by the launches, five a layer in each.
+// batched GEMM wins where its 64 x 128 tiles and its runs of k fill the
+// chip. TinyLlama INT4, row tiles against the better of the two: 5 tokens
+// 1.01 ms (1.02), 9 1.02 (1.36), 16 1.05 (1.95), 20 1.53 (2.28), 48 1.79
+// (2.21), 64 1.83 (2.32), 80 2.84 (2.34); two layers of the 7B widths INT4: 2
+// tokens 0.27 (0.20), 5 0.27 (0.31), 16 0.26 (0.35), 32 0.36 (0.34), 48 0.50
+// (0.35). Small widths are bound by the launches, five a layer against seven
+// (step_gqa4, 128 tokens: 0.11 against 0.17).
 size_t row_gemm_min(const DecodeShape &s)
 {
     return s.dim < 1024 ? 2 : s.dim < 4096 ? 6 : 5;
@@ -231,7 +232,7 @@ size_t row_gemm_min(const DecodeShape &s)
 
 size_t row_gemm_max(const DecodeShape &s)
 {
-    return s.dim < 4096 ? size_t(kRowGemmMax) : 64;
+    return s.dim < 1024 ? size_t(kRowGemmMax) : s.dim < 4096 ? 64 : 16;
 }
 
 bool use_row_gemm(const nut_model &m, size_t count)

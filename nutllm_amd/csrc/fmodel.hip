@@ -42,6 +42,9 @@ struct FGemm {
     int n[3], tiles[3];
     int tiles_m, tiles_n;
     ProjectOut to;
+    // kAdd: k in gridDim.y runs; run 0 adds to the hidden rows, run r stores
+    // to parts + (r - 1) * m * n[0]
+    float *parts;
 };
 
 template <int TI, int TJ, int WK, int D, int EPI>
@@ -77,7 +80,8 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
     gemm_f32_clear(acc);
     int c0, c1;
     bool tail;
-    gemm_f32_share<WK>(k, wave, c0, c1, tail);
+    const int run = EPI == kAdd ? blockIdx.y : 0, runs = EPI == kAdd ? gridDim.y : 1;
+    gemm_f32_share(k, run * WK + wave, runs * WK, c0, c1, tail);
     gemm_f32_run<TI, TJ, NB, 0, D, NORM>(pa, pb, size_t(n),
                                           NORM ? f.norm_w + 4 * (lane & 7) : nullptr, k, c0, c1,
                                           tail, lds + wave * 16 * TI * kChunkLd, acc, sq);
@@ -104,12 +108,33 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
             for (int j = 0; j < TJ; j++)
                 out[j] *= scale;
         }
+        if (EPI == kAdd && run > 0) {
+            float *dst = f.parts + (size_t(run - 1) * m + row) * n + first;
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+                if (first + j >= col)
+                    dst[j] = out[j];
+            return;
+        }
         project_store<EPI, TJ>(f.to, seg, n, row, col, first, out);
     });
 }
 
+// h += the runs' products, in order; n floats a run.
+__global__ __launch_bounds__(256) void add_parts_kernel(float *h, const float *parts, int count,
+                                                        int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n)
+        return;
+    float v = h[i];
+    for (int p = 0; p < count; p++)
+        v += parts[size_t(p) * n + i];
+    h[i] = v;
+}
+
 template <int TI, int TJ, int WK, int D, int EPI>
-void launch_ftile(FGemm &f, hipStream_t stream)
+void launch_ftile(FGemm &f, hipStream_t stream, int runs = 1)
 {
     const int cols = 16 * TJ / (EPI == kSwiglu ? 2 : 1);
     f.tiles_m = (f.m + 16 * TI - 1) / (16 * TI);
@@ -119,9 +144,11 @@ void launch_ftile(FGemm &f, hipStream_t stream)
         f.tiles_n += f.tiles[s];
     }
     hipLaunchKernelGGL((fgemm_kernel<TI, TJ, WK, D, EPI>),
-                       dim3(gemm_f32_grid(f.tiles_m, f.tiles_n)), dim3(64 * WK), 0, stream, f);
+                       dim3(gemm_f32_grid(f.tiles_m, f.tiles_n), runs), dim3(64 * WK), 0, stream, f);
     check_launch("fp32 model: projection");
 }
+
+constexpr int kFRuns = 4; // most runs of k
 
 // The tile by the model of gemm_f32_choose over all the launch's columns
 // (gate and up count twice), with factors measured here, where the weights
@@ -141,6 +168,18 @@ template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
         n *= 2;
     if (f.m <= 16) {
         if constexpr (EPI == kAdd) {
+            // k of a long product (W2) in runs, so that all CUs read whole
+            // 128-byte lines of it: 46 MB 24 -> 14 us with the sums'
+            // launch. A product as short as Wo takes as long either way.
+            const int tiles = (n + 31) / 32;
+            const int runs = std::min(kFRuns, 256 / tiles);
+            if (f.parts != nullptr && runs > 1 && f.k >= 4096) {
+                launch_ftile<1, 2, 8, 2, EPI>(f, stream, runs);
+                hipLaunchKernelGGL(add_parts_kernel, dim3((f.m * n + 255) / 256), dim3(256), 0,
+                                   stream, f.to.out, f.parts, runs - 1, f.m * n);
+                check_launch("fp32 model: sums");
+                return;
+            }
             n >= 4096 ? launch_ftile<1, 2, 16, 2, EPI>(f, stream)
                       : launch_ftile<1, 1, 16, 3, EPI>(f, stream);
         } else {
@@ -348,16 +387,18 @@ void check_fready(const nut_fmodel &m)
 }
 
 // One layer for t rows at positions first .. first + t - 1; `attend` puts
-// the rows' context into ctx from q and the layer's cache.
+// the rows' context into ctx from q and the layer's cache. parts: room for
+// kFRuns - 1 products of 16 rows, or null.
 template <class Attend>
 void launch_layer(const DecodeShape &s, const float *const (&w)[7], const float *attention_norm,
                   const float *ffn_norm, const float2 *rope, float *kc, float *vc, float *h,
-                  float *q, float *ctx, float *act, int t, int first, hipStream_t stream,
-                  Attend &&attend)
+                  float *q, float *ctx, float *act, float *parts, int t, int first,
+                  hipStream_t stream, Attend &&attend)
 {
     const int kvd = s.kv_heads * s.head_dim;
     FGemm f{};
     f.m = t;
+    f.parts = parts;
     f.to = ProjectOut{nullptr, rope, kc, vc, first, s.head_dim, s.max_seq};
     auto gemm = [&](const float *x, const float *norm, int k, int w0, int count, int n0,
                     float *out) {
@@ -399,7 +440,8 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
         for (int i = 0; i < 7; i++)
             w[i] = L.w[i].as<float>();
         launch_layer(s, w, L.attention_norm.as<float>(), L.ffn_norm.as<float>(),
-                     m.rope.as<float2>(), kc, vc, h, q, ctx, act, t, first, m.stream, [&]() {
+                     m.rope.as<float2>(), kc, vc, h, q, ctx, act, m.parts.as<float>(), t, first,
+                     m.stream, [&]() {
             if (t == 1 && m.split_attention) {
                 launch_attention_split(s, q, kc, vc, length, m.attn_part.as<uint64_t>(),
                                        m.attn_count.as<int>(), ctx, state, m.stream);
@@ -496,7 +538,7 @@ void launch_layer_dense(const DecodeShape &s, const LayerView &w, const float2 *
     }
     check_launch("prefill: dense weights");
     launch_layer(s, at, w.attention_norm, w.ffn_norm, rope, k_layer, v_layer, b.hidden, b.query,
-                 b.context, b.act, t, 0, stream, [&]() {
+                 b.context, b.act, nullptr, t, 0, stream, [&]() {
         launch_attention_f32(s, b.query, k_layer, v_layer, b.context, t, stream);
     });
 }
@@ -529,6 +571,7 @@ nut_fmodel *create_fmodel(const nut_config &config, bool tied)
     m->context.allocate(config.dim * sizeof(float));
     m->act.allocate(config.ffn_dim * sizeof(float));
     m->host.allocate(config.dim * sizeof(float));
+    m->parts.allocate(size_t(kFRuns - 1) * 16 * config.dim * sizeof(float));
     m->state.allocate(sizeof(StepState));
     m->token.allocate(sizeof(int));
     hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "hipStreamCreate");

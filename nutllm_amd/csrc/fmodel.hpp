@@ -25,6 +25,7 @@ struct nut_fmodel {
     nut::DeviceBuffer embeddings, final_norm, lm_head, rope;
     // workspace of one decode step
     nut::DeviceBuffer hidden, query, context, act, state, token;
+    nut::DeviceBuffer parts; // products of the runs of k of up to 16 rows
     // a decode step's split attention (step.hip), where the shape has it
     bool split_attention = false;
     nut::DeviceBuffer attn_part, attn_count;

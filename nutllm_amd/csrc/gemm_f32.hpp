@@ -221,14 +221,14 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
     }
 }
 
-// Chunks [c0, c1) of wave w's share of k, and whether it takes the tail.
-template <int WK>
-__device__ __forceinline__ void gemm_f32_share(int k, int wave, int &c0, int &c1, bool &tail)
+// Chunks [c0, c1) of share `i` of `count` of k, and whether it takes the tail.
+__device__ __forceinline__ void gemm_f32_share(int k, int i, int count, int &c0, int &c1,
+                                               bool &tail)
 {
     const int full = k / kChunk;
-    c0 = int((long long)full * wave / WK);
-    c1 = int((long long)full * (wave + 1) / WK);
-    tail = wave == WK - 1 && k % kChunk != 0;
+    c0 = int((long long)full * i / count);
+    c1 = int((long long)full * (i + 1) / count);
+    tail = i == count - 1 && k % kChunk != 0;
 }
 
 template <int TI, int TJ, int NA>
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f32_wave(
     gemm_f32_clear(acc);
     int c0, c1;
     bool tail;
-    gemm_f32_share<WK>(k, wk, c0, c1, tail);
+    gemm_f32_share(k, wk, WK, c0, c1, tail);
     gemm_f32_run<TI, TJ, 1, NA, D, false>(pa, pb, size_t(n), nullptr, k, c0, c1, tail,
                                     lds + wave * 16 * TI * kChunkLd, acc, sq);
     if (WK > 1)

@@ -2,7 +2,7 @@
 transformer, at the edges of their tiles: one row, one less and one more than
 a 16-row attention tile and a 64-key block, prompts long enough for every GEMM
 tile, head sizes with an attention kernel of their own and one without, widths
-that no 32-wide k chunk divides.
+that no 32-wide k chunk divides, a feed-forward width whose product is split.
 
 The bound on the relative error (2-norm) is 5e-6 per call: an fp32 chain of k
 terms errs by about sqrt(k) 2^-24 relative to its rms, k <= 300 here, over two
@@ -19,6 +19,7 @@ SHAPES = {
     "hd64": (4, 1, 64, 300, 64),
     "hd128": (2, 2, 128, 257, 40),
     "hd48": (2, 1, 48, 130, 33),
+    "long": (2, 1, 64, 4131, 30),  # W2's k in runs, the last with a tail
 }
 
 

@@ -331,9 +331,9 @@ inline unsigned gemm_f32_grid(int tiles_m, int tiles_n)
 // MFMA cycles of the whole tile times what L2 traffic and the waves' own
 // overhead add for that tile at 4096^3 (44: 1.24, 34: 1.39, 33: 1.31, 24:
 // 1.45, 22: 1.48, 12: 1.8, 11: 2.4), plus a start and an end. Measured, the
-// pick against the others: 768^3 33 12.8 us (44 18.6, 34 14.8, 22 16.3),
-// 1000 x 2047 x 1531 24 67 us (44 80, 34 67-73, 22 72), 313^3 12 4.6 us (22
-// 5.6, 44 12.6), 64 x 4096 x 256 11 10.5 us (12 13.4, 22 23.5), 4096^3 44
+// pick against the others: 768^3 33 12.1 us (44 18.6, 34 14.8, 22 16.3),
+// 1000 x 2047 x 1531 34 66 us (44 80, 24 67, 22 72), 313^3 12 4.6 us (22 5.6,
+// 44 12.6), 64 x 4096 x 256 11 10.5 us (12 13.4, 22 23.5), 4096^3 44
 // 1,080 us (24 1,266, 22 1,340).
 struct GemmTile {
     int ti, tj;

@@ -14,7 +14,7 @@ void launch_tile(const float *a, const float *b, float *c, int m, int k, int n,
                  hipStream_t stream)
 {
     const int tiles_m = (m + 16 * TI - 1) / (16 * TI), tiles_n = (n + 16 * TJ - 1) / (16 * TJ);
-    hipLaunchKernelGGL((matmul_f32_wave<TI, TJ, 1, 1, WK, NA, D>),
+    hipLaunchKernelGGL((matmul_f32_wave<TI, TJ, WK, NA, D>),
                        dim3(gemm_f32_grid(tiles_m, tiles_n)), dim3(64 * WK), 0, stream, a, b, c,
                        m, k, n, tiles_m, tiles_n);
 }

@@ -246,12 +246,13 @@ __device__ __forceinline__ void gemm_f32_clear(floatx4 (&acc)[NA][TI][TJ])
 // Adds the partial tiles of the WK waves that share a tile (`red`: theirs,
 // WK * TJ * 256 floats of LDS; wk: this wave's place) and hands every output
 // row's columns to epi(i, v, vals): row 16 i + 4 g + v of the tile, this
-// lane's TJ columns. Wave wk takes the v of 4 wk / WK ..; called by the whole
+// lane's TJ columns, from wave v for each of the four v; called by the whole
 // workgroup.
 template <int TI, int TJ, int WK, int NS, class Epi>
 __device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NS][TI][TJ], float *red,
                                                 int wk, Epi &&epi)
 {
+    static_assert(WK >= 4, "wave v takes element v");
     const int lane = threadIdx.x & 63;
     floatx4(&acc)[TI][TJ] = parts[0];
 #pragma unroll
@@ -261,20 +262,6 @@ __device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NS][TI][TJ], fl
 #pragma unroll
             for (int j = 0; j < TJ; j++)
                 acc[i][j] += parts[u][i][j];
-    if constexpr (WK == 1) {
-#pragma unroll
-        for (int i = 0; i < TI; i++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                float out[TJ];
-#pragma unroll
-                for (int j = 0; j < TJ; j++)
-                    out[j] = acc[i][j][v];
-                epi(i, v, out);
-            }
-        return;
-    }
-    constexpr int VS = WK >= 4 ? 1 : 4 / WK; // v per wave
 #pragma unroll
     for (int i = 0; i < TI; i++) {
         if (i > 0)
@@ -285,21 +272,17 @@ __device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NS][TI][TJ], fl
             for (int v = 0; v < 4; v++)
                 red[((wk * TJ + j) * 4 + v) * 64 + lane] = acc[i][j][v];
         __syncthreads();
-        if (wk * VS < 4) {
+        if (wk < 4) {
+            float out[TJ];
 #pragma unroll
-            for (int u = 0; u < VS; u++) {
-                const int v = wk * VS + u;
-                float out[TJ];
+            for (int j = 0; j < TJ; j++) {
+                float s = red[(j * 4 + wk) * 64 + lane];
 #pragma unroll
-                for (int j = 0; j < TJ; j++) {
-                    float s = red[(j * 4 + v) * 64 + lane];
-#pragma unroll
-                    for (int w = 1; w < WK; w++)
-                        s += red[((w * TJ + j) * 4 + v) * 64 + lane];
-                    out[j] = s;
-                }
-                epi(i, v, out);
+                for (int w = 1; w < WK; w++)
+                    s += red[((w * TJ + j) * 4 + wk) * 64 + lane];
+                out[j] = s;
             }
+            epi(i, wk, out);
         }
     }
 }
@@ -370,24 +353,22 @@ inline GemmTile gemm_f32_choose(int m, int k, int n)
     return gemm_f32_pick(tiles, m, k, n);
 }
 
-// C = A B; a workgroup of WM x WN x WK waves owns WM x WN tiles, WK waves
-// sharing the k of each.
-template <int TI, int TJ, int WM, int WN, int WK, int NA, int D>
-__global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f32_wave(
+// C = A B, a tile per workgroup, whose WK waves share its k.
+template <int TI, int TJ, int WK, int NA, int D>
+__global__ __launch_bounds__(64 * WK) void matmul_f32_wave(
     const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c, int m, int k,
     int n, int tiles_m, int tiles_n)
 {
     // the waves' A chunks, then their partial tiles
-    constexpr int kStage = WM * WN * WK * 16 * TI * kChunkLd;
-    constexpr int kRed = WK == 1 ? 0 : WM * WN * WK * TJ * 256;
+    constexpr int kStage = WK * 16 * TI * kChunkLd;
+    constexpr int kRed = WK * TJ * 256;
     __shared__ __attribute__((aligned(16))) float lds[kStage > kRed ? kStage : kRed];
     int tm, tn;
     if (!gemm_f32_tile(tiles_m, tiles_n, tm, tn))
         return; // workgroup-uniform
     const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wk = wave % WK, wn = wave / WK % WN, wm = wave / (WK * WN);
-    const int row0 = (tm * WM + wm) * 16 * TI, col = (tn * WN + wn) * 16 * TJ + TJ * li;
+    const int row0 = tm * 16 * TI, col = tn * 16 * TJ + TJ * li;
     const int first = min(col, n - TJ); // n >= TJ
     const float *pa[2 * TI];
 #pragma unroll
@@ -399,13 +380,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f32_wave(
     gemm_f32_clear(acc);
     int c0, c1;
     bool tail;
-    gemm_f32_share(k, wk, WK, c0, c1, tail);
+    gemm_f32_share(k, wave, WK, c0, c1, tail);
     gemm_f32_run<TI, TJ, 1, NA, D, false>(pa, pb, size_t(n), nullptr, k, c0, c1, tail,
                                     lds + wave * 16 * TI * kChunkLd, acc, sq);
-    if (WK > 1)
-        __syncthreads();
+    __syncthreads();
     gemm_f32_reduce<TI, TJ, WK>(
-        acc, lds + (wm * WN + wn) * WK * TJ * 256, wk,
+        acc, lds, wave,
         [&](int i, int v, const float (&out)[TJ]) {
             const int row = row0 + 16 * i + 4 * g + v;
             if (row >= m || col >= n)

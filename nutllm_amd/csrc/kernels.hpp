@@ -140,7 +140,7 @@ bool attention_f32_supported(const DecodeShape &s);
 void launch_attention_f32(const DecodeShape &s, const float *q, const float *k_layer,
                           const float *v_layer, float *ctx, int t, hipStream_t stream);
 
-// The projections of a short prompt's rows on f16 MFMA (rowgemm.hip), t <=
+// The projections of a short prompt's rows on bf16 MFMA (rowgemm.hip), t <=
 // kRowGemmMax rows of fp32 activations: blocks of 32, inputs a multiple of
 // 128 wide.
 constexpr int kRowGemmMax = 128;

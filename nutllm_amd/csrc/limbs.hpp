@@ -1,6 +1,5 @@
 // limbs.hpp — fp32 activations as two f16 limbs and quantisation codes as
-// exact f16, the operands of the prompt GEMMs' f16 MFMA (prefill.hip,
-// rowgemm.hip).
+// exact f16, the operands of the batched prefill's f16 MFMA (prefill.hip).
 #pragma once
 
 #include "device.hpp"

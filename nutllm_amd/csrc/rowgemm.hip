@@ -4,17 +4,17 @@
 // Up to kRowGemmMax rows a layer's weights are read once, and what counts is
 // that the whole chip has its loads in flight (TinyLlama INT4, a layer of 20
 // tokens: 104 us on the step kernels, which dot every row once a token, 141
-// in the batched GEMM's 64 x 128 tiles, 70 here; 16 tokens 88 -> 47): 16 TJ outputs per workgroup,
-// its WK waves sharing k, so that a 2,048-wide matrix is 64 to 128
-// workgroups of 8 or 16 waves. The numbers are those of the batched GEMM
-// (prefill.hip): codes exact in f16, activations as two f16 limbs (split
-// here, from fp32 rows, so RMSNorm needs no pass of its own), products on
-// v_mfma_f32_16x16x32_f16, whose K = 32 is one quant block, the block's
-// scale applied in fp32. The rows are not normalised yet when they are split
-// (a hidden value is often a few hundredths), so the low limb is kept 2^11
-// times its size: as it stands it would fall among f16's subnormals and lose
-// bits (error against 64 bits of 100 tokens through 12 layers 3.5e-6, so
-// 9.6e-7).
+// in the batched GEMM's 64 x 128 tiles, 70 here; 16 tokens 88 -> 47): 16 TJ
+// outputs per workgroup, its WK waves sharing k, so that a 2,048-wide matrix
+// is 64 to 128 workgroups of 8 or 16 waves. Codes are
+// exact in bf16 and an fp32 activation is the sum of three bf16 limbs
+// without a remainder (8 bits each, fp32's own exponent range, so rows that
+// are not normalised yet may be of any size and RMSNorm needs no pass of its
+// own); products on v_mfma_f32_16x16x32_bf16, whose K = 32 is one quant
+// block, the block's scale applied in fp32. Two f16 limbs, as the batched
+// GEMM has them for its normalised rows, are one product less but lose small
+// rows to f16's subnormals (100 tokens through 12 layers: error 3.5e-6; so,
+// 8 to 60 tokens, 1.0e-6 to 1.6e-6) and large ones to its range.
 //
 // Weights go from memory to registers: lane (li, g) (li = lane % 16, g =
 // lane / 16) loads 16 bytes of output row TJ li + j, 64 consecutive bytes a
@@ -25,7 +25,6 @@
 // Activations go through a few KB of LDS of the wave's own, as in
 // gemm_f32.hpp, whose reduction over the waves and whose epilogues this
 // shares.
-#include "limbs.hpp"
 #include "kernels.hpp"
 #include "project.hpp"
 #include "runtime.hpp"
@@ -102,6 +101,43 @@ __device__ __forceinline__ void spread_codes(const Codes<QT> &in, uint2 (&out)[4
             out[2 * h + 1] = make_uint2(b0, b1);
         }
     }
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// The top halves of two fp32 values as two bf16 (a in the low half).
+__device__ __forceinline__ uint32_t top_halves(float a, float b)
+{
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+
+// Eight codes (INT8: 8 bytes, INT4: 4, even k in the low nibble) as bf16:
+// whole numbers of at most 8 bits, whose fp32 form ends in zeros.
+template <int QT> __device__ __forceinline__ bf16x8 codes_bf16(uint2 raw)
+{
+    uint32_t out[4];
+    if constexpr (QT == 1) {
+        const uint32_t t = raw.x ^ 0x88888888u;
+        const uint32_t lo = opaque(t & 0x0f0f0f0fu), hi = opaque((t >> 4) & 0x0f0f0f0fu);
+        out[0] = top_halves(ubyte0(lo) - 8.0f, ubyte0(hi) - 8.0f);
+        out[1] = top_halves(ubyte1(lo) - 8.0f, ubyte1(hi) - 8.0f);
+        out[2] = top_halves(ubyte2(lo) - 8.0f, ubyte2(hi) - 8.0f);
+        out[3] = top_halves(ubyte3(lo) - 8.0f, ubyte3(hi) - 8.0f);
+    } else {
+        const uint32_t w[2] = {raw.x ^ 0x80808080u, raw.y ^ 0x80808080u};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            out[2 * h] = top_halves(ubyte0(w[h]) - 128.0f, ubyte1(w[h]) - 128.0f);
+            out[2 * h + 1] = top_halves(ubyte2(w[h]) - 128.0f, ubyte3(w[h]) - 128.0f);
+        }
+    }
+    return __builtin_bit_cast(bf16x8, make_uint4(out[0], out[1], out[2], out[3]));
+}
+
+// v without its low 16 bits: the bf16 limb of v, as fp32.
+__device__ __forceinline__ float top_limb(float v)
+{
+    return __uint_as_float(__float_as_uint(v) & 0xffff0000u);
 }
 
 template <int QT, int TI, int TJ, int WK, int EPI>
@@ -200,11 +236,11 @@ __global__ __launch_bounds__(64 * WK) void rowgemm_kernel(RowGemm f)
             if (b < 2 || more)
                 load_x(b & 1, uint32_t(c) * kRun + 32 * (b + 2));
             __builtin_amdgcn_wave_barrier(); // a wave's LDS accesses keep their order
-            half8 w[TJ];
+            bf16x8 w[TJ];
             float s[TJ];
 #pragma unroll
             for (int j = 0; j < TJ; j++) {
-                w[j] = codes8<QT>(codes[j][b]);
+                w[j] = codes_bf16<QT>(codes[j][b]);
                 const uint32_t pair = b < 2 ? cur[j].scales.x : cur[j].scales.y;
                 s[j] = half_bits_to_float(uint16_t(b & 1 ? pair >> 16 : pair));
             }
@@ -212,26 +248,36 @@ __global__ __launch_bounds__(64 * WK) void rowgemm_kernel(RowGemm f)
             for (int i = 0; i < TI; i++) {
                 const float4 u = *reinterpret_cast<const float4 *>(get + 16 * i * kChunkLd);
                 const float4 v = *reinterpret_cast<const float4 *>(get + 16 * i * kChunkLd + 4);
-                const float e[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-                half8 hi, lo;
+                float e[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+                bf16x8 limb[3];
 #pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    const _Float16 h = (_Float16)e[q];
-                    hi[q] = h;
-                    lo[q] = (_Float16)((e[q] - (float)h) * 2048.0f);
-                }
-#pragma unroll
-                for (int j = 0; j < TJ; j++) {
-                    const floatx4 zero = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-                    const floatx4 d =
-                        __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, w[j], zero, 0, 0, 0);
-                    const floatx4 e2 =
-                        __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, w[j], zero, 0, 0, 0);
+                for (int l = 0; l < 3; l++) {
+                    uint32_t packed[4];
 #pragma unroll
                     for (int q = 0; q < 4; q++)
-                        acc[0][i][j][q] =
-                            fmaf(s[j], fmaf(e2[q], 0x1p-11f, d[q]), acc[0][i][j][q]);
+                        packed[q] = top_halves(e[2 * q], e[2 * q + 1]);
+                    limb[l] = __builtin_bit_cast(
+                        bf16x8, make_uint4(packed[0], packed[1], packed[2], packed[3]));
+                    if (l < 2) {
+#pragma unroll
+                        for (int q = 0; q < 8; q++)
+                            e[q] -= top_limb(e[q]);
+                    }
                 }
+                // the small limbs first
+                floatx4 d[TJ];
+#pragma unroll
+                for (int l = 2; l >= 0; l--)
+#pragma unroll
+                    for (int j = 0; j < TJ; j++)
+                        d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            limb[l], w[j],
+                            l == 2 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : d[j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < TJ; j++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        acc[0][i][j][q] = fmaf(s[j], d[j][q], acc[0][i][j][q]);
             }
             __builtin_amdgcn_wave_barrier();
             // without this and the one on sq the compiler keeps several

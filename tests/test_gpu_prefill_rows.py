@@ -46,3 +46,24 @@ def test_row_tiles_match_steps(gpu, model, tokens):
     finally:
         dev.set_path(0)
         rows.close(), steps.close()
+
+
+@pytest.mark.parametrize("scale", [1e-5, 1.0, 1e8])
+@pytest.mark.parametrize("qtype", [0, 1], ids=["int8", "int4"])
+def test_row_tiles_take_rows_of_any_size(gpu, qtype, scale):
+    """Hidden rows far below f16's smallest and far above its largest value:
+    the tiles split them before they are normalised."""
+    m = W.build("step_gqa4", qtype, 31, max_seq=64, norm_seed=5)
+    m.embeddings = (m.embeddings * np.float32(scale)).astype(np.float32)
+    dev = m.to_device()
+    rows, steps = gpu.KVCache(m.config), gpu.KVCache(m.config)
+    try:
+        ids = gpu.synth_tokens(9, m.config.vocab_size, 20).astype(np.int32)
+        got = dev.prefill(rows, ids)
+        dev.set_path(1)
+        want = dev.prefill(steps, ids)
+        assert np.all(np.isfinite(want)) and rel(got, want) <= 5e-6
+        for a, b in zip(rows.read_positions(0, 20), steps.read_positions(0, 20)):
+            assert rel(a, b) <= 5e-6
+    finally:
+        rows.close(), steps.close(), dev.close()

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
     __shared__ __attribute__((aligned(16))) float lds[kStage > kRed ? kStage : kRed];
     __shared__ float squares[NORM ? WK : 1][16 * TI];
     int tm, tn;
-    if (!gemm_f32_tile(f.tiles_m, f.tiles_n, tm, tn))
+    if (!gemm_f32_tile(f.tiles_m, f.tiles_n, blockIdx.x, tm, tn))
         return; // workgroup-uniform
     int seg = 0;
     if (EPI == kQkv)

@@ -13,10 +13,12 @@ template <int TI, int TJ, int WK, int NA, int D>
 void launch_tile(const float *a, const float *b, float *c, int m, int k, int n,
                  hipStream_t stream)
 {
-    const int tiles_m = (m + 16 * TI - 1) / (16 * TI), tiles_n = (n + 16 * TJ - 1) / (16 * TJ);
-    hipLaunchKernelGGL((matmul_f32_wave<TI, TJ, WK, NA, D>),
-                       dim3(gemm_f32_grid(tiles_m, tiles_n)), dim3(64 * WK), 0, stream, a, b, c,
-                       m, k, n, tiles_m, tiles_n);
+    const int tiles_m = (m - 1) / (16 * TI) + 1, tiles_n = (n - 1) / (16 * TJ) + 1;
+    // one dimension of a grid holds less than 2^32 threads
+    const unsigned count = gemm_f32_grid(tiles_m, tiles_n), row = 1u << 22;
+    const dim3 grid = count <= row ? dim3(count) : dim3(row, (count + row - 1) / row);
+    hipLaunchKernelGGL((matmul_f32_wave<TI, TJ, WK, NA, D>), grid, dim3(64 * WK), 0, stream, a, b,
+                       c, m, k, n, tiles_m, tiles_n);
 }
 
 } // namespace

@@ -290,12 +290,14 @@ __device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NS][TI][TJ], fl
 // Tile of this workgroup: workgroups go to the 8 XCDs round-robin, each XCD
 // takes a contiguous run of the tiles, and the run goes through blocks of
 // eight tile rows, so that the operands of the tiles an XCD has in flight
-// share its L2. False for the grid's padding (gemm_f32_grid).
-__device__ __forceinline__ bool gemm_f32_tile(int tiles_m, int tiles_n, int &tm, int &tn)
+// share its L2. id: the workgroup's place in the grid. False for the grid's
+// padding (gemm_f32_grid).
+__device__ __forceinline__ bool gemm_f32_tile(int tiles_m, int tiles_n, unsigned id, int &tm,
+                                              int &tn)
 {
     const int tiles = tiles_m * tiles_n, per = (tiles + 7) / 8;
-    const int t = int(blockIdx.x & 7) * per + int(blockIdx.x >> 3);
-    if (int(blockIdx.x >> 3) >= per || t >= tiles)
+    const int t = int(id & 7) * per + int(id >> 3);
+    if (int(id >> 3) >= per || t >= tiles)
         return false;
     const int group = t / (8 * tiles_n), in = t - group * 8 * tiles_n;
     const int rows = min(8, tiles_m - 8 * group);
@@ -364,16 +366,19 @@ __global__ __launch_bounds__(64 * WK) void matmul_f32_wave(
     constexpr int kRed = WK * TJ * 256;
     __shared__ __attribute__((aligned(16))) float lds[kStage > kRed ? kStage : kRed];
     int tm, tn;
-    if (!gemm_f32_tile(tiles_m, tiles_n, tm, tn))
+    if (!gemm_f32_tile(tiles_m, tiles_n, blockIdx.y * gridDim.x + blockIdx.x, tm, tn))
         return; // workgroup-uniform
     const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int row0 = tm * 16 * TI, col = tn * 16 * TJ + TJ * li;
-    const int first = min(col, n - TJ); // n >= TJ
+    // rows and columns of the tile counted from its first: m and n may be as
+    // large as an int holds
+    const int row0 = tm * 16 * TI, rows = m - row0;
+    const int col0 = tn * 16 * TJ, off = TJ * li, cols = n - col0;
+    const int first = col0 + min(off, cols - TJ); // n >= TJ
     const float *pa[2 * TI];
 #pragma unroll
     for (int t = 0; t < 2 * TI; t++)
-        pa[t] = a + size_t(min(row0 + 8 * t + (lane >> 3), m - 1)) * k + 4 * (lane & 7);
+        pa[t] = a + size_t(row0 + min(8 * t + (lane >> 3), rows - 1)) * k + 4 * (lane & 7);
     const float *pb[1] = {b + size_t(8 * g) * n + first};
     floatx4 acc[gemm_f32_accs(NA)][TI][TJ];
     float sq[2 * TI] = {};
@@ -387,16 +392,16 @@ __global__ __launch_bounds__(64 * WK) void matmul_f32_wave(
     gemm_f32_reduce<TI, TJ, WK>(
         acc, lds, wave,
         [&](int i, int v, const float (&out)[TJ]) {
-            const int row = row0 + 16 * i + 4 * g + v;
-            if (row >= m || col >= n)
+            const int row = 16 * i + 4 * g + v;
+            if (row >= rows || off >= cols)
                 return;
-            float *dst = c + size_t(row) * n + first;
-            if (first == col) {
+            float *dst = c + size_t(row0 + row) * n + first;
+            if (first == col0 + off) {
                 store_u<TJ>(dst, out);
             } else {
 #pragma unroll
                 for (int j = 0; j < TJ; j++)
-                    if (first + j >= col)
+                    if (first + j >= col0 + off)
                         dst[j] = out[j];
             }
         });

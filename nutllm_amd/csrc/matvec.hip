@@ -361,7 +361,10 @@ void launch_matvec_q(const QMat &m, const float *x, float *y,
     // (measured per shape with rocprofv3)
     const bool staged = m.type == 1 ? staged_x_bytes<1>(m.cols) <= 65536
                                     : m.rows >= 4096 && staged_x_bytes<0>(m.cols) <= 65536;
-    if (fast_layout(m) && staged) {
+    // these kernels have a workgroup for every few rows, and a grid holds less
+    // than 2^32 threads (32 a row); more rows go through in a loop
+    const bool loop = m.rows > 1 << 26;
+    if (fast_layout(m) && !loop && staged) {
         // two rows per wave, one where that leaves fewer than 256 workgroups
         if (m.rows >= 2048)
             m.type == 1 ? launch_staged<1, 2>(m, x, y, stream)
@@ -369,7 +372,7 @@ void launch_matvec_q(const QMat &m, const float *x, float *y,
         else
             m.type == 1 ? launch_staged<1, 1>(m, x, y, stream)
                         : launch_staged<0, 1>(m, x, y, stream);
-    } else if (fast_layout(m)) {
+    } else if (fast_layout(m) && !loop) {
         // rows per wave: enough waves to fill 256 CUs, as many rows in
         // flight per wave as that allows
         const int r = m.rows >= 4096 ? 4 : m.rows >= 1024 ? 2 : 1;
@@ -381,7 +384,7 @@ void launch_matvec_q(const QMat &m, const float *x, float *y,
             r == 4 ? launch_fast<0, 4>(m, x, y, stream)
                    : r == 2 ? launch_fast<0, 2>(m, x, y, stream)
                             : launch_fast<0, 1>(m, x, y, stream);
-    } else if (m.block_size >= 16 && (m.block_size & (m.block_size - 1)) == 0 &&
+    } else if (!loop && m.block_size >= 16 && (m.block_size & (m.block_size - 1)) == 0 &&
                ragged_lds_bytes(m.cols) <= 65536) {
         const int log_block = __builtin_ctz(unsigned(m.block_size));
         const int per = kRaggedRows * kRaggedThreads / kWave;

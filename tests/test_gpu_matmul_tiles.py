@@ -42,3 +42,12 @@ def test_matmul_non_finite_rows_stay_apart(gpu):
     assert np.all(np.isnan(c[36]))
     assert not np.any(np.isfinite(c[:, 50]))
     assert np.all(np.isfinite(c[:36, :50]))
+
+
+def test_matmul_rows_past_one_grid_dimension(gpu):
+    """More 16-row tiles than one dimension of a grid has workgroups (2^32
+    threads): products of one term each, which are exact."""
+    m = 140_000_000
+    a = np.arange(m, dtype=np.float32)
+    c = gpu.matmul_f32(a.reshape(m, 1), np.full((1, 1), 0.5, np.float32))
+    assert np.array_equal(c.ravel(), 0.5 * a)

@@ -84,3 +84,14 @@ def test_decode_step_other_blocks(gpu, qtype, block):
             assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
     finally:
         ca.close(), cb.close(), a.close(), b.close()
+
+
+def test_matvec_rows_past_one_grid(gpu):
+    """More rows than a grid of a workgroup per 16 rows covers (2^32 threads):
+    codes times scales of one, which are exact."""
+    rows = 140_000_000
+    data = (np.arange(rows) % 251 - 125).astype(np.int8)
+    scales = np.full((rows + 31) // 32, 0x3c00, np.uint16)
+    y = gpu.matvec_quantized(data.view(np.uint8), scales, rows, 1, 0,
+                             np.full(1, 0.5, np.float32))
+    assert np.array_equal(y, np.float32(0.5) * data)

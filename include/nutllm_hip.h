@@ -104,6 +104,10 @@ int nut_free(void *d_ptr);
  * loaded, its own and nut_malloc's (no reference counterpart: a
  * diagnostic, for checking that nut_decode_noalloc allocates nothing). */
 int nut_device_allocations(unsigned long long *count);
+/* Test hook (no reference counterpart): of the calling thread's next device
+ * allocations by this library, `skip` succeed and `count` then fail as if the
+ * device had no memory left; count = 0 takes it back. */
+int nut_fail_allocations(unsigned skip, unsigned count);
 int nut_memcpy_h2d(void *d_dst, const void *src, size_t bytes);
 int nut_memcpy_d2h(void *dst, const void *d_src, size_t bytes);
 /* Device-to-device copy (synchronous); also the known-size copy that

@@ -105,6 +105,7 @@ _SIGS = {
     "nut_malloc": (C.c_int, [_P, _SZ]),
     "nut_free": (C.c_int, [_P]),
     "nut_device_allocations": (C.c_int, [_P]),
+    "nut_fail_allocations": (C.c_int, [C.c_uint, C.c_uint]),
     "nut_memcpy_h2d": (C.c_int, [_P, _P, _SZ]),
     "nut_memcpy_d2h": (C.c_int, [_P, _P, _SZ]),
     "nut_memcpy_d2d": (C.c_int, [_P, _P, _SZ]),
@@ -245,6 +246,12 @@ def device_allocations():
     n = C.c_ulonglong(0)
     check(lib().nut_device_allocations(C.byref(n)))
     return n.value
+
+
+def fail_allocations(skip, count):
+    """Test hook: of this thread's next device allocations `skip` succeed and
+    `count` then fail as if the device had no memory left."""
+    check(lib().nut_fail_allocations(skip, count))
 
 
 def device_count():

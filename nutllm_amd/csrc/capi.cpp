@@ -75,6 +75,11 @@ int nut_malloc(void **d_ptr, size_t bytes)
     });
 }
 
+int nut_fail_allocations(unsigned skip, unsigned count)
+{
+    return nut::guarded([&]() { nut::fail_allocations(skip, count); });
+}
+
 int nut_device_allocations(unsigned long long *count)
 {
     return nut::guarded([&]() {

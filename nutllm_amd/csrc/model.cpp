@@ -172,7 +172,7 @@ void prefill_steps(nut_model &m, nut_kvcache &kv, size_t count)
 {
     const DecodeShape &s = m.shape;
     prepare_fast_steps(m);
-    if (m.mt_hidden.get() == nullptr) {
+    if (m.mt_act.get() == nullptr) { // the last: all are there
         m.mt_hidden.allocate(size_t(kStepTokensMax) * s.dim * sizeof(float));
         m.mt_query.allocate(size_t(kStepTokensMax) * s.dim * sizeof(float));
         m.mt_context.allocate(size_t(kStepTokensMax) * s.dim * sizeof(float));
@@ -250,7 +250,7 @@ bool use_row_gemm(const nut_model &m, size_t count)
 void prefill_rows(nut_model &m, nut_kvcache &kv, size_t count)
 {
     const DecodeShape &s = m.shape;
-    if (m.rg_hidden.get() == nullptr) {
+    if (m.rg_act.get() == nullptr) {
         m.rg_hidden.allocate(size_t(kRowGemmMax) * s.dim * sizeof(float));
         m.rg_query.allocate(size_t(kRowGemmMax) * s.dim * sizeof(float));
         m.rg_context.allocate(size_t(kRowGemmMax) * s.dim * sizeof(float));
@@ -327,7 +327,7 @@ void prefill_batch(nut_model &m, nut_kvcache &kv, size_t count)
 {
     const nut_config &c = m.config;
     const DecodeShape &s = m.shape;
-    if (m.pf_h.get() == nullptr) {
+    if (m.pf_kv.get() == nullptr) {
         const size_t rows = c.max_seq;
         m.pf_h.allocate(rows * c.dim * sizeof(float));
         m.pf_x.allocate(rows * c.dim * sizeof(float));
@@ -628,7 +628,7 @@ void prepare_screen(nut_model &m, const uint8_t *&codes, const uint16_t *&scales
     if ((vocab + kTokenGrid - 1) / kTokenGrid > kScreenRowsMax || dim % 32 != 0)
         return;
     if (!m.screen_ready) {
-        if (m.classifier8.get() == nullptr) {
+        if (m.classifier8_scales.get() == nullptr) {
             m.classifier8.allocate(size_t(vocab) * dim);
             m.classifier8_scales.allocate(size_t(vocab) * (dim / 32) * sizeof(uint16_t));
         }
@@ -642,11 +642,12 @@ void prepare_screen(nut_model &m, const uint8_t *&codes, const uint16_t *&scales
 
 void prepare_token_kernel(nut_model &m)
 {
-    if (m.exchange.get() == nullptr) {
+    if (m.token_error.get() == nullptr) {
         const size_t entries = token_exchange_entries(m.shape);
         m.exchange.allocate(entries * sizeof(uint64_t));
         hip_check(hipMemset(m.exchange.get(), 0, entries * sizeof(uint64_t)), "hipMemset");
         m.token_error.allocate(sizeof(int));
+        launch_set_int(m.token_error.as<int>(), 0, m.stream);
     }
 }
 

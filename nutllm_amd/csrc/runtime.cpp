@@ -65,15 +65,48 @@ unsigned long long device_allocations() { return g_allocations.load(); }
 
 void count_device_allocation() { g_allocations.fetch_add(1); }
 
-void DeviceBuffer::allocate(size_t bytes)
+namespace {
+thread_local unsigned g_skip_allocations = 0, g_fail_allocations = 0;
+
+bool injected_failure()
+{
+    if (g_fail_allocations == 0)
+        return false;
+    if (g_skip_allocations > 0) {
+        g_skip_allocations--;
+        return false;
+    }
+    g_fail_allocations--;
+    return true;
+}
+} // namespace
+
+void fail_allocations(unsigned skip, unsigned count)
+{
+    g_skip_allocations = skip;
+    g_fail_allocations = count;
+}
+
+hipError_t DeviceBuffer::replace(size_t bytes)
 {
     release();
     if (bytes == 0)
         bytes = 1;
-    hip_check(hipMalloc(&ptr_, bytes), "hipMalloc");
+    void *p = nullptr;
+    const hipError_t error = injected_failure() ? hipErrorOutOfMemory : hipMalloc(&p, bytes);
+    if (error != hipSuccess) {
+        (void)hipGetLastError(); // not the next launch's error
+        return error;
+    }
     count_device_allocation();
+    ptr_ = p;
     bytes_ = bytes;
+    return hipSuccess;
 }
+
+void DeviceBuffer::allocate(size_t bytes) { hip_check(replace(bytes), "hipMalloc"); }
+
+bool DeviceBuffer::try_allocate(size_t bytes) { return replace(bytes) == hipSuccess; }
 
 void DeviceBuffer::release()
 {

@@ -29,6 +29,9 @@ void ensure_device();
 // hipMalloc it issues: DeviceBuffer::allocate and nut_malloc).
 unsigned long long device_allocations();
 void count_device_allocation();
+// Test hook: of this thread's next DeviceBuffer allocations `skip` succeed and
+// `count` then fail as if the device had no memory left.
+void fail_allocations(unsigned skip, unsigned count);
 
 // RAII device allocation.
 class DeviceBuffer {
@@ -44,13 +47,18 @@ public:
         other.ptr_ = nullptr;
         other.bytes_ = 0;
     }
+    // Raises NUT_EDEVICE, and stays empty, when there is no memory left.
     void allocate(size_t bytes);
+    // The same for callers with another way to go on: false instead.
+    bool try_allocate(size_t bytes);
     void release();
     template <typename T> T *as() const { return static_cast<T *>(ptr_); }
     void *get() const { return ptr_; }
     size_t bytes() const { return bytes_; }
 
 private:
+    hipError_t replace(size_t bytes);
+
     void *ptr_ = nullptr;
     size_t bytes_ = 0;
 };

@@ -386,10 +386,12 @@ void check_fready(const nut_fmodel &m)
 }
 
 // One layer for t rows at positions first .. first + t - 1; `attend` puts
-// the rows' context into ctx from q and the layer's cache. parts: room for
-// kFRuns - 1 products of 16 rows, or null.
-template <class Attend>
-void launch_layer(const DecodeShape &s, const float *const (&w)[7], const float *attention_norm,
+// the rows' context into ctx from q and the layer's cache. weights(i, n, w):
+// w = the matrices i .. i + n - 1 (query, key, value, output, gate, up, down),
+// asked for before each launch in turn. parts: room for kFRuns - 1 products of
+// 16 rows, or null.
+template <class Weights, class Attend>
+void launch_layer(const DecodeShape &s, Weights &&weights, const float *attention_norm,
                   const float *ffn_norm, const float2 *rope, float *kc, float *vc, float *h,
                   float *q, float *ctx, float *act, float *parts, int t, int first,
                   hipStream_t stream, Attend &&attend)
@@ -404,10 +406,9 @@ void launch_layer(const DecodeShape &s, const float *const (&w)[7], const float 
         f.x = x;
         f.norm_w = norm;
         f.k = k;
-        for (int i = 0; i < count; i++) {
-            f.w[i] = w[w0 + i];
+        weights(w0, count, f.w);
+        for (int i = 0; i < count; i++)
             f.n[i] = i == 0 ? n0 : w0 == 0 ? kvd : n0;
-        }
         f.to.out = out;
     };
     gemm(h, attention_norm, s.dim, 0, 3, s.dim, q);
@@ -435,10 +436,11 @@ void enqueue_layers(nut_fmodel &m, nut_kvcache &kv, float *h, int t, int first, 
         const nut_fmodel::Layer &L = m.layers[l];
         float *kc = kv.keys.as<float>() + l * layer_elems;
         float *vc = kv.values.as<float>() + l * layer_elems;
-        const float *w[7];
-        for (int i = 0; i < 7; i++)
-            w[i] = L.w[i].as<float>();
-        launch_layer(s, w, L.attention_norm.as<float>(), L.ffn_norm.as<float>(),
+        const auto weights = [&](int i, int n, const float **w) {
+            for (int j = 0; j < n; j++)
+                w[j] = L.w[i + j].as<float>();
+        };
+        launch_layer(s, weights, L.attention_norm.as<float>(), L.ffn_norm.as<float>(),
                      m.rope.as<float2>(), kc, vc, h, q, ctx, act, m.parts.as<float>(), t, first,
                      m.stream, [&]() {
             if (t == 1 && m.split_attention) {
@@ -516,10 +518,10 @@ void launch_attention_f32(const DecodeShape &s, const float *q, const float *k_l
                        : launch_fattention<16>(s, q, k_layer, v_layer, ctx, t, stream);
 }
 
-size_t dense_layer_floats(const DecodeShape &s)
+size_t dense_group_floats(const DecodeShape &s)
 {
     const size_t d = s.dim, kvd = size_t(s.kv_heads) * s.head_dim, f = s.ffn_dim;
-    return 2 * d * d + 2 * d * kvd + 3 * d * f;
+    return std::max(d * d + 2 * d * kvd, 2 * d * f);
 }
 
 void launch_layer_dense(const DecodeShape &s, const LayerView &w, const float2 *rope,
@@ -527,16 +529,19 @@ void launch_layer_dense(const DecodeShape &s, const LayerView &w, const float2 *
                         hipStream_t stream)
 {
     const QMat *mats[7] = {&w.query, &w.key, &w.value, &w.output, &w.gate, &w.up, &w.down};
-    const float *at[7];
-    for (int i = 0; i < 7; i++) {
-        const QMat &m = *mats[i];
-        hipLaunchKernelGGL(dense_kernel, dim3((m.cols + 31) / 32, (m.rows + 31) / 32), dim3(256),
-                           0, stream, m, dense);
-        at[i] = dense;
-        dense += size_t(m.rows) * m.cols;
-    }
-    check_launch("prefill: dense weights");
-    launch_layer(s, at, w.attention_norm, w.ffn_norm, rope, k_layer, v_layer, b.hidden, b.query,
+    // the launch before has read its matrices when the next ones are written
+    const auto weights = [&](int i, int n, const float **at) {
+        float *to = dense;
+        for (int j = 0; j < n; j++) {
+            const QMat &m = *mats[i + j];
+            hipLaunchKernelGGL(dense_kernel, dim3((m.cols + 31) / 32, (m.rows + 31) / 32),
+                               dim3(256), 0, stream, m, to);
+            at[j] = to;
+            to += size_t(m.rows) * m.cols;
+        }
+        check_launch("prefill: dense weights");
+    };
+    launch_layer(s, weights, w.attention_norm, w.ffn_norm, rope, k_layer, v_layer, b.hidden, b.query,
                  b.context, b.act, nullptr, t, 0, stream, [&]() {
         launch_attention_f32(s, b.query, k_layer, v_layer, b.context, t, stream);
     });
@@ -643,6 +648,29 @@ void decode_token(nut_fmodel &m, nut_kvcache &kv, int token, float *hidden)
     kv.length += 1;
 }
 
+namespace {
+
+// Rows of every activation for the longest prompt so far: false where there is
+// no memory for them (token by token needs none).
+bool reserve_rows(nut_fmodel &m, size_t count)
+{
+    if (count <= m.rows_held)
+        return true;
+    m.rows_held = 0;
+    const size_t row = count * m.config.dim * sizeof(float);
+    if (m.pf_tokens.try_allocate(count * sizeof(int)) && m.pf_h.try_allocate(row) &&
+        m.pf_q.try_allocate(row) && m.pf_ctx.try_allocate(row) &&
+        m.pf_act.try_allocate(count * m.config.ffn_dim * sizeof(float))) {
+        m.rows_held = count;
+        return true;
+    }
+    for (DeviceBuffer *b : {&m.pf_tokens, &m.pf_h, &m.pf_q, &m.pf_ctx, &m.pf_act})
+        b->release();
+    return false;
+}
+
+} // namespace
+
 void prefill_tokens(nut_fmodel &m, nut_kvcache &kv, const int *tokens, size_t count,
                     float *rows)
 {
@@ -655,15 +683,12 @@ void prefill_tokens(nut_fmodel &m, nut_kvcache &kv, const int *tokens, size_t co
     for (size_t t = 0; t < count; t++)
         require(tokens[t] >= 0 && size_t(tokens[t]) < m.config.vocab_size, NUT_EOUTOFRANGE,
                 "kv cache: token id out of range");
-    if (count > m.rows_held) {
-        // rows of every activation for the longest prompt so far
-        m.rows_held = 0;
-        m.pf_tokens.allocate(count * sizeof(int));
-        m.pf_h.allocate(count * m.config.dim * sizeof(float));
-        m.pf_q.allocate(count * m.config.dim * sizeof(float));
-        m.pf_ctx.allocate(count * m.config.dim * sizeof(float));
-        m.pf_act.allocate(count * m.config.ffn_dim * sizeof(float));
-        m.rows_held = count;
+    if (!reserve_rows(m, count)) {
+        for (size_t t = 0; t < count; t++) {
+            float *row = rows == nullptr ? nullptr : rows + t * m.config.dim;
+            decode_token(m, kv, tokens[t], row);
+        }
+        return;
     }
     hip_check(hipMemcpyAsync(m.pf_tokens.get(), tokens, count * sizeof(int),
                              hipMemcpyHostToDevice, m.stream),

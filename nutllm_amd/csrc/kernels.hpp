@@ -155,9 +155,10 @@ void launch_layer_rows(const DecodeShape &s, const LayerView &w, const float2 *r
                        hipStream_t stream);
 
 // The same for any block layout (fmodel.hip), attention_f32_supported shapes
-// and any t: the layer's weights as fp32 in `dense` (dense_layer_floats(s)
-// floats, free again when the layer is done), then the fp32 path's launches.
-size_t dense_layer_floats(const DecodeShape &s);
+// and any t: the fp32 path's launches, the weights of each written out as fp32
+// to `dense` before it (dense_group_floats(s) floats: those of the widest
+// launch; free again when the layer is done).
+size_t dense_group_floats(const DecodeShape &s);
 void launch_layer_dense(const DecodeShape &s, const LayerView &w, const float2 *rope,
                         float *k_layer, float *v_layer, const RowBuffers &b, int t, float *dense,
                         hipStream_t stream);

@@ -270,8 +270,8 @@ void prefill_rows(nut_model &m, nut_kvcache &kv, size_t count)
 }
 
 // Prompts of two tokens and more whose layers have no step kernel (head sizes
-// of 16 and 32, widths that no 32-wide block divides, other block sizes): a
-// layer's weights are written out as fp32 once for the whole prompt, where
+// of 16 and 32, widths that no 32-wide block divides, other block sizes): each
+// launch's weights are written out as fp32 once for the whole prompt, where
 // the token-by-token way read and decoded them for every token (the tiny test
 // shape, 500 tokens: 42 ms of kernels, 84 ms with their launches).
 bool use_dense(const nut_model &m, size_t count)
@@ -279,20 +279,32 @@ bool use_dense(const nut_model &m, size_t count)
     return m.path == 0 && count >= 2 && attention_f32_supported(m.shape) && !fast_steps(m);
 }
 
+// Its workspace: false where there is no memory for it (the token-by-token
+// way needs none).
+bool reserve_dense(nut_model &m, size_t count)
+{
+    const DecodeShape &s = m.shape;
+    if (count <= m.dn_rows)
+        return true;
+    // rows for the longest prompt so far
+    m.dn_rows = 0;
+    const size_t row = count * s.dim * sizeof(float);
+    if ((m.dn_weights.get() != nullptr ||
+         m.dn_weights.try_allocate(dense_group_floats(s) * sizeof(float))) &&
+        m.dn_hidden.try_allocate(row) && m.dn_query.try_allocate(row) &&
+        m.dn_context.try_allocate(row) &&
+        m.dn_act.try_allocate(count * s.ffn_dim * sizeof(float))) {
+        m.dn_rows = count;
+        return true;
+    }
+    for (DeviceBuffer *b : {&m.dn_weights, &m.dn_hidden, &m.dn_query, &m.dn_context, &m.dn_act})
+        b->release();
+    return false;
+}
+
 void prefill_dense(nut_model &m, nut_kvcache &kv, size_t count)
 {
     const DecodeShape &s = m.shape;
-    if (m.dn_weights.get() == nullptr)
-        m.dn_weights.allocate(dense_layer_floats(s) * sizeof(float));
-    if (count > m.dn_rows) {
-        // for the longest prompt so far
-        m.dn_rows = 0;
-        m.dn_hidden.allocate(count * s.dim * sizeof(float));
-        m.dn_query.allocate(count * s.dim * sizeof(float));
-        m.dn_context.allocate(count * s.dim * sizeof(float));
-        m.dn_act.allocate(count * s.ffn_dim * sizeof(float));
-        m.dn_rows = count;
-    }
     const RowBuffers b{m.dn_hidden.as<float>(), m.dn_query.as<float>(),
                        m.dn_context.as<float>(), m.dn_act.as<float>()};
     launch_embed_rows(m.embeddings.as<float>(), m.prompt.as<int>(), b.hidden, int(count), s.dim,
@@ -845,7 +857,7 @@ void prefill(nut_model &m, nut_kvcache &kv, const int *tokens, size_t count,
             prefill_rows(m, kv, valid);
         } else if (use_prefill_gemm(m, valid)) {
             prefill_batch(m, kv, valid);
-        } else if (use_dense(m, valid)) {
+        } else if (use_dense(m, valid) && reserve_dense(m, valid)) {
             prefill_dense(m, kv, valid);
         } else if (m.path != 2 && valid > 1 && fast_steps(m)) {
             prefill_steps(m, kv, valid);

@@ -72,7 +72,7 @@ struct nut_model {
     nut::DeviceBuffer mt_hidden, mt_query, mt_context, mt_act;
     // Short prompts on the row tiles: kRowGemmMax rows each.
     nut::DeviceBuffer rg_hidden, rg_query, rg_context, rg_act;
-    // Prompts of layouts without a step kernel: a layer's weights as fp32, and
+    // Prompts of layouts without a step kernel: a launch's weights as fp32, and
     // dn_rows rows of activations.
     nut::DeviceBuffer dn_weights, dn_hidden, dn_query, dn_context, dn_act;
     size_t dn_rows = 0;

@@ -67,7 +67,10 @@ __device__ __forceinline__ void two_rows(const QMat &m, int row,
                                          float (&out)[2])
 {
     if (fast_layout(m)) {
-        qrows_fast<2>(m, row, xs, xsum, out);
+        if (m.block_size == 32)
+            qrows_fast<2, false>(m, row, xs, xsum, out);
+        else
+            qrows_fast<2, true>(m, row, xs, xsum, out);
     } else {
         out[0] = qrow_generic(m, row, xs);
         out[1] = row + 1 < m.rows ? qrow_generic(m, row + 1, xs) : 0.0f;

@@ -154,6 +154,9 @@ __device__ __forceinline__ float ubyte1(uint32_t v) { return float((v >> 8) & 0x
 __device__ __forceinline__ float ubyte2(uint32_t v) { return float((v >> 16) & 0xffu); }
 __device__ __forceinline__ float ubyte3(uint32_t v) { return float(v >> 24); }
 
+// Byte b as a signed value (v_cvt_f32_i32 reads it in place).
+__device__ __forceinline__ float sbyte(uint32_t v, int b) { return float(int8_t(v >> (8 * b))); }
+
 // Keeps v opaque to known-bits folding, so byte conversions of a masked
 // word stay single v_cvt_f32_ubyte{0..3} instead of a bit-field extract
 // per nibble. Emits no instruction.
@@ -167,50 +170,84 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v)
 // Byte b of word j holds weights 8j+2b (low nibble) and 8j+2b+1 (high).
 // High nibbles are converted in place (16 u) and their accumulator scaled
 // by 1/16 once; power-of-two scaling commutes with rounding, so the result
-// equals accumulating u x. SIGNED: sum_k q_k x[k] instead, the offset taken
-// off every code (one more operation a weight, and partial sums without the
-// offset's share, whose rounding is most of the other form's error).
-template <bool SIGNED = false>
+// equals accumulating u x.
 __device__ __forceinline__ float dot_int4_chunk(uint4 w, const float *x)
 {
     const uint32_t words[4] = {w.x, w.y, w.z, w.w};
-    constexpr float kLo = SIGNED ? 8.0f : 0.0f, kHi = SIGNED ? 128.0f : 0.0f;
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const uint32_t lo = opaque((words[j] ^ 0x88888888u) & 0x0f0f0f0fu);
         const uint32_t hi = opaque((words[j] ^ 0x88888888u) & 0xf0f0f0f0u);
         const float *xs = x + 8 * j;
-        a0 = fmaf(ubyte0(lo) - kLo, xs[0], a0);
-        a1 = fmaf(ubyte0(hi) - kHi, xs[1], a1);
-        a0 = fmaf(ubyte1(lo) - kLo, xs[2], a0);
-        a1 = fmaf(ubyte1(hi) - kHi, xs[3], a1);
-        a0 = fmaf(ubyte2(lo) - kLo, xs[4], a0);
-        a1 = fmaf(ubyte2(hi) - kHi, xs[5], a1);
-        a0 = fmaf(ubyte3(lo) - kLo, xs[6], a0);
-        a1 = fmaf(ubyte3(hi) - kHi, xs[7], a1);
+        a0 = fmaf(ubyte0(lo), xs[0], a0);
+        a1 = fmaf(ubyte0(hi), xs[1], a1);
+        a0 = fmaf(ubyte1(lo), xs[2], a0);
+        a1 = fmaf(ubyte1(hi), xs[3], a1);
+        a0 = fmaf(ubyte2(lo), xs[4], a0);
+        a1 = fmaf(ubyte2(hi), xs[5], a1);
+        a0 = fmaf(ubyte3(lo), xs[6], a0);
+        a1 = fmaf(ubyte3(hi), xs[7], a1);
     }
     return fmaf(a1, 0.0625f, a0);
 }
 
-// sum_k u_k x[k] over one INT8 chunk (16 weights, offset-binary codes), or
-// sum_k q_k x[k] (SIGNED).
-template <bool SIGNED = false>
+// sum_k u_k x[k] over one INT8 chunk (16 weights, offset-binary codes).
 __device__ __forceinline__ float dot_int8_chunk(uint4 w, const float *x)
 {
     const uint32_t words[4] = {w.x ^ 0x80808080u, w.y ^ 0x80808080u,
                                w.z ^ 0x80808080u, w.w ^ 0x80808080u};
-    constexpr float kOff = SIGNED ? 128.0f : 0.0f;
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const float *xs = x + 4 * j;
-        a0 = fmaf(ubyte0(words[j]) - kOff, xs[0], a0);
-        a1 = fmaf(ubyte1(words[j]) - kOff, xs[1], a1);
-        a0 = fmaf(ubyte2(words[j]) - kOff, xs[2], a0);
-        a1 = fmaf(ubyte3(words[j]) - kOff, xs[3], a1);
+        a0 = fmaf(ubyte0(words[j]), xs[0], a0);
+        a1 = fmaf(ubyte1(words[j]), xs[1], a1);
+        a0 = fmaf(ubyte2(words[j]), xs[2], a0);
+        a1 = fmaf(ubyte3(words[j]), xs[3], a1);
     }
     return a0 + a1;
+}
+
+// sum_k q_k s x[k] over one INT4 chunk, s its block's scale: q s is exact in
+// fp32 (4 and 11 bits), and the sum is a tree over chains of four, which errs
+// no more than a lane that adds one weight at a time does at any row length;
+// dot_int4_chunk's sum with the offset in it errs by about four times as much.
+// Codes are converted as bytes of 16 q, which is one operation a weight.
+__device__ __forceinline__ float dot_int4_scaled(uint4 w, const float *x, float s)
+{
+    const uint32_t words[4] = {w.x, w.y, w.z, w.w};
+    s *= 0.0625f;
+    float a[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t lo = opaque((words[j] << 4) & 0xf0f0f0f0u);
+        const uint32_t hi = opaque(words[j] & 0xf0f0f0f0u);
+        const float *xs = x + 8 * j;
+        float a0 = sbyte(lo, 0) * s * xs[0], a1 = sbyte(hi, 0) * s * xs[1];
+#pragma unroll
+        for (int b = 1; b < 4; b++) {
+            a0 = fmaf(sbyte(lo, b) * s, xs[2 * b], a0);
+            a1 = fmaf(sbyte(hi, b) * s, xs[2 * b + 1], a1);
+        }
+        a[j] = a0 + a1;
+    }
+    return (a[0] + a[1]) + (a[2] + a[3]);
+}
+
+// The same over one INT8 chunk (16 weights; q s has 8 and 11 bits).
+__device__ __forceinline__ float dot_int8_scaled(uint4 w, const float *x, float s)
+{
+    const uint32_t words[4] = {w.x, w.y, w.z, w.w};
+    float a[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        a[j] = sbyte(words[j], 0) * s * x[4 * j];
+#pragma unroll
+        for (int b = 1; b < 4; b++)
+            a[j] = fmaf(sbyte(words[j], b) * s, x[4 * j + b], a[j]);
+    }
+    return (a[0] + a[1]) + (a[2] + a[3]);
 }
 
 // A quantised matrix in HBM: reference layout, data verbatim.
@@ -261,8 +298,8 @@ __device__ __forceinline__ void stage_x(const float *x, float *xs,
 
 // Dot products of R consecutive fast-layout rows row0..row0+R-1 with the
 // staged x; rows past the end re-read the last row (callers drop them).
-// Every lane of the wave returns all R sums.
-template <int R>
+// Every lane of the wave returns all R sums. WB: blocks wider than 32.
+template <int R, bool WB>
 __device__ __forceinline__ void qrows_fast(const QMat &m, int row0,
                                            const float *xs,
                                            const float *xsum, float (&out)[R])
@@ -271,7 +308,7 @@ __device__ __forceinline__ void qrows_fast(const QMat &m, int row0,
     const bool int4 = m.type == 1;
     const int row_bytes = int4 ? m.cols / 2 : m.cols;
     const int chunks = row_bytes / 16;
-    const int shift = scale_shift(m);
+    const int shift = WB ? scale_shift(m) : 0;
     const int blocks_per_row = m.cols >> (shift + 5);
     const float bias = int4 ? 8.0f : 128.0f;
     float acc[R];
@@ -291,6 +328,12 @@ __device__ __forceinline__ void qrows_fast(const QMat &m, int row0,
                 m.scales[size_t(rr) * blocks_per_row + block]);
         }
         const float *xc = xs + c * (int4 ? 32 : 16);
+        if (WB) {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                acc[r] += int4 ? dot_int4_scaled(w[r], xc, s[r]) : dot_int8_scaled(w[r], xc, s[r]);
+            continue;
+        }
         const float xc_sum = xsum[c];
 #pragma unroll
         for (int r = 0; r < R; r++) {

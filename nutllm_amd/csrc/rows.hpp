@@ -137,14 +137,14 @@ __device__ __forceinline__ void rows_matvec(const uint8_t *const (&rp)[R],
             xc[4 * q + 3] = v.w;
         }
         if (WB) {
-            // wider blocks keep the error of a sum of q s x itself (5000 x
-            // 4096 INT4 at block 64: 7.7e-7 in offset binary, 1.1e-7 so)
+            // wider blocks keep the error of a sum of q s x itself, added a
+            // weight at a time (4096 x 64 INT4 at block 64: 7e-8, and 8.4e-8
+            // with the block's scale applied to the chunk's sum; 5000 x 4096:
+            // 9.4e-8, and 7.7e-7 in offset binary)
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float d =
-                    QT == 1 ? dot_int4_chunk<true>(w[r], xc) : dot_int8_chunk<true>(w[r], xc);
-                acc[r] = fmaf(s[r], d, acc[r]);
-            }
+            for (int r = 0; r < R; r++)
+                acc[r] += QT == 1 ? dot_int4_scaled(w[r], xc, s[r])
+                                  : dot_int8_scaled(w[r], xc, s[r]);
             return;
         }
         float xsum = 0.0f;

@@ -1,0 +1,94 @@
+"""Rounding errors of sums against float64: their size for the order in which
+each kernel adds, and that they are not one-sided.
+
+A sum of n terms that is formed in chains errs, relative to the sum's own size
+and over random terms, by U sqrt(A): U = 0.43 x 2^-24 is the root mean square
+of one fp32 rounding (uniform within half an ulp, mantissas spread evenly over
+their logarithm), and A the mean over all roundings of the variance that the
+partial sum rounded has, as a share of the whole's. A chain of c terms of n
+adds (c + 1) / 2 to A, each level of a tree 1, a rounded factor 1. The chains
+stated are those of a lane that adds one weight at a time, or of the matrix
+kernel with k over eight waves: what these calls were always summed as."""
+import numpy as np
+import pytest
+
+from nutllm_amd import workloads as W
+from test_gpu_matvec_ragged import dequantised
+
+pytestmark = pytest.mark.gpu
+
+U = 0.43 * 2.0 ** -24
+BOTH = pytest.mark.parametrize("qtype", [0, 1], ids=["int8", "int4"])
+
+
+def rel(got, want):
+    return np.linalg.norm(got - want) / np.linalg.norm(want)
+
+
+def lane_sum(n):
+    """One weight at a time over 64 lanes, then six levels of a tree."""
+    return (-(-n // 64) + 1) / 2 + 6
+
+
+def rms(x):
+    return x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-5)
+
+
+def value_rows(gpu, cfg, qtype, block, ids, path=0):
+    """The V rows that a one-layer model's prompt (one token: decode step)
+    leaves in the cache, and their float64 values."""
+    rng = np.random.default_rng(cfg.dim + block)
+    dim, ffn, kvd = cfg.dim, cfg.ffn_dim, cfg.kv_heads * cfg.head_dim
+    shapes = dict(query=(dim, dim), key=(kvd, dim), value=(kvd, dim), output=(dim, dim),
+                  gate=(ffn, dim), up=(ffn, dim), down=(dim, ffn))
+    emb = rng.standard_normal((cfg.vocab_size, dim)).astype(np.float32)
+    norm = (1 + 0.1 * rng.standard_normal(dim)).astype(np.float32)
+    mats = {}
+    for name, (r, c) in shapes.items():
+        w = (rng.standard_normal((r, c)) * c ** -0.5).astype(np.float32)
+        mats[name] = (*gpu.quantize(w, qtype, block), r, c, block)
+    m, cache = gpu.DeviceModel(cfg, qtype), gpu.KVCache(cfg)
+    try:
+        m.set_globals(emb, np.ones(dim, np.float32), emb)
+        m.set_layer(0, mats, norm, norm)
+        m.set_path(path)
+        if len(ids) == 1:
+            m.decode(cache, int(ids[0]))
+        else:
+            m.prefill(cache, np.asarray(ids, np.int32))
+        _, v = cache.read_positions(0, len(ids))
+        got = np.asarray(v[0], np.float64).transpose(1, 0, 2).reshape(len(ids), kvd)
+    finally:
+        cache.close(), m.close()
+    data, scales = mats["value"][:2]
+    w = dequantised(data, scales, kvd, dim, qtype, block)
+    return got, rms(emb[ids].astype(np.float64)) * norm @ w.T
+
+
+def one_layer(gpu, heads, kv_heads, head_dim, ffn, max_seq=160):
+    return gpu.Config(layers=1, heads=heads, dim=heads * head_dim, head_dim=head_dim, ffn_dim=ffn,
+                      vocab_size=300, kv_heads=kv_heads, max_seq=max_seq, eos_token=1)
+
+
+@BOTH
+@pytest.mark.parametrize("cols,block", [(64, 64), (256, 64), (512, 128)])
+def test_wide_blocks_err_as_a_lane_sum(gpu, qtype, cols, block):
+    """Blocks of 64 and wider on the row kernels: 8 % over the lane sum's error
+    (4,096 outputs settle it to 1 %)."""
+    rng = np.random.default_rng(cols)
+    rows = 4096
+    data, scales = gpu.quantize(rng.standard_normal((rows, cols)).astype(np.float32), qtype, block)
+    x = rng.standard_normal(cols).astype(np.float32)
+    y = gpu.matvec_quantized(data, scales, rows, cols, qtype, x, block)
+    want = dequantised(data, scales, rows, cols, qtype, block) @ x.astype(np.float64)
+    assert rel(y, want) <= 1.08 * U * np.sqrt(lane_sum(cols))
+
+
+@BOTH
+@pytest.mark.parametrize("block", [64, 128])
+def test_wide_blocks_err_as_a_lane_sum_in_general_steps(gpu, qtype, block):
+    """The general step kernels (head size 32) at blocks of 64 and wider: x is
+    scaled and weighted before (two roundings); 256 outputs settle the error
+    to 5 %, the bound is 25 % over it."""
+    got, want = value_rows(gpu, one_layer(gpu, 8, 8, 32, 512), qtype, block, [7])
+    assert rel(got, want) <= 1.25 * U * np.sqrt(lane_sum(256) + 2)

@@ -92,3 +92,15 @@ def test_wide_blocks_err_as_a_lane_sum_in_general_steps(gpu, qtype, block):
     to 5 %, the bound is 25 % over it."""
     got, want = value_rows(gpu, one_layer(gpu, 8, 8, 32, 512), qtype, block, [7])
     assert rel(got, want) <= 1.25 * U * np.sqrt(lane_sum(256) + 2)
+
+
+@BOTH
+@pytest.mark.parametrize("cols,block", [(33, 16), (100, 32), (255, 32), (500, 64)])
+def test_straddled_blocks_err_as_a_lane_sum(gpu, qtype, cols, block):
+    rng = np.random.default_rng(cols)
+    rows = 4096
+    data, scales = gpu.quantize(rng.standard_normal((rows, cols)).astype(np.float32), qtype, block)
+    x = rng.standard_normal(cols).astype(np.float32)
+    y = gpu.matvec_quantized(data, scales, rows, cols, qtype, x, block)
+    want = dequantised(data, scales, rows, cols, qtype, block) @ x.astype(np.float64)
+    assert rel(y, want) <= 1.08 * U * np.sqrt(lane_sum(cols))

@@ -31,11 +31,18 @@ void launch_matmul_f32(const float *a, const float *b, float *c, int m, int k,
     // tile and k gives every wave a chunk (33 x 4001 x 3333: 25.7 us against
     // 30.4 with four), four elsewhere.
     // Two accumulators per output keep a chain of additions as short as eight
-    // waves' (768^3: rel error 1.8e-7 against 2.5e-7 with one).
-    const bool deep = t.count <= 256 && k >= 8 * kChunk;
+    // waves' (768^3: rel error 1.8e-7 against 2.5e-7 with one). The 64 x 64
+    // tile has the registers for one: where it leaves CUs idle it has eight
+    // waves for that (960 x 2048 x 960: 2.9e-7 against 4.1e-7 with four, at 43
+    // and 41 us), or two accumulators where k has fewer than eight chunks.
+    const bool deep = k >= 8 * kChunk, few = size_t(m / 64) * (n / 64) < 256;
     switch (t.ti * 10 + t.tj) {
     case 44:
-        launch_tile<4, 4, 4, 1, 1>(a, b, c, m, k, n, stream);
+        if (few)
+            deep ? launch_tile<4, 4, 8, 1, 1>(a, b, c, m, k, n, stream)
+                 : launch_tile<4, 4, 4, 2, 1>(a, b, c, m, k, n, stream);
+        else
+            launch_tile<4, 4, 4, 1, 1>(a, b, c, m, k, n, stream);
         break;
     case 34:
         launch_tile<3, 4, 4, 2, 2>(a, b, c, m, k, n, stream);
@@ -47,14 +54,14 @@ void launch_matmul_f32(const float *a, const float *b, float *c, int m, int k,
         launch_tile<2, 4, 4, 2, 2>(a, b, c, m, k, n, stream);
         break;
     case 22:
-        deep ? launch_tile<2, 2, 8, 2, 1>(a, b, c, m, k, n, stream)
-             : launch_tile<2, 2, 4, 2, 1>(a, b, c, m, k, n, stream);
+        deep && t.count <= 256 ? launch_tile<2, 2, 8, 2, 1>(a, b, c, m, k, n, stream)
+                               : launch_tile<2, 2, 4, 2, 1>(a, b, c, m, k, n, stream);
         break;
     case 12:
         launch_tile<1, 2, 4, 2, 2>(a, b, c, m, k, n, stream);
         break;
     default:
-        launch_tile<1, 1, 8, 1, 2>(a, b, c, m, k, n, stream);
+        launch_tile<1, 1, 8, 2, 2>(a, b, c, m, k, n, stream);
     }
     check_launch("threaded matmul");
 }

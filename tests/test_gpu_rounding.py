@@ -104,3 +104,16 @@ def test_straddled_blocks_err_as_a_lane_sum(gpu, qtype, cols, block):
     y = gpu.matvec_quantized(data, scales, rows, cols, qtype, x, block)
     want = dequantised(data, scales, rows, cols, qtype, block) @ x.astype(np.float64)
     assert rel(y, want) <= 1.08 * U * np.sqrt(lane_sum(cols))
+
+
+@pytest.mark.parametrize("mkn", [(960, 2048, 960), (960, 256, 960), (960, 128, 960),
+                                 (32, 128, 32)])
+def test_matmul_errs_as_eight_waves(gpu, mkn):
+    """k in eight chains, three levels of a tree, where 64 x 64 tiles leave
+    CUs idle."""
+    m, k, n = mkn
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert rel(gpu.matmul_f32(a, b), want) <= 1.1 * U * np.sqrt((k / 8 + 1) / 2 + 3)

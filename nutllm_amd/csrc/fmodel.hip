@@ -46,7 +46,7 @@ struct FGemm {
     float *parts;
 };
 
-template <int TI, int TJ, int WK, int D, int EPI>
+template <int TI, int TJ, int WK, int D, int P, int EPI>
 __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
 {
     constexpr bool NORM = EPI != kAdd;
@@ -81,9 +81,9 @@ __global__ __launch_bounds__(64 * WK) void fgemm_kernel(FGemm f)
     bool tail;
     const int run = EPI == kAdd ? blockIdx.y : 0, runs = EPI == kAdd ? gridDim.y : 1;
     gemm_f32_share(k, run * WK + wave, runs * WK, c0, c1, tail);
-    gemm_f32_run<TI, TJ, NB, 0, D, NORM>(pa, pb, size_t(n),
-                                          NORM ? f.norm_w + 4 * (lane & 7) : nullptr, k, c0, c1,
-                                          tail, lds + wave * 16 * TI * kChunkLd, acc, sq);
+    gemm_f32_run<TI, TJ, NB, -P, D, NORM>(pa, pb, size_t(n),
+                                           NORM ? f.norm_w + 4 * (lane & 7) : nullptr, k, c0, c1,
+                                           tail, lds + wave * 16 * TI * kChunkLd, acc, sq);
     if (NORM) {
         // eight lanes hold a row's squares of this wave's share
 #pragma unroll
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void add_parts_kernel(float *h, const float *p
     h[i] = v;
 }
 
-template <int TI, int TJ, int WK, int D, int EPI>
+template <int TI, int TJ, int WK, int D, int P, int EPI>
 void launch_ftile(FGemm &f, hipStream_t stream, int runs = 1)
 {
     const int cols = 16 * TJ / (EPI == kSwiglu ? 2 : 1);
@@ -142,7 +142,7 @@ void launch_ftile(FGemm &f, hipStream_t stream, int runs = 1)
         f.tiles[s] = (f.n[s] + cols - 1) / cols;
         f.tiles_n += f.tiles[s];
     }
-    hipLaunchKernelGGL((fgemm_kernel<TI, TJ, WK, D, EPI>),
+    hipLaunchKernelGGL((fgemm_kernel<TI, TJ, WK, D, P, EPI>),
                        dim3(gemm_f32_grid(f.tiles_m, f.tiles_n), runs), dim3(64 * WK), 0, stream, f);
     check_launch("fp32 model: projection");
 }
@@ -155,6 +155,12 @@ constexpr int kFRuns = 4; // most runs of k
 // us (44 194, 34 187, 22 192, 14 202), of 64 22 49 (44 51, 24 59), of 20 24 31
 // (44 50, 22 41); W2 of 301 rows 34 87 (44 110, 22 98), of 150 24 62 (34 87,
 // 22 64), of 64 12 28 (22 37, 14 37); Q/K/V of 301 rows 14 38 (44 48, 24 47).
+// A chunk's sum is formed in four chains (2 x 2: two) where the tile has the
+// registers and the time for it, which is where narrow widths need it: their
+// sums have few chunks (width 256 block 64, 70 tokens: error 2.4e-7 with one
+// chain, 1.9e-7 so). More chains cost time: two at 14 and 24 made 301 tokens of
+// four layers 2.15 ms instead of 2.00, four at 22 64 rows of two 334 us instead
+// of 317, eight in a decode step's tiles two steps at 700 770 us instead of 680.
 // Up to 16 rows the weights' way from HBM is what
 // counts: sixteen waves share the k of a narrow tile, so that the whole chip
 // has its loads in flight at once.
@@ -173,17 +179,17 @@ template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
             const int tiles = (n + 31) / 32;
             const int runs = std::min(kFRuns, 256 / tiles);
             if (f.parts != nullptr && runs > 1 && f.k >= 4096) {
-                launch_ftile<1, 2, 8, 2, EPI>(f, stream, runs);
+                launch_ftile<1, 2, 8, 2, 4, EPI>(f, stream, runs);
                 hipLaunchKernelGGL(add_parts_kernel, dim3((f.m * n + 255) / 256), dim3(256), 0,
                                    stream, f.to.out, f.parts, runs - 1, f.m * n);
                 check_launch("fp32 model: sums");
                 return;
             }
-            n >= 4096 ? launch_ftile<1, 2, 16, 2, EPI>(f, stream)
-                      : launch_ftile<1, 1, 16, 3, EPI>(f, stream);
+            n >= 4096 ? launch_ftile<1, 2, 16, 2, 4, EPI>(f, stream)
+                      : launch_ftile<1, 1, 16, 3, 4, EPI>(f, stream);
         } else {
-            n >= 8192 ? launch_ftile<1, 4, 8, 1, EPI>(f, stream)
-                      : launch_ftile<1, 2, 16, 2, EPI>(f, stream);
+            n >= 8192 ? launch_ftile<1, 4, 8, 1, 4, EPI>(f, stream)
+                      : launch_ftile<1, 2, 16, 2, 4, EPI>(f, stream);
         }
         return;
     }
@@ -192,22 +198,22 @@ template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
     const GemmTile t = gemm_f32_pick(tiles, f.m, f.k, n);
     switch (t.ti * 10 + t.tj) {
     case 44:
-        launch_ftile<4, 4, 4, 1, EPI>(f, stream);
+        launch_ftile<4, 4, 4, 1, 1, EPI>(f, stream);
         break;
     case 34:
-        launch_ftile<3, 4, 4, 1, EPI>(f, stream);
+        launch_ftile<3, 4, 4, 1, 1, EPI>(f, stream);
         break;
     case 24:
-        launch_ftile<2, 4, 4, 2, EPI>(f, stream);
+        launch_ftile<2, 4, 4, 2, 1, EPI>(f, stream);
         break;
     case 22:
-        launch_ftile<2, 2, 4, 2, EPI>(f, stream);
+        launch_ftile<2, 2, 4, 2, 2, EPI>(f, stream);
         break;
     case 14:
-        launch_ftile<1, 4, 4, 1, EPI>(f, stream);
+        launch_ftile<1, 4, 4, 1, 1, EPI>(f, stream);
         break;
     default:
-        launch_ftile<1, 2, 8, 2, EPI>(f, stream);
+        launch_ftile<1, 2, 8, 2, 4, EPI>(f, stream);
     }
 }
 

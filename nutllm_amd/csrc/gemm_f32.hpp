@@ -74,10 +74,10 @@ constexpr int kChunkLd = 36; // floats per A row in LDS: 16-byte reads of 16
 // it (each supplies TJ / NB columns per lane). NORM: A's values are
 // multiplied by nw[k] (nw at 4 (lane % 8)) and sq[t] gathers the squares of
 // the values before that. NA: accumulators per output, each taking a run of
-// a chunk's k (shorter chains of additions, a smaller rounding error); NA 0:
-// one accumulator, to which every chunk's own sum is added, the shortest
-// chains of all.
-constexpr int gemm_f32_accs(int na) { return na == 0 ? 1 : na; }
+// a chunk's k (shorter chains of additions, a smaller rounding error); NA < 0:
+// one accumulator, to which every chunk's own sum, formed in -NA chains, is
+// added, the shortest chains of all.
+constexpr int gemm_f32_accs(int na) { return na < 0 ? 1 : na; }
 
 template <int TI, int TJ, int NB, int NA, int D, bool NORM>
 __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
@@ -145,22 +145,29 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
                 fa[i][4 * h + 3] = v.w;
             }
         __builtin_amdgcn_wave_barrier();
-        if constexpr (NA == 0) {
-            floatx4 part[TI][TJ];
+        if constexpr (NA < 0) {
+            constexpr int P = -NA;
+            floatx4 part[P][TI][TJ];
 #pragma unroll
             for (int s = 0; s < 8; s++)
 #pragma unroll
                 for (int i = 0; i < TI; i++)
 #pragma unroll
                     for (int j = 0; j < TJ; j++)
-                        part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        part[s % P][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
                             fa[i][s], fb[s][j],
-                            s == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : part[i][j], 0, 0, 0);
+                            s < P ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : part[s % P][i][j], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < TI; i++)
 #pragma unroll
-                for (int j = 0; j < TJ; j++)
-                    acc[0][i][j] += part[i][j];
+                for (int j = 0; j < TJ; j++) {
+#pragma unroll
+                    for (int step = 1; step < P; step *= 2)
+#pragma unroll
+                        for (int u = 0; u < P; u += 2 * step)
+                            part[u][i][j] += part[u + step][i][j];
+                    acc[0][i][j] += part[0][i][j];
+                }
         } else {
 #pragma unroll
             for (int s = 0; s < 8; s++)
@@ -276,11 +283,16 @@ __device__ __forceinline__ void gemm_f32_reduce(floatx4 (&parts)[NS][TI][TJ], fl
             float out[TJ];
 #pragma unroll
             for (int j = 0; j < TJ; j++) {
-                float s = red[(j * 4 + wk) * 64 + lane];
+                float part[WK];
 #pragma unroll
-                for (int w = 1; w < WK; w++)
-                    s += red[((w * TJ + j) * 4 + wk) * 64 + lane];
-                out[j] = s;
+                for (int w = 0; w < WK; w++)
+                    part[w] = red[((w * TJ + j) * 4 + wk) * 64 + lane];
+#pragma unroll
+                for (int step = 1; step < WK; step *= 2)
+#pragma unroll
+                    for (int w = 0; w < WK; w += 2 * step)
+                        part[w] += part[w + step];
+                out[j] = part[0];
             }
             epi(i, wk, out);
         }

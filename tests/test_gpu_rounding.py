@@ -117,3 +117,16 @@ def test_matmul_errs_as_eight_waves(gpu, mkn):
     b = rng.standard_normal((k, n)).astype(np.float32)
     want = a.astype(np.float64) @ b.astype(np.float64)
     assert rel(gpu.matmul_f32(a, b), want) <= 1.1 * U * np.sqrt((k / 8 + 1) / 2 + 3)
+
+
+@BOTH
+@pytest.mark.parametrize("tokens", [2, 20, 70])
+def test_dense_prompts_err_as_short_chains(gpu, qtype, tokens):
+    """Prompts whose weights are written out as fp32 (head size 32, blocks of
+    48): a chunk of 32 k in four chains and two levels, three over the waves,
+    and the row's two factors; 512 outputs and more settle it to 4 %, the bound
+    is 15 % over it. One chain per chunk and the waves one after the other,
+    23 in A, would be 20 % over the bound."""
+    got, want = value_rows(gpu, one_layer(gpu, 8, 8, 32, 512), qtype, 48,
+                           np.arange(3, 3 + tokens))
+    assert rel(got, want) <= 1.15 * U * np.sqrt((8 + 1) / 2 + 2 + 3 + 2)

@@ -286,15 +286,21 @@ __global__ __launch_bounds__(64) void fattention_kernel(const float *q, const fl
     load_k(0);
     load_v(0);
     for (int b = 0; b < keys; b += KB) {
-        floatx4 sc[KT];
+        floatx4 sc[KT], sd[KT];
 #pragma unroll
         for (int u = 0; u < KT; u++)
-            sc[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            sc[u] = sd[u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int s = 0; s < QS; s++)
+        for (int s = 0; s < QS / 2; s++)
 #pragma unroll
-            for (int u = 0; u < KT; u++)
+            for (int u = 0; u < KT; u++) {
                 sc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[s], kf[u][s], sc[u], 0, 0, 0);
+                sd[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[QS / 2 + s], kf[u][QS / 2 + s],
+                                                             sd[u], 0, 0, 0);
+            }
+#pragma unroll
+        for (int u = 0; u < KT; u++)
+            sc[u] += sd[u];
         if (b + KB < keys)
             load_k(b + KB);
 #pragma unroll
@@ -336,17 +342,30 @@ __global__ __launch_bounds__(64) void fattention_kernel(const float *q, const fl
             apart = !__all(finite);
         }
         if (!apart) {
+            float p[KT][4];
 #pragma unroll
             for (int u = 0; u < KT; u++) {
                 const float4 p4 =
                     *reinterpret_cast<const float4 *>(&ps[li * PLD + 16 * u + 4 * g]);
-                const float p[4] = {p4.x, p4.y, p4.z, p4.w};
+                p[u][0] = p4.x;
+                p[u][1] = p4.y;
+                p[u][2] = p4.z;
+                p[u][3] = p4.w;
+            }
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+                floatx4 part[KT];
 #pragma unroll
                 for (int s = 0; s < 4; s++)
 #pragma unroll
-                    for (int j = 0; j < TJ; j++)
-                        o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], vf[4 * u + s][j], o[j],
-                                                                    0, 0, 0);
+                    for (int u = 0; u < KT; u++)
+                        part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            p[u][s], vf[4 * u + s][j],
+                            s == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : part[u], 0, 0, 0);
+#pragma unroll
+                for (int u = 1; u < KT; u++)
+                    part[0] += part[u];
+                o[j] += part[0];
             }
         } else {
             for (int e = 0; e < KB && b + e < keys; e++)

@@ -119,6 +119,53 @@ def test_matmul_errs_as_eight_waves(gpu, mkn):
     assert rel(gpu.matmul_f32(a, b), want) <= 1.1 * U * np.sqrt((k / 8 + 1) / 2 + 3)
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(8, 2, 16), (8, 4, 32), (4, 2, 64), (2, 2, 128)])
+def test_attention_error_does_not_grow_with_the_keys(gpu, heads, kv_heads, head_dim):
+    """A layer whose hidden state is its attention's result (V and Wo select
+    dimensions, V large beside the embeddings), 1,200 keys. Scores in two
+    chains; P V in chains of 16 keys, a tree over a block's (64 keys, 32 at
+    head size 128), the blocks one after the other; 1.7 times that for the
+    exponentials and the rescaling. One chain over all keys, 600 in A, would
+    be three times the bound."""
+    rng = np.random.default_rng(head_dim)
+    tokens, dim, kvd = 1200, heads * head_dim, kv_heads * head_dim
+    cfg = gpu.Config(layers=1, heads=heads, dim=dim, head_dim=head_dim, ffn_dim=16, vocab_size=2000,
+                     kv_heads=kv_heads, max_seq=tokens, eos_token=1)
+    emb = (0.1 * rng.standard_normal((2000, dim))).astype(np.float32)
+    w = {name: (rng.standard_normal((dim, n)) * dim ** -0.5).astype(np.float32)
+         for name, n in (("query", dim), ("key", kvd))}
+    w["value"] = (1024.0 * np.eye(dim, kvd)).astype(np.float32)
+    w["output"] = np.eye(dim, dtype=np.float32)
+    w.update(gate=np.zeros((dim, 16), np.float32), up=np.zeros((dim, 16), np.float32),
+             down=np.zeros((16, dim), np.float32))
+    ones = np.ones(dim, np.float32)
+    m, cache = gpu.DeviceFModel(cfg, tied=True), gpu.KVCache(cfg)
+    try:
+        m.set_globals(emb, ones)
+        m.set_layer(0, w, ones, ones)
+        ids = rng.integers(2, 2000, tokens).astype(np.int32)
+        rows = m.prefill(cache, ids)[-64:].astype(np.float64)
+        k, v = (np.asarray(t[0], np.float64) for t in cache.read_positions(0, tokens))
+    finally:
+        cache.close(), m.close()
+    x = emb[ids].astype(np.float64)
+    q = (rms(x) @ w["query"].astype(np.float64)).reshape(tokens, heads, head_dim)
+    angle = (np.arange(tokens)[:, None] * 10000.0 ** (-2.0 * np.arange(head_dim // 2) / head_dim))
+    cos, sin = np.cos(angle)[:, None], np.sin(angle)[:, None]
+    q = np.stack((q[..., 0::2] * cos - q[..., 1::2] * sin,
+                  q[..., 0::2] * sin + q[..., 1::2] * cos), -1).reshape(q.shape)[-64:]
+    want = x[-64:].copy()
+    for h in range(heads):
+        s = q[:, h] @ k[h * kv_heads // heads].T / np.sqrt(head_dim)
+        s[np.arange(tokens)[None] > np.arange(tokens - 64, tokens)[:, None]] = -np.inf
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want[:, h * head_dim:(h + 1) * head_dim] += (p / p.sum(-1, keepdims=True)
+                                                    @ v[h * kv_heads // heads])
+    block = 32 if head_dim == 128 else 64
+    terms = (head_dim / 2 + 1) / 2 + 1 + 17 / 2 + 2 + tokens / block / 2
+    assert rel(rows, want) <= 1.7 * U * np.sqrt(terms)
+
+
 @BOTH
 @pytest.mark.parametrize("tokens", [2, 20, 70])
 def test_dense_prompts_err_as_short_chains(gpu, qtype, tokens):

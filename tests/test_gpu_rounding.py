@@ -167,6 +167,19 @@ def test_attention_error_does_not_grow_with_the_keys(gpu, heads, kv_heads, head_
 
 
 @BOTH
+@pytest.mark.parametrize("tokens", [16, 64])
+def test_row_tiles_round_to_both_sides(gpu, qtype, tokens):
+    """The errors of a prompt's V rows on the row tiles have no common sign (an
+    MFMA that adds large products to a small C rounds that down, 0.4 of the
+    error on average): 0.1 is several times the spread of the mean over 1,024
+    or more outputs of about one rounding each."""
+    got, want = value_rows(gpu, one_layer(gpu, 16, 4, 64, 1024), qtype, 32,
+                           np.arange(3, 3 + tokens))
+    error = got - want
+    assert abs(error.mean()) <= 0.1 * np.sqrt((error * error).mean())
+
+
+@BOTH
 @pytest.mark.parametrize("tokens", [2, 20, 70])
 def test_dense_prompts_err_as_short_chains(gpu, qtype, tokens):
     """Prompts whose weights are written out as fp32 (head size 32, blocks of

@@ -219,25 +219,31 @@ size_t prefill_gemm_min(const DecodeShape &s)
 // layer has their layout and per-token steps are not forced. A tile costs
 // the same for 2 rows as for 16, a step-kernel chunk a little per token; the
 // batched GEMM wins where its 64 x 128 tiles and its runs of k fill the
-// chip. TinyLlama INT4, row tiles against the better of the two: 5 tokens
-// 1.01 ms (1.02), 9 1.02 (1.36), 16 1.05 (1.95), 20 1.53 (2.28), 48 1.79
-// (2.21), 64 1.83 (2.32), 80 2.84 (2.34); two layers of the 7B widths INT4: 2
-// tokens 0.27 (0.20), 5 0.27 (0.31), 16 0.26 (0.35), 32 0.36 (0.34), 48 0.50
-// (0.35). Small widths are bound by the launches, five a layer against seven
-// (step_gqa4, 128 tokens: 0.11 against 0.17).
-size_t row_gemm_min(const DecodeShape &s)
+// chip. Measured (us, two layers, tinyllama four), row tiles against chunk:
+// width 512 INT4 5 tokens 87 (85), 6 87 (87), 12 87 (92), INT8 8 87 (87), 12 87
+// (87); 1024 INT4 5 95 (92), 6 94 (99), INT8 8 100 (95), 9 100 (101); 2048 INT4
+// 5 206 (200), 6 207 (216), INT8 5 218 (205), 6 218 (220); 2560 INT4 4 139
+// (139), INT8 4 146 (137), 5 146 (151); 4096 INT4 4 249 (212), 5 248 (251),
+// INT8 4 301 (291), 5 299 (338). Against the batch: 1536 64 tokens 162 (212);
+// 2048 64 364 (440), 65 496 (441); 2560 32 201 (249), 33 290 (251); 3584 32 279
+// (304), 33 426 (303); 4096 16 251 (328), 17 333 (328). Layers without step
+// kernels have neither: 2 tokens at width 3072 147 us against 750 in the dense
+// form and 645 token by token.
+size_t row_gemm_min(const nut_model &m)
 {
-    return s.dim < 1024 ? 2 : s.dim < 4096 ? 6 : 5;
+    if (!fast_steps(m))
+        return 2;
+    return m.shape.dim >= 2560 ? 5 : m.type == NUT_INT8 && m.shape.dim <= 1024 ? 9 : 6;
 }
 
 size_t row_gemm_max(const DecodeShape &s)
 {
-    return s.dim < 1024 ? size_t(kRowGemmMax) : s.dim < 4096 ? 64 : 16;
+    return s.dim < 1024 ? size_t(kRowGemmMax) : s.dim <= 2048 ? 64 : s.dim < 4096 ? 32 : 16;
 }
 
 bool use_row_gemm(const nut_model &m, size_t count)
 {
-    if (m.path != 0 || count < row_gemm_min(m.shape) || count > row_gemm_max(m.shape))
+    if (m.path != 0 || count > row_gemm_max(m.shape) || count < row_gemm_min(m))
         return false;
     for (const DeviceLayer &l : m.layers)
         if (!row_gemm_supported(m.shape, l.view))

@@ -340,11 +340,11 @@ template <int QT, int EPI> void launch_rows(RowGemm f, hipStream_t stream)
 {
     const int n = f.w[0].rows;
     if constexpr (EPI == kAdd) {
-        if (n < 4096) {
-            f.m <= 16 ? launch_tile<QT, 1, 1, 16, EPI>(f, stream)
-                      : launch_tile<QT, 2, 1, 8, EPI>(f, stream);
-            return;
-        }
+        // prompts of more than 16 rows come here at widths below 4096 only
+        n >= 4096   ? launch_tile<QT, 1, 2, 16, EPI>(f, stream)
+        : f.m <= 16 ? launch_tile<QT, 1, 1, 16, EPI>(f, stream)
+                    : launch_tile<QT, 2, 1, 8, EPI>(f, stream);
+        return;
     }
     if constexpr (EPI == kSwiglu) {
         if (n >= 2048 && f.m <= 16) {

@@ -2,10 +2,12 @@
 (tiny) on fp32 weights, against the per-token kernels.
 
 Lengths at the edges of the tiles (16 and 32 rows) and of the range that takes
-them, INT8 and INT4, head sizes 64 and 128: the last hidden state, the K/V rows
-of every position and the step that follows. The bar is 5e-6 on the relative
-error: fp32 sums, and activations as two f16 limbs (2^-22 each), over two
-layers; the step kernels themselves are within 2e-6 of 64 bits here."""
+them (6 or 9 rows on at small widths; the shorter ones, and those past its end,
+run on the step kernels and the batched GEMM), INT8 and INT4, head sizes 64 and
+128: the last hidden state, the K/V rows of every position and the step that
+follows. The bar is 5e-6 on the relative error: fp32 sums, and activations as
+three bf16 limbs without a remainder, over two layers; the step kernels
+themselves are within 2e-6 of 64 bits here."""
 import numpy as np
 import pytest
 
@@ -46,6 +48,55 @@ def test_row_tiles_match_steps(gpu, model, tokens):
     finally:
         dev.set_path(0)
         rows.close(), steps.close()
+
+
+# heads, kv_heads, head_dim, ffn: one layer, and the lengths tested with it.
+# Real widths take the forms of wide outputs; layers with three query heads per
+# KV head or head size 32 have no step kernels and take the tiles from 2 rows.
+WIDE = {
+    "w2048": ((32, 4, 64, 5632), (6, 16, 17, 40, 64)),
+    "w3072": ((24, 6, 128, 1152), (5, 16, 32)),
+    "w4096": ((32, 8, 128, 4224), (5, 16)),
+    "group3": ((6, 2, 64, 640), (2, 5, 17, 128)),
+    "head32": ((8, 4, 32, 384), (2, 16, 33)),
+}
+
+
+@pytest.mark.parametrize("qtype", [0, 1], ids=["int8", "int4"])
+@pytest.mark.parametrize("shape", list(WIDE))
+def test_row_tiles_match_steps_at_other_widths(gpu, qtype, shape):
+    (heads, kvh, hd, ffn), lengths = WIDE[shape]
+    dim, kvd = heads * hd, kvh * hd
+    cfg = gpu.Config(layers=1, heads=heads, dim=dim, head_dim=hd, ffn_dim=ffn, vocab_size=400,
+                     kv_heads=kvh, max_seq=160, eos_token=1)
+    rng = np.random.default_rng(ffn)
+    dims = dict(query=(dim, dim), key=(kvd, dim), value=(kvd, dim), output=(dim, dim),
+                gate=(ffn, dim), up=(ffn, dim), down=(dim, ffn))
+    mats = {}
+    for name, (r, c) in dims.items():
+        w = rng.standard_normal((r, c), np.float32) * np.float32(c ** -0.5)
+        mats[name] = (*gpu.quantize(w, qtype), r, c)
+    norms = [(1 + 0.1 * rng.standard_normal(dim)).astype(np.float32) for _ in range(2)]
+    emb = rng.standard_normal((400, dim), np.float32)
+    dev, rows, steps = gpu.DeviceModel(cfg, qtype), gpu.KVCache(cfg), gpu.KVCache(cfg)
+    try:
+        dev.set_globals(emb, norms[0], emb)
+        dev.set_layer(0, mats, *norms)
+        for tokens in lengths:
+            ids = rng.integers(2, 400, tokens).astype(np.int32)
+            got = dev.prefill(rows, ids)
+            dev.set_path(1)
+            want = dev.prefill(steps, ids)
+            dev.set_path(0)
+            assert rel(got, want) <= 5e-6
+            for a, b in zip(rows.read_positions(0, tokens), steps.read_positions(0, tokens)):
+                assert rel(a, b) <= 5e-6
+                error = np.abs(np.asarray(a, np.float64) - b)  # no part of a tile is wrong
+                assert error.max() <= 5e-5 * np.sqrt((np.asarray(b, np.float64) ** 2).mean())
+            assert rel(dev.decode(rows, 3), dev.decode(steps, 3)) <= 5e-6
+    finally:
+        dev.set_path(0)
+        dev.close(), rows.close(), steps.close()
 
 
 @pytest.mark.parametrize("scale", [1e-5, 1.0, 1e8])

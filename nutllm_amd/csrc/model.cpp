@@ -275,14 +275,30 @@ void prefill_rows(nut_model &m, nut_kvcache &kv, size_t count)
                       m.stream);
 }
 
-// Prompts of two tokens and more whose layers have no step kernel (head sizes
-// of 16 and 32, widths that no 32-wide block divides, other block sizes): each
-// launch's weights are written out as fp32 once for the whole prompt, where
-// the token-by-token way read and decoded them for every token (the tiny test
-// shape, 500 tokens: 42 ms of kernels, 84 ms with their launches).
+// Prompts whose layers have no step kernel (head sizes of 16 and 32, widths
+// that no 32-wide block divides, other query groups) and that neither the row
+// tiles nor the batch take: each launch's weights are written out as fp32 once
+// for the whole prompt, where the token-by-token way reads and decodes them for
+// every token (the tiny test shape, 500 tokens: 42 ms of kernels, 84 ms with
+// their launches). From this many tokens (us of two layers at 2 tokens, against
+// token by token): blocks of 48, width 768 181 (290), 2048 342 (780), 3072 754
+// (1198); of 64, whose codes are read 16 bytes at a time, INT4 768 190 (239),
+// 3072 847 (1065), 8192 (one layer) 2091 (2050), INT8 2304 389 (466), 3072 755
+// (645), 8192 1882 (1167), at 3 tokens 3072 757 (946), 8192 1888 (1740).
+size_t dense_min(const nut_model &m)
+{
+    for (const DeviceLayer &l : m.layers)
+        for (const QMat *q : {&l.view.query, &l.view.key, &l.view.value, &l.view.output,
+                              &l.view.gate, &l.view.up, &l.view.down})
+            if (!fast_layout(*q))
+                return 2;
+    return 2 + (m.shape.dim > 6144) + (m.type == NUT_INT8 && m.shape.dim > 2560);
+}
+
 bool use_dense(const nut_model &m, size_t count)
 {
-    return m.path == 0 && count >= 2 && attention_f32_supported(m.shape) && !fast_steps(m);
+    return m.path == 0 && attention_f32_supported(m.shape) && !fast_steps(m) &&
+           count >= dense_min(m);
 }
 
 // Its workspace: false where there is no memory for it (the token-by-token

@@ -7,6 +7,7 @@
 
 #include "kernels.hpp"
 #include "runtime.hpp"
+#include "sample.hpp"
 
 struct nut_model;
 struct nut_kvcache;
@@ -121,9 +122,10 @@ struct HostArea {
 };
 static_assert(sizeof(HostArea) % 16 == 0, "words are 16-byte aligned");
 constexpr size_t kSampleChunk = 4096; // sorted candidates read at once
+static_assert(kSampleTotals % 2 == 0 && kSampleChunk % 4 == 0, "candidates 16-byte aligned");
 inline size_t host_words(const nut_config &c)
 {
-    const size_t sampler = 2 * 128 + 2 * kSampleChunk; // totals, then p and ids
+    const size_t sampler = 2 * kSampleTotals + 2 * kSampleChunk; // totals, then p and ids
     size_t n = c.dim > c.vocab_size ? c.dim : c.vocab_size;
     n = c.max_seq + 1 > n ? c.max_seq + 1 : n;
     return (sampler > n ? sampler : n) + 4;

@@ -14,7 +14,7 @@ namespace nut {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kBlocks = 128;
+constexpr int kBlocks = kSampleTotals;
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 

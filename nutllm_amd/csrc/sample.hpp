@@ -7,6 +7,10 @@
 
 namespace nut {
 
+// Block totals that sample_sort returns: even, so that what follows them in
+// 4-byte words is 16-byte aligned.
+constexpr int kSampleTotals = 128;
+
 // Workspace of sample_sort for a vocabulary of `vocab` tokens: keys and
 // ids in and out, block totals, a flag, and rocPRIM's temporary storage.
 size_t sample_workspace_bytes(int vocab);
@@ -18,7 +22,7 @@ size_t sample_workspace_bytes(int vocab);
 // the reference's std::sort comparator, lines 56-61) to sorted_p /
 // sorted_ids, p in token order to token_p, one double partial sum of p per
 // block to totals (block order), and 1 to *bad when a p is not finite.
-// Returns the number of totals. workspace holds sample_workspace_bytes(vocab).
+// Returns the number of totals, kSampleTotals. workspace holds sample_workspace_bytes(vocab).
 int sample_sort(const float *logits, int vocab, const float *part_val, int parts,
                 float temperature, void *workspace, float **sorted_p, int **sorted_ids,
                 float **token_p, double **totals, int **bad, hipStream_t stream);

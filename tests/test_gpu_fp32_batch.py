@@ -1,12 +1,15 @@
 """The fp32 path's prompt batches and decode steps against a float64 numpy
 transformer, at the edges of their tiles: one row, one less and one more than
-a 16-row attention tile and a 64-key block, prompts long enough for every GEMM
-tile, head sizes with an attention kernel of their own and one without, widths
-that no 32-wide k chunk divides, a feed-forward width whose product is split.
+a 16-row attention tile and a 64-key block, head sizes with an attention kernel
+of their own and one without, widths that no 32-wide k chunk divides, and one
+layer of real widths at the lengths that take each GEMM tile in each of the
+projections, k whole and in two, three and four runs (tile_choice.py says which
+a case takes, test_cpu_tiles.py that they are all there).
 
 The bound on the relative error (2-norm) is 5e-6 per call: an fp32 chain of k
-terms errs by about sqrt(k) 2^-24 relative to its rms, k <= 300 here, over two
-layers of five products each (about 1e-6), with a factor of five to spare."""
+terms errs by about sqrt(k) 2^-24 / 4 relative to its rms, k <= 300 here, or at
+the real widths, whose waves share k, k <= 1,500, over two layers or one of five
+products each (about 1e-6), with a factor of five to spare."""
 import numpy as np
 import pytest
 
@@ -20,6 +23,13 @@ SHAPES = {
     "hd128": (2, 2, 128, 257, 40),
     "hd48": (2, 1, 48, 130, 33),
     "long": (2, 1, 64, 4131, 30),  # W2's k in runs, the last with a tail
+}
+# one layer each: the shape and the prompt lengths that are tested with it
+WIDE = {
+    "w2048": ((32, 4, 64, 5632, 64), (40, 301)),
+    "w2560": ((20, 2, 128, 4100, 64), (16, 301)),
+    "w4096": ((32, 16, 128, 4200, 64), (1, 16, 40, 80, 180, 200)),
+    "w4096n": ((32, 1, 128, 1100, 64), (16,)),
 }
 
 
@@ -67,10 +77,10 @@ class Exact:
         return x
 
 
-def build(gpu, shape, rng, vocab_fill=None):
-    heads, kvh, hd, ffn, vocab = SHAPES[shape]
+def build(gpu, shape, rng, vocab_fill=None, count=2):
+    heads, kvh, hd, ffn, vocab = SHAPES[shape] if shape in SHAPES else WIDE[shape][0]
     dim = heads * hd
-    cfg = gpu.Config(layers=2, heads=heads, dim=dim, head_dim=hd, ffn_dim=ffn, vocab_size=vocab,
+    cfg = gpu.Config(layers=count, heads=heads, dim=dim, head_dim=hd, ffn_dim=ffn, vocab_size=vocab,
                      kv_heads=kvh, max_seq=320, eos_token=1)
     emb = rng.standard_normal((vocab, dim)).astype(np.float32)
     if vocab_fill is not None:
@@ -80,8 +90,8 @@ def build(gpu, shape, rng, vocab_fill=None):
     m = gpu.DeviceFModel(cfg, tied=True)
     m.set_globals(emb, np.ones(dim, np.float32))
     layers = []
-    for i in range(2):
-        w = {k: (rng.standard_normal(s) * s[0] ** -0.5).astype(np.float32)
+    for i in range(count):
+        w = {k: (rng.standard_normal(s, np.float32) * s[0] ** -0.5).astype(np.float32)
              for k, s in dims.items()}
         an, fn = ((1 + 0.1 * rng.standard_normal(dim)).astype(np.float32) for _ in range(2))
         m.set_layer(i, w, an, fn)
@@ -108,6 +118,28 @@ def test_batch_and_steps_match_float64(gpu, shape, tokens):
         for i in range(2):
             want = exact.v[i].transpose(1, 0, 2)
             assert np.linalg.norm(v[i] - want) <= 5e-6 * np.linalg.norm(want)
+    finally:
+        cache.close()
+        m.close()
+
+
+@pytest.mark.parametrize("shape", list(WIDE))
+def test_real_widths_match_float64(gpu, shape):
+    rng = np.random.default_rng(17)
+    cfg, m, exact = build(gpu, shape, rng, count=1)
+    cache = gpu.KVCache(cfg)
+    try:
+        for tokens in WIDE[shape][1]:
+            ids = rng.integers(2, cfg.vocab_size, tokens).astype(np.int32)
+            rows, want = m.prefill(cache, ids), exact.run(ids, 0)
+            print(shape, tokens, flush=True)
+            # row by row: a row tile or a column tile that went wrong shows
+            error = np.linalg.norm(rows - want, axis=1)
+            assert np.all(error <= 5e-6 * np.linalg.norm(want, axis=1))
+            assert np.all(np.abs(rows - want) <= 5e-5 * np.sqrt((want * want).mean()))
+            k, v = cache.read_positions(0, tokens)
+            for got, ref in ((k[0], exact.k[0]), (v[0], exact.v[0])):
+                assert np.linalg.norm(got - ref.transpose(1, 0, 2)) <= 5e-6 * np.linalg.norm(ref)
     finally:
         cache.close()
         m.close()

@@ -2,8 +2,9 @@
 
 Each shape is one where a tile, its k chunk or its last columns can go wrong:
 fewer rows, columns or k than a tile, one more or less than a whole number of
-them, and one shape for every tile size that the launch chooses among. The
-bound is that of any summation order in fp32: every output's error is at most
+them, and a ragged shape for every form that the launch chooses among
+(tile_choice.py says which a shape takes, test_cpu_tiles.py that all are there).
+The bound is that of any summation order in fp32: every output's error is at most
 k 2^-23 sum |a b| (k fused steps of half an ulp each, doubled for the partial
 sums' additions)."""
 import numpy as np
@@ -12,12 +13,18 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("mkn", [
+SHAPES = [
     (1, 1, 1), (1, 33, 2), (3, 31, 3), (2, 64, 5), (17, 32, 16), (16, 33, 17),
     (15, 95, 31), (33, 4001, 130), (48, 257, 768), (768, 100, 768),
     (1000, 63, 1531), (313, 313, 313), (64, 1000, 63), (500, 65, 777),
     (65, 129, 4100), (2049, 40, 129),
-])
+    # the widest tile with four waves, with eight and with two accumulators;
+    # the 2 x 2 tile with eight waves and with four
+    (1757, 69, 849), (963, 291, 961), (967, 97, 953), (2145, 281, 33), (67, 69, 1747),
+]
+
+
+@pytest.mark.parametrize("mkn", SHAPES)
 def test_matmul_tile_edges(gpu, mkn):
     m, k, n = mkn
     rng = np.random.default_rng(m * 7 + k * 3 + n)

@@ -93,10 +93,8 @@ def test_matvec_f32_classifier(gpu, shape):
     assert rel_l2(y, ref) <= TOL
 
 
-# 768^3 and 224 x 640 x 96 run the k-split kernel (32 x 32 tiles, k over
-# eight waves), 256 x 320 x 256 (k not a multiple of 128) the tiled kernel
-# with 32 x 32 tiles, 1024 x 256 x 1024 64 x 64 tiles (256 of them), the
-# odd shapes the generic kernel
+# one kernel, whose tile and waves the launch picks for the shape (every form of
+# it, at ragged sizes, is in test_gpu_matmul_tiles.py)
 @pytest.mark.parametrize("mkn", [(768, 768, 768), (224, 640, 96), (256, 320, 256),
                                  (1024, 256, 1024), (7, 9, 8), (65, 33, 130)])
 def test_matmul_f32(gpu, mkn):
@@ -443,18 +441,21 @@ def test_tiny_matches_reference_golden(gpu, qtype, tag, norms):
     dev.close()
 
 
-@pytest.mark.parametrize("prompt_len", [2, 5, 6, 15, 29])
-def test_tinyllama_int4_prefill_step_chunk(gpu, tinyllama_int4, prompt_len):
-    """Prompts below the GEMM threshold (30 tokens) run as one chunk of
-    consecutive tokens through the step kernels (each launch covers every
-    token of the chunk; the arithmetic per token is the decode step's; from
-    6 tokens the row launches take four rows per wave). Hidden state and
-    K/V rows within rel-L2 1e-5 of the oracle's per-token prefill."""
+@pytest.mark.parametrize("prompt_len,path", [(2, 0), (5, 0), (5, 1), (6, 1), (15, 1), (29, 1),
+                                             (6, 0), (15, 0), (30, 0), (40, 0), (64, 0)])
+def test_tinyllama_int4_prefill_step_chunk(gpu, tinyllama_int4, prompt_len, path):
+    """Short prompts: one chunk of consecutive tokens through the step kernels
+    (each launch covers every token of the chunk; the arithmetic per token is
+    the decode step's; from 6 tokens the row launches take four rows per wave),
+    which is the way of up to 5 tokens at this width and of all with the step
+    kernels forced (path 1), and the row tiles, the way of 6 to 64. Hidden state
+    and K/V rows within rel-L2 1e-5 of the oracle's per-token prefill."""
     model, _, _, dev = tinyllama_int4
     prompt = gpu.synth_tokens(17, model.config.vocab_size, prompt_len)
     cache = gpu.KVCache(model.config)
-    dev.set_path(0)
+    dev.set_path(path)
     h = dev.prefill(cache, prompt)
+    dev.set_path(0)
     om = O.oracle_model(model)
     assert rel_l2(h, om.prefill(prompt)) <= TOL
     for layer in (0, model.config.layers - 1):
@@ -470,20 +471,25 @@ def test_tinyllama_int4_prefill_step_chunk(gpu, tinyllama_int4, prompt_len):
 PREFILL_TOL = 2e-3  # rel-L2, batched (GEMM) prefill
 
 
-@pytest.mark.parametrize("prompt_len", [30, 40, 64, 130, 300])
-def test_tinyllama_int4_prefill_gemm(gpu, tinyllama_int4, prompt_len):
-    """Prompts of 30+ tokens run as a batch (MFMA GEMMs, causal attention).
+@pytest.mark.parametrize("prompt_len,path", [(30, 2), (40, 2), (64, 2), (65, 0), (127, 0),
+                                             (128, 0), (130, 0), (300, 0)])
+def test_tinyllama_int4_prefill_gemm(gpu, tinyllama_int4, prompt_len, path):
+    """Prompts as a batch (MFMA GEMMs, causal attention), the way of 65 tokens
+    and more at this width, and of 30 and more without the row tiles (path 2).
     Hidden state and K/V rows within rel-L2 2e-3 of the fp32 step arithmetic
-    (oracle for 30 and 40 tokens, the device step kernels for 64, 130 and
-    300: one whole 64-query attention tile with no padding, then three and
-    five tiles), and the greedy ids that follow the prefill identical to the
-    oracle's. 30 tokens is the shortest batched prompt (34 padding rows in
-    its tile)."""
+    (oracle for 30, 40, 65 and 127 tokens, the device step kernels for 64, 128,
+    130 and 300: one and two whole 64-query attention tiles with no padding,
+    then three and five tiles), and the greedy ids that follow the prefill
+    identical to the oracle's. 30 tokens leave 34 padding rows in their tile,
+    65 tokens 63 in their second."""
     model, _, _, dev = tinyllama_int4
     prompt = gpu.synth_tokens(11, model.config.vocab_size, prompt_len)
     cache = gpu.KVCache(model.config)
+    oracle = prompt_len in (30, 40, 65, 127)
+    dev.set_path(path)
     h = dev.prefill(cache, prompt)
-    if prompt_len <= 40:
+    dev.set_path(0)
+    if oracle:
         om = O.oracle_model(model)
         ref = om.prefill(prompt)
         kv_ref = lambda l, kvh, p: om.kv_row(l, kvh, p)  # noqa: E731
@@ -502,8 +508,10 @@ def test_tinyllama_int4_prefill_gemm(gpu, tinyllama_int4, prompt_len):
                 k, v = cache.key_value(layer, kvh, p)
                 rk, rv = kv_ref(layer, kvh, p)
                 assert rel_l2(k, rk) <= PREFILL_TOL and rel_l2(v, rv) <= PREFILL_TOL
-    if prompt_len <= 40:
+    if oracle:
+        dev.set_path(path)
         ids, _ = dev.generate(prompt, 8)
+        dev.set_path(0)
         ref_ids, _, _ = om.generate(prompt, 8)
         assert ids == ref_ids
 

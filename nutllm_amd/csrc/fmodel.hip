@@ -188,8 +188,11 @@ template <int EPI> void launch_fgemm(FGemm f, hipStream_t stream)
             n >= 4096 ? launch_ftile<1, 2, 16, 2, 4, EPI>(f, stream)
                       : launch_ftile<1, 1, 16, 3, 4, EPI>(f, stream);
         } else {
-            n >= 8192 ? launch_ftile<1, 4, 8, 1, 4, EPI>(f, stream)
-                      : launch_ftile<1, 2, 16, 2, 4, EPI>(f, stream);
+            // four chains spill here: from width 2048, where two are as good,
+            // Q/K/V takes 13.7 us instead of 16
+            n >= 8192     ? launch_ftile<1, 4, 8, 1, 4, EPI>(f, stream)
+            : f.k >= 2048 ? launch_ftile<1, 2, 16, 2, 2, EPI>(f, stream)
+                          : launch_ftile<1, 2, 16, 2, 4, EPI>(f, stream);
         }
         return;
     }

@@ -112,8 +112,8 @@ void launch_pick_token(const DecodeShape &s, const float *part_val,
 // attn_count holds 2 * heads * kStepTokensMax ints, zero before the first
 // step (the kernels keep both consistent from then on). 31 tokens: one
 // chunk costs about 0.55 ms plus 0.09 ms per token on the TinyLlama INT4
-// shape, so a prompt below the batched-prefill threshold runs as one chunk
-// (15-token chunks took 2.81 ms for 20 tokens, one chunk 2.28 ms).
+// shape (15-token chunks took 2.81 ms for 20 tokens, one chunk 2.28 ms); the
+// shortest prompts run so, longer ones on the row tiles.
 constexpr int kStepTokensMax = 31;
 struct StepBuffers {
     float *hidden, *query, *context, *act;

@@ -126,8 +126,7 @@ __global__ __launch_bounds__(kThreads) void matvec_q_staged(QMat m, const float 
 // The last cols % 16 weights go one to a lane. Bounded by its VALU work and
 // the latency of the first loads; one weight per lane and load, as before,
 // spent a 64-bit division and three loads on each: 5000 x 3001 INT4 26.4 us,
-// now 8
-// (two matrices a pass 70.6 -> 15.8).
+// now 8 (two matrices a pass 70.6 -> 15.8).
 constexpr int kRaggedRows = 2, kRaggedThreads = 512;
 constexpr int kRunLd = 20; // floats of x per run in LDS (16, padded)
 

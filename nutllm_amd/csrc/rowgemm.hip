@@ -4,7 +4,7 @@
 // Up to kRowGemmMax rows a layer's weights are read once, and what counts is
 // that the whole chip has its loads in flight (TinyLlama INT4, a layer of 20
 // tokens: 104 us on the step kernels, which dot every row once a token, 141
-// in the batched GEMM's 64 x 128 tiles, 70 here; 16 tokens 88 -> 47): 16 TJ
+// in the batched GEMM's 64 x 128 tiles, 73 here; 16 tokens 88 -> 49): 16 TJ
 // outputs per workgroup, its WK waves sharing k, so that a 2,048-wide matrix
 // is 64 to 128 workgroups of 8 or 16 waves. Codes are
 // exact in bf16 and an fp32 activation is the sum of three bf16 limbs

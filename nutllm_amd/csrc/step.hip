@@ -353,7 +353,9 @@ __global__ __launch_bounds__(kThreads) void attention_kernel(
             for (int w = 1; w < kWaves; w++)
                 cm = fmaxf(cm, wmax[group & 1][w][g]);
             const float mn = fmaxf(m[g], cm);
-            const float alpha = expf(m[g] - mn);
+            // no score above -inf yet: weights 0, not NaN
+            const float from = mn == -INFINITY ? 0.0f : mn;
+            const float alpha = expf(m[g] - from);
             m[g] = mn;
             l[g] *= alpha;
 #pragma unroll
@@ -362,7 +364,7 @@ __global__ __launch_bounds__(kThreads) void attention_kernel(
 #pragma unroll
             for (int j = 0; j < PF; j++)
                 if (c0 + j < c_end) { // workgroup-uniform
-                    const float e = valid[j] ? expf(sc[j][g] - mn) : 0.0f;
+                    const float e = valid[j] ? expf(sc[j][g] - from) : 0.0f;
                     l[g] += e;
 #pragma unroll
                     for (int i = 0; i < S; i++)

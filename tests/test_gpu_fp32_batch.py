@@ -162,3 +162,31 @@ def test_non_finite_token_leaves_earlier_rows(gpu, shape):
     finally:
         cache.close()
         m.close()
+
+
+@pytest.mark.parametrize("head_dim", [48, 64, 128])
+@pytest.mark.parametrize("hidden", [31, 32, 200])
+def test_keys_at_minus_infinity_have_no_weight(gpu, head_dim, hidden):
+    """A decode step over keys whose scores overflow to minus infinity (whole
+    runs of the split attention among them) and five ordinary ones after them:
+    the ordinary ones alone count, as in one softmax over all."""
+    rng = np.random.default_rng(hidden)
+    SHAPES["inf"] = (2, 2, head_dim, 100, 50)
+    cfg, m, exact = build(gpu, "inf", rng, count=1)
+    cache = gpu.KVCache(cfg)
+    try:
+        token = 7
+        w, an, _ = exact.layers[0]
+        q = rope((rms(exact.emb[[token]], an) @ w["query"]).reshape(1, 2, head_dim), hidden + 5)[0]
+        k = rng.standard_normal((hidden + 5, 2, head_dim)).astype(np.float32)
+        v = rng.standard_normal((hidden + 5, 2, head_dim)).astype(np.float32)
+        k[:hidden] = -3e38 * np.sign(q)
+        cache.write_positions(0, k.transpose(1, 0, 2)[None], v.transpose(1, 0, 2)[None])
+        exact.k[0], exact.v[0] = k.astype(np.float64), v.astype(np.float64)
+        cache.set_length(hidden + 5)
+        got, want = m.decode(cache, token), exact.run([token], hidden + 5)[0]
+        assert np.linalg.norm(got - want) <= 5e-6 * np.linalg.norm(want)
+    finally:
+        del SHAPES["inf"]
+        cache.close()
+        m.close()

@@ -31,7 +31,8 @@ def model(request, gpu):
     dev.close()
 
 
-@pytest.mark.parametrize("tokens", [2, 3, 15, 16, 17, 31, 32, 33, 64, 65, 127, 128])
+@pytest.mark.parametrize("tokens", [2, 3, 8, 9, 15, 16, 17, 31, 32, 33, 64, 65, 127, 128,
+                                    129])
 def test_row_tiles_match_steps(gpu, model, tokens):
     cfg, dev = model
     ids = gpu.synth_tokens(9, cfg.vocab_size, tokens).astype(np.int32)
@@ -50,13 +51,14 @@ def test_row_tiles_match_steps(gpu, model, tokens):
         rows.close(), steps.close()
 
 
-# heads, kv_heads, head_dim, ffn: one layer, and the lengths tested with it.
+# heads, kv_heads, head_dim, ffn: one layer, and the lengths tested with it, the
+# last of w3072 and w4096 the shortest that the batched GEMM takes there.
 # Real widths take the forms of wide outputs; layers with three query heads per
 # KV head or head size 32 have no step kernels and take the tiles from 2 rows.
 WIDE = {
     "w2048": ((32, 4, 64, 5632), (6, 16, 17, 40, 64)),
-    "w3072": ((24, 6, 128, 1152), (5, 16, 32)),
-    "w4096": ((32, 8, 128, 4224), (5, 16)),
+    "w3072": ((24, 6, 128, 1152), (5, 16, 32, 33)),
+    "w4096": ((32, 8, 128, 4224), (5, 16, 17)),
     "group3": ((6, 2, 64, 640), (2, 5, 17, 128)),
     "head32": ((8, 4, 32, 384), (2, 16, 33)),
 }

@@ -17,9 +17,9 @@
 // are its outputs. All vector accesses to memory are 4-byte aligned only
 // (unaligned vector access is on for this target), so one kernel serves
 // every row length. Rows past m read row m - 1, columns past n the last TJ
-// columns; what they give is not stored. The k tail is read value by value,
-// zeros past the end. Partial tiles are added in LDS in wave order: the
-// result does not depend on timing.
+// columns; what they give is not stored. The k tail is read value by value
+// and is zeros past the end. Partial tiles are added in LDS in a fixed order:
+// the result does not depend on timing.
 #pragma once
 
 #include "device.hpp"
@@ -203,39 +203,53 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
             }
     }
     if (tail) { // wave-uniform
+        // every value is loaded, from the last k where it is past the end, and
+        // replaced by a zero there: loads behind a condition each took as long
+        // as several chunks
         const int kt = k & ~(kChunk - 1), k4 = 4 * (lane & 7), g8 = 8 * (lane >> 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int at = min(kt + k4 + e, k - 1) - k4;
+#pragma unroll
+            for (int t = 0; t < 2 * TI; t++)
+                ra[0][t][e] = pa[t][at];
+            if (NORM)
+                rn[0][e] = nw[at];
+        }
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const ptrdiff_t at = min(kt + g8 + s, k - 1) - g8;
+#pragma unroll
+            for (int q = 0; q < NB; q++)
+                load_u<TB>(pb[q] + at * ptrdiff_t(ldb), &rb[0][s][q * TB]);
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const bool in = kt + k4 + e < k;
 #pragma unroll
             for (int t = 0; t < 2 * TI; t++)
-                ra[0][t][e] = in ? pa[t][kt + e] : 0.0f;
+                ra[0][t][e] = in ? ra[0][t][e] : 0.0f;
             if (NORM)
-                rn[0][e] = in ? nw[kt + e] : 0.0f;
+                rn[0][e] = in ? rn[0][e] : 0.0f;
         }
 #pragma unroll
-        for (int s = 0; s < 8; s++) {
+        for (int s = 0; s < 8; s++)
 #pragma unroll
             for (int j = 0; j < TJ; j++)
-                rb[0][s][j] = 0.0f;
-            if (kt + g8 + s < k) {
-#pragma unroll
-                for (int q = 0; q < NB; q++)
-                    load_u<TB>(pb[q] + size_t(kt + s) * ldb, &rb[0][s][q * TB]);
-            }
-        }
+                rb[0][s][j] = kt + g8 + s < k ? rb[0][s][j] : 0.0f;
         multiply(ra[0], rb[0], rn[0]);
     }
 }
 
-// Chunks [c0, c1) of share `i` of `count` of k, and whether it takes the tail.
+// Chunks [c0, c1) of share `i` of `count` of k, and whether it takes the tail:
+// the first, which has no more chunks than any other.
 __device__ __forceinline__ void gemm_f32_share(int k, int i, int count, int &c0, int &c1,
                                                bool &tail)
 {
     const int full = k / kChunk;
     c0 = int((long long)full * i / count);
     c1 = int((long long)full * (i + 1) / count);
-    tail = i == count - 1 && k % kChunk != 0;
+    tail = i == 0 && k % kChunk != 0;
 }
 
 template <int TI, int TJ, int NA>

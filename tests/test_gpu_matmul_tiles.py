@@ -18,9 +18,15 @@ SHAPES = [
     (15, 95, 31), (33, 4001, 130), (48, 257, 768), (768, 100, 768),
     (1000, 63, 1531), (313, 313, 313), (64, 1000, 63), (500, 65, 777),
     (65, 129, 4100), (2049, 40, 129),
-    # the widest tile with four waves, with eight and with two accumulators;
+    # 48 x 64; the widest tile with four waves, with eight and with two accumulators;
     # the 2 x 2 tile with eight waves and with four
-    (1757, 69, 849), (963, 291, 961), (967, 97, 953), (2145, 281, 33), (67, 69, 1747),
+    (1000, 65, 1531), (1757, 69, 849), (963, 291, 961), (967, 97, 953), (2145, 281, 33),
+    (67, 69, 1747),
+    # a tile to each wave (k < 64): its last rows and columns, one k, a whole
+    # chunk, a chunk and one; the smallest grid that has it and one less
+    (8191, 1, 1), (8129, 37, 15), (8200, 5, 16), (8177, 32, 17), (9001, 33, 32), (8321, 63, 33),
+    (1, 47, 8190), (3, 31, 8195), (515, 32, 1030), (1000, 61, 1537),
+    (1024, 63, 512), (1024, 63, 448), (1024, 64, 512),
 ]
 
 
@@ -52,9 +58,9 @@ def test_matmul_non_finite_rows_stay_apart(gpu):
 
 
 def test_matmul_rows_past_one_grid_dimension(gpu):
-    """More 16-row tiles than one dimension of a grid has workgroups (2^32
-    threads): products of one term each, which are exact."""
-    m = 140_000_000
+    """More workgroups (64 rows each) than the launch puts into one dimension
+    of a grid, 2^22: products of one term each, which are exact."""
+    m = 270_000_000
     a = np.arange(m, dtype=np.float32)
     c = gpu.matmul_f32(a.reshape(m, 1), np.full((1, 1), 0.5, np.float32))
     assert np.array_equal(c.ravel(), 0.5 * a)

@@ -34,6 +34,9 @@ def pick(tiles, m, k, n):
 
 def matmul_form(m, k, n):
     """(ti, tj, waves, accumulators) of matmul_f32's launch."""
+    wide = 4 if n > 32 else 2 if n > 16 else 1
+    if k < 64 and -(-m // 64) * -(-n // (16 * wide)) >= 128:
+        return 1, wide, 1, 2
     ti, tj, count = pick(table("gemm_f32.hpp", "gemm_f32_choose(int m"), m, k, n)
     deep = k >= 256
     if (ti, tj) == (4, 4):
@@ -46,7 +49,8 @@ def matmul_form(m, k, n):
 
 
 MATMUL_FORMS = {(4, 4, 4, 1), (4, 4, 8, 1), (4, 4, 4, 2), (3, 4, 4, 2), (3, 3, 4, 2), (2, 4, 4, 2),
-                (2, 2, 8, 2), (2, 2, 4, 2), (1, 2, 4, 2), (1, 1, 8, 2)}
+                (2, 2, 8, 2), (2, 2, 4, 2), (1, 2, 4, 2), (1, 1, 8, 2), (1, 4, 1, 2), (1, 2, 1, 2),
+                (1, 1, 1, 2)}
 
 
 def fgemm_form(epilogue, m, k, n):

@@ -43,8 +43,9 @@ __global__ __launch_bounds__(256) void matmul_f32_shallow(const float *__restric
     floatx4 acc[2][1][TJ];
     float sq[2] = {};
     gemm_f32_clear(acc);
-    gemm_f32_run<1, TJ, 1, 2, 1, false>(pa, pb, size_t(n), nullptr, k, 0, k / kChunk,
-                                        k % kChunk != 0, lds + wave * 16 * kChunkLd, acc, sq);
+    gemm_f32_run<1, TJ, 1, 2, 1, false, Tail::last>(pa, pb, size_t(n), nullptr, k, 0, k / kChunk,
+                                                    k % kChunk != 0, lds + wave * 16 * kChunkLd,
+                                                    acc, sq);
     if (off >= cols)
         return;
 #pragma unroll
@@ -75,13 +76,16 @@ inline dim3 tile_grid(int tiles_m, int tiles_n)
     return count <= row ? dim3(count) : dim3(row, (count + row - 1) / row);
 }
 
-template <int TI, int TJ, int WK, int NA, int D>
+// The tail's code by k, in whole chunks or ragged; measured for each form.
+template <int TI, int TJ, int WK, int NA, int D, Tail WHOLE = Tail::none, Tail RAGGED = Tail::first>
 void launch_tile(const float *a, const float *b, float *c, int m, int k, int n,
                  hipStream_t stream)
 {
     const int tiles_m = (m - 1) / (16 * TI) + 1, tiles_n = (n - 1) / (16 * TJ) + 1;
-    hipLaunchKernelGGL((matmul_f32_wave<TI, TJ, WK, NA, D>), tile_grid(tiles_m, tiles_n),
-                       dim3(64 * WK), 0, stream, a, b, c, m, k, n, tiles_m, tiles_n);
+    const auto kernel = k % kChunk ? matmul_f32_wave<TI, TJ, WK, NA, D, RAGGED>
+                                   : matmul_f32_wave<TI, TJ, WK, NA, D, WHOLE>;
+    hipLaunchKernelGGL(kernel, tile_grid(tiles_m, tiles_n), dim3(64 * WK), 0, stream, a, b, c, m,
+                       k, n, tiles_m, tiles_n);
 }
 
 template <int TJ>
@@ -121,11 +125,14 @@ void launch_matmul_f32(const float *a, const float *b, float *c, int m, int k,
     // tile has the registers for one: where it leaves CUs idle it has eight
     // waves for that (960 x 2048 x 960: 2.9e-7 against 4.1e-7 with four, at 43
     // and 41 us), or two accumulators where k has fewer than eight chunks.
+    // Where the tail's code stands changes the loop's schedule: 960 x 2048 x 960
+    // 41.8 us with it last, 43.4 without; 64 x 4096 x 64 9.1 and 10.0; 33 x 4096
+    // x 3333 24.7 us with it first, 28.6 without.
     const bool deep = k >= 8 * kChunk, few = size_t(m / 64) * (n / 64) < 256;
     switch (t.ti * 10 + t.tj) {
     case 44:
         if (few)
-            deep ? launch_tile<4, 4, 8, 1, 1>(a, b, c, m, k, n, stream)
+            deep ? launch_tile<4, 4, 8, 1, 1, Tail::last, Tail::last>(a, b, c, m, k, n, stream)
                  : launch_tile<4, 4, 4, 2, 1>(a, b, c, m, k, n, stream);
         else
             launch_tile<4, 4, 4, 1, 1>(a, b, c, m, k, n, stream);
@@ -140,14 +147,15 @@ void launch_matmul_f32(const float *a, const float *b, float *c, int m, int k,
         launch_tile<2, 4, 4, 2, 2>(a, b, c, m, k, n, stream);
         break;
     case 22:
-        deep && t.count <= 256 ? launch_tile<2, 2, 8, 2, 1>(a, b, c, m, k, n, stream)
-                               : launch_tile<2, 2, 4, 2, 1>(a, b, c, m, k, n, stream);
+        deep && t.count <= 256
+            ? launch_tile<2, 2, 8, 2, 1, Tail::first>(a, b, c, m, k, n, stream)
+            : launch_tile<2, 2, 4, 2, 1>(a, b, c, m, k, n, stream);
         break;
     case 12:
         launch_tile<1, 2, 4, 2, 2>(a, b, c, m, k, n, stream);
         break;
     default:
-        launch_tile<1, 1, 8, 2, 2>(a, b, c, m, k, n, stream);
+        launch_tile<1, 1, 8, 2, 2, Tail::last, Tail::last>(a, b, c, m, k, n, stream);
     }
     check_launch("threaded matmul");
 }

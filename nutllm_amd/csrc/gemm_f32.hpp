@@ -77,9 +77,15 @@ constexpr int kChunkLd = 36; // floats per A row in LDS: 16-byte reads of 16
 // a chunk's k (shorter chains of additions, a smaller rounding error); NA < 0:
 // one accumulator, to which every chunk's own sum, formed in -NA chains, is
 // added, the shortest chains of all.
+// T: where the tail's code stands, if it is there at all. Before the loop, its
+// loads are hidden behind the other waves' work (1612 x 207 x 1566: 21.4 us,
+// 26.1 after it), but it takes registers, which a kernel with no loop to speak
+// of has not to give (5236 x 5 x 7775: 62.3 us, 48.0 after it). A GEMM of whole
+// chunks is faster without it (4096^3: 1,082 us, 1,118 with it before the loop).
+enum class Tail { none, first, last };
 constexpr int gemm_f32_accs(int na) { return na < 0 ? 1 : na; }
 
-template <int TI, int TJ, int NB, int NA, int D, bool NORM>
+template <int TI, int TJ, int NB, int NA, int D, bool NORM, Tail T>
 __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
                                              const float *const (&pb)[NB], size_t ldb,
                                              const float *nw, int k, int c0, int c1, bool tail,
@@ -179,30 +185,7 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
                             fa[i][s], fb[s][j], acc[s * NA / 8][i][j], 0, 0, 0);
         }
     };
-    const int count = c1 - c0;
-#pragma unroll
-    for (int d = 0; d < D; d++)
-        if (d < count)
-            load(d);
-    int q0 = 0;
-    // whole rounds whose every slot loads again
-    for (; q0 + 2 * D <= count; q0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-            multiply(ra[d], rb[d], rn[d]);
-            load(d);
-        }
-    }
-    for (; q0 < count; q0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; d++)
-            if (q0 + d < count) { // wave-uniform
-                multiply(ra[d], rb[d], rn[d]);
-                if (q0 + d + D < count)
-                    load(d);
-            }
-    }
-    if (tail) { // wave-uniform
+    auto remainder = [&] {
         // every value is loaded, from the last k where it is past the end, and
         // replaced by a zero there: loads behind a condition each took as long
         // as several chunks
@@ -238,7 +221,34 @@ __device__ __forceinline__ void gemm_f32_run(const float *const (&pa)[2 * TI],
             for (int j = 0; j < TJ; j++)
                 rb[0][s][j] = kt + g8 + s < k ? rb[0][s][j] : 0.0f;
         multiply(ra[0], rb[0], rn[0]);
+    };
+    if (T == Tail::first && tail) // wave-uniform
+        remainder();
+    const int count = c1 - c0;
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if (d < count)
+            load(d);
+    int q0 = 0;
+    // whole rounds whose every slot loads again
+    for (; q0 + 2 * D <= count; q0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            multiply(ra[d], rb[d], rn[d]);
+            load(d);
+        }
     }
+    for (; q0 < count; q0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++)
+            if (q0 + d < count) { // wave-uniform
+                multiply(ra[d], rb[d], rn[d]);
+                if (q0 + d + D < count)
+                    load(d);
+            }
+    }
+    if (T == Tail::last && tail)
+        remainder();
 }
 
 // Chunks [c0, c1) of share `i` of `count` of k, and whether it takes the tail:
@@ -382,7 +392,7 @@ inline GemmTile gemm_f32_choose(int m, int k, int n)
 }
 
 // C = A B, a tile per workgroup, whose WK waves share its k.
-template <int TI, int TJ, int WK, int NA, int D>
+template <int TI, int TJ, int WK, int NA, int D, Tail T>
 __global__ __launch_bounds__(64 * WK) void matmul_f32_wave(
     const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c, int m, int k,
     int n, int tiles_m, int tiles_n)
@@ -412,8 +422,8 @@ __global__ __launch_bounds__(64 * WK) void matmul_f32_wave(
     int c0, c1;
     bool tail;
     gemm_f32_share(k, wave, WK, c0, c1, tail);
-    gemm_f32_run<TI, TJ, 1, NA, D, false>(pa, pb, size_t(n), nullptr, k, c0, c1, tail,
-                                    lds + wave * 16 * TI * kChunkLd, acc, sq);
+    gemm_f32_run<TI, TJ, 1, NA, D, false, T>(pa, pb, size_t(n), nullptr, k, c0, c1, tail,
+                                             lds + wave * 16 * TI * kChunkLd, acc, sq);
     __syncthreads();
     gemm_f32_reduce<TI, TJ, WK>(
         acc, lds, wave,
